@@ -331,6 +331,9 @@ mpm::GridDev griddev(mpm_sim* s) {
     return g;
 }
 
+// The current planes' ids (u32 bits): the original index of every slot's particle.
+const float* id_plane(const mpm_sim* s) { return s->ps[s->ps_cur] + (size_t)mpm::CID * s->cap; }
+
 // ---- profiling helpers ----
 // Timing-only events: no system-scope fence when recorded, so recording
 // writes back and invalidates no caches and does not slow the next launch.
@@ -1124,9 +1127,9 @@ int diff_backward_pass(mpm_sim* s, bool has_gv, bool checked, Stage& span) {
     HIP_TRY(s, mpm::launch_copy_u32(s->status + mpm::ST_GATHERS, s->dsnap, s->stream));
     HIP_TRY(s, hipMemsetAsync(s->adj, 0, (size_t)mpm::NADJ * plane * 4, s->stream));
     HIP_TRY(s, hipMemsetAsync(s->gml, 0, 2 * (size_t)s->max_schunks * sizeof(double), s->stream));
-    HIP_TRY(s, mpm::launch_permute_in(s->adj, cap, mpm::AX, 3, s->slot_of_id, s->staging, s->n, s->stream));
+    HIP_TRY(s, mpm::launch_permute_in(s->adj, cap, mpm::AX, 3, id_plane(s), s->staging, s->n, s->stream));
     if (has_gv)
-        HIP_TRY(s, mpm::launch_permute_in(s->adj, cap, mpm::AV, 3, s->slot_of_id, s->staging + 3 * (size_t)s->n,
+        HIP_TRY(s, mpm::launch_permute_in(s->adj, cap, mpm::AV, 3, id_plane(s), s->staging + 3 * (size_t)s->n,
                                           s->n, s->stream));
     const float dt = s->diff_dt;
     const size_t st_words = (size_t)mpm::NCOMP * plane;
@@ -1276,7 +1279,7 @@ int adj_layout(int field, int* comp0, int* ncomp) {
 int read_adjoint(mpm_sim* s, int field, float* out) {
     int c0, nc;
     if (adj_layout(field, &c0, &nc) != 0) return fail(s, MPM_ERR_INVALID, "no adjoint for this field");
-    HIP_TRY(s, mpm::launch_unpermute(s->adj, s->cap, c0, nc, s->slot_of_id, s->staging, s->n, s->stream));
+    HIP_TRY(s, mpm::launch_unpermute(s->adj, s->cap, c0, nc, id_plane(s), s->staging, s->n, s->stream));
     HIP_TRY(s, hipMemcpyAsync(out, s->staging, (size_t)s->n * nc * 4, hipMemcpyDeviceToHost, s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     return MPM_OK;
@@ -1295,7 +1298,7 @@ int read_backward_outputs(mpm_sim* s, float* gx0, float* gv0, float* gE, double*
     size_t off = 0;
     for (const Out3& o : outs) {
         if (!o.dst) continue;
-        HIP_TRY(s, mpm::launch_unpermute(s->adj, s->cap, o.comp, o.nc, s->slot_of_id, s->staging + off, s->n,
+        HIP_TRY(s, mpm::launch_unpermute(s->adj, s->cap, o.comp, o.nc, id_plane(s), s->staging + off, s->n,
                                          s->stream));
         off += n * o.nc;
     }
@@ -1323,7 +1326,7 @@ int read_backward_outputs_device(mpm_sim* s, float* gx0, float* gv0, float* gE, 
     const Out3 outs[3] = {{gx0, mpm::AX, 3}, {gv0, mpm::AV, 3}, {gE, mpm::AE, 1}};
     for (const Out3& o : outs)
         if (o.dst)
-            HIP_TRY(s, mpm::launch_unpermute(s->adj, s->cap, o.comp, o.nc, s->slot_of_id, o.dst, s->n, s->stream));
+            HIP_TRY(s, mpm::launch_unpermute(s->adj, s->cap, o.comp, o.nc, id_plane(s), o.dst, s->n, s->stream));
     if (gml) HIP_TRY(s, mpm::launch_sum_pairs(s->gml, s->status + mpm::ST_NCHUNKS, s->max_schunks, gml, s->stream));
     return MPM_OK;
 }
@@ -1577,7 +1580,7 @@ int mpm_write_field(mpm_sim* sim, int field, const void* data, uint32_t n) {
     if (n == 0) return MPM_OK;
     if (!data) return fail(sim, MPM_ERR_INVALID, "data must not be NULL");
     HIP_TRY(sim, hipMemcpyAsync(sim->staging, data, (size_t)n * nc * 4, hipMemcpyHostToDevice, sim->stream));
-    HIP_TRY(sim, mpm::launch_permute_in(sim->ps[sim->ps_cur], sim->cap, c0, nc, sim->slot_of_id, sim->staging, n,
+    HIP_TRY(sim, mpm::launch_permute_in(sim->ps[sim->ps_cur], sim->cap, c0, nc, id_plane(sim), sim->staging, n,
                                         sim->stream));
     HIP_TRY(sim, hipStreamSynchronize(sim->stream));
     if (field == MPM_FIELD_YOUNGS) sim->has_E = 1;
@@ -1593,7 +1596,7 @@ int mpm_read_field(mpm_sim* sim, int field, void* out, uint32_t n) {
     if (n != sim->n) return fail(sim, MPM_ERR_INVALID, "output length must equal the particle count");
     if (n == 0) return MPM_OK;
     if (!out) return fail(sim, MPM_ERR_INVALID, "out must not be NULL");
-    HIP_TRY(sim, mpm::launch_unpermute(sim->ps[sim->ps_cur], sim->cap, c0, nc, sim->slot_of_id, sim->staging, n,
+    HIP_TRY(sim, mpm::launch_unpermute(sim->ps[sim->ps_cur], sim->cap, c0, nc, id_plane(sim), sim->staging, n,
                                        sim->stream));
     HIP_TRY(sim, hipMemcpyAsync(out, sim->staging, (size_t)n * nc * 4, hipMemcpyDeviceToHost, sim->stream));
     HIP_TRY(sim, hipStreamSynchronize(sim->stream));
@@ -1608,7 +1611,7 @@ int mpm_read_field_device(mpm_sim* sim, int field, void* out_dev, uint32_t n) {
     if (n != sim->n) return fail(sim, MPM_ERR_INVALID, "output length must equal the particle count");
     if (n == 0) return MPM_OK;
     if (!out_dev) return fail(sim, MPM_ERR_INVALID, "out must not be NULL");
-    HIP_TRY(sim, mpm::launch_unpermute(sim->ps[sim->ps_cur], sim->cap, c0, nc, sim->slot_of_id,
+    HIP_TRY(sim, mpm::launch_unpermute(sim->ps[sim->ps_cur], sim->cap, c0, nc, id_plane(sim),
                                        static_cast<float*>(out_dev), n, sim->stream));
     return MPM_OK;
 }

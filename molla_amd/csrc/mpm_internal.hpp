@@ -238,11 +238,12 @@ hipError_t launch_reorder(const float* src, float* dst, uint32_t cap, const uint
                           uint32_t n, hipStream_t s);
 hipError_t launch_index_slots(const float* ps, uint32_t cap, uint32_t* slot_of_id, uint32_t n,
                               hipStream_t s);
-hipError_t launch_unpermute(const float* ps, uint32_t cap, int comp0, int ncomp,
-                            const uint32_t* slot_of_id, float* out, uint32_t n, hipStream_t s);
-hipError_t launch_permute_in(float* ps, uint32_t cap, int comp0, int ncomp,
-                             const uint32_t* slot_of_id, const float* in, uint32_t n,
-                             hipStream_t s);
+// `ncomp` (1, 3 or 9) planes <-> n x ncomp words in original order; ids: the
+// id plane of the planes' slot order.
+hipError_t launch_unpermute(const float* ps, uint32_t cap, int comp0, int ncomp, const float* ids, float* out,
+                            uint32_t n, hipStream_t s);
+hipError_t launch_permute_in(float* ps, uint32_t cap, int comp0, int ncomp, const float* ids, const float* in,
+                             uint32_t n, hipStream_t s);
 // Soil checkpoint: planes -> 40-word streams (ids in original order), and
 // streams -> planes in identity slot order; aux = 12 words per particle.
 hipError_t launch_ckpt_pack(const float* ps, uint32_t cap, const uint32_t* slot_of_id, const uint32_t* aux,
