@@ -80,15 +80,12 @@ struct mpm_sim {
     uint32_t max_schunks = 0;
     uint32_t part_cap = 0;     // chunks with an LDS partial slot
     uint32_t* chunk_of_slot = nullptr;
-    uint32_t* cflags = nullptr;
-    uint32_t* cexcl = nullptr;
-    uint32_t* scan_scratch = nullptr;
-    uint32_t* smark = nullptr;  // static-list rebuild: per-tile mark, its scan, scan scratch
-    uint32_t* spos = nullptr;
-    uint32_t* sscan = nullptr;
+    uint64_t* lscan = nullptr;  // layout tables: per-tile (static mark, chunks) pairs and their prefix sums
+    uint32_t max_W = 0;         // tiles of the longest tile row
     uint32_t* list[2] = {nullptr, nullptr};
     uint32_t* status = nullptr;  // ST_WORDS u32
     uint32_t* slot_of_id = nullptr;
+    bool index_valid = false;  // slot_of_id describes the current slots (the fused layout sorts leave it behind)
     uint32_t* keys = nullptr;
     uint32_t* vals = nullptr;
     uint32_t* sort_scratch = nullptr;
@@ -260,9 +257,8 @@ void release(mpm_sim* s) {
     void* bufs[] = {s->d_scenes, s->d_mats, s->ps[0], s->ps[1], s->gmp, s->gv, s->tile_flag, s->tile_scene,
                     s->list[0], s->list[1], s->status, s->slot_of_id, s->keys, s->vals, s->sort_scratch,
                     s->d_chunks, s->affine, s->staging, s->tile_lb, s->slist,
-                    s->src_slot, s->chunk_box, s->part, s->schunks, s->chunk_of_slot, s->cflags,
-                    s->cexcl, s->scan_scratch, s->smark, s->spos, s->sscan, s->tile_slot, s->tile_mark,
-                    s->slot_tile, s->defer_list, s->srec};
+                    s->src_slot, s->chunk_box, s->part, s->schunks, s->chunk_of_slot, s->lscan, s->tile_slot,
+                    s->tile_mark, s->slot_tile, s->defer_list, s->srec};
     for (void* b : bufs)
         if (b) (void)hipFree(b);
     for (float* c : s->ckpt) (void)hipFree(c);
@@ -410,6 +406,12 @@ int particle_blocks(mpm_sim* s) {
     return int(s->n_chunks);
 }
 
+// Launch bound of the sorted layout's chunk walks (the chunk count is on the
+// device; a walk strides over what lies beyond).
+uint32_t chunk_bound(const mpm_sim* s) {
+    return std::min<uint32_t>(s->max_schunks, s->n / 256 + s->n / 64 + s->n_scenes + 64);
+}
+
 // Cells of grid storage: every tile of a dense grid, the pool of a sparse one.
 size_t grid_cells(const mpm_sim* s) { return (size_t)(s->pool_cap ? s->pool_cap : s->total_tiles) * 64; }
 
@@ -442,12 +444,7 @@ int ensure_grid(mpm_sim* s) {
     HIP_TRY(s, dalloc(&s->part, (size_t)s->part_cap * mpm::LDS_CELLS));
     HIP_TRY(s, dalloc(&s->schunks, s->max_schunks));
     HIP_TRY(s, dalloc(&s->chunk_of_slot, s->cap));
-    HIP_TRY(s, dalloc(&s->cflags, s->cap));
-    HIP_TRY(s, dalloc(&s->cexcl, s->cap));
-    HIP_TRY(s, dalloc(&s->scan_scratch, mpm::scan_scratch_words(s->cap)));
-    HIP_TRY(s, dalloc(&s->smark, s->total_tiles));
-    HIP_TRY(s, dalloc(&s->spos, s->total_tiles));
-    HIP_TRY(s, dalloc(&s->sscan, mpm::scan_scratch_words(s->total_tiles)));
+    HIP_TRY(s, dalloc(&s->lscan, mpm::layout_scratch_words(s->total_tiles)));
     HIP_TRY(s, hipMemsetAsync(s->chunk_box, 0, 2 * (size_t)s->part_cap * sizeof(int4), s->stream));
     HIP_TRY(s, hipMemsetAsync(s->gmp, 0, cells * sizeof(float4), s->stream));
     HIP_TRY(s, hipMemsetAsync(s->gv, 0, cells * sizeof(float4), s->stream));
@@ -478,17 +475,31 @@ int clear_grid(mpm_sim* s) {
     return MPM_OK;
 }
 
-__global__ void k_iota(uint32_t* p, uint32_t n) {
-    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) p[i] = i;
+// slot_of_id of the current slots, where a sort since has left it behind.
+int ensure_index(mpm_sim* s) {
+    if (s->index_valid) return MPM_OK;
+    if (!s->dry) HIP_TRY(s, mpm::launch_index_slots(s->ps[s->ps_cur], s->cap, s->slot_of_id, s->n, s->stream));
+    s->index_valid = true;
+    return MPM_OK;
 }
 
-// keys[id] -> stable sort -> reorder particle planes into tile order.
+// Tile keys -> stable sort -> (reorder) tables of the layout and the particle
+// planes in tile order.
 int sort_particles(mpm_sim* s, bool reorder) {
     s->boxes_valid = false;  // the chunk list is rebuilt
     s->layout_gen++;
+    // The fused layout only needs particles grouped by tile: ties keep the
+    // current slot order.  The deterministic mode and the key query keep the
+    // reference order (ties by original id), which fixes its summation order.
+    const bool by_slot = reorder && s->p2g_mode == MPM_P2G_FUSED;
+    if (reorder && !by_slot) {
+        int rc = ensure_index(s);
+        if (rc != MPM_OK) return rc;
+    }
     if (s->dry) {
         if (reorder) {
             s->ps_cur = 1 - s->ps_cur;
+            s->index_valid = !by_slot;
             s->sorted = true;
             s->since_sort = 0;
             s->sorts++;
@@ -497,49 +508,63 @@ int sort_particles(mpm_sim* s, bool reorder) {
     }
     Stage st(s, MPM_STAGE_SORT);
     mpm::StepArgs a = args(s, 0.f, s->list_cur);
-    // The fused layout only needs particles grouped by tile: ties keep the
-    // current slot order.  The deterministic mode and the key query keep the
-    // reference order (ties by original id), which fixes its summation order.
-    const bool by_slot = reorder && s->p2g_mode == MPM_P2G_FUSED;
-    HIP_TRY(s, mpm::launch_tile_keys(a, s->keys, by_slot ? 1 : 0, s->stream));
-    unsigned blocks = std::min<uint32_t>((s->n + 255) / 256, 8192u);
-    hipLaunchKernelGGL(k_iota, dim3(std::max(blocks, 1u)), dim3(256), 0, s->stream, s->vals, s->n);
-    HIP_TRY(s, hipGetLastError());
     const int bits = int(ceil_log2(std::max(s->total_tiles, 2u)));
-    HIP_TRY(s, mpm::radix_sort_pairs(s->keys, s->vals, s->n, bits, s->sort_scratch, s->stream));
-    if (reorder) {
-        const int other = 1 - s->ps_cur;
-        // The active list and the chunk list depend on the sorted keys only.
-        HIP_TRY(s, mpm::launch_static_rebuild(s->d_scenes, s->tile_scene, s->tile_flag, s->slist,
-                                              s->status + mpm::ST_SCOUNT, s->keys, s->n, s->tile_lb,
-                                              s->total_tiles, s->smark, s->spos, s->sscan, s->stream));
-        // several particles per thread only for the shader model's fused
-        // layout (the differentiable model and its adjoint take one)
-        s->chunk_ppt = (by_slot && s->sh[0].model == MPM_MODEL_SHADER) ? s->ppt : 1u;
-        HIP_TRY(s, mpm::build_sorted_chunks(s->d_scenes, s->tile_scene, s->keys, s->tile_lb, s->n, s->cflags,
-                                            s->cexcl, s->scan_scratch, s->schunks, s->status + mpm::ST_NCHUNKS,
-                                            s->chunk_of_slot, CHUNK * s->chunk_ppt, s->seg_tiles, s->total_tiles,
-                                            s->stream));
-        s->srec_valid = s->srec != nullptr;
-        if (s->srec)
-            HIP_TRY(s, mpm::launch_static_records(s->d_scenes, s->tile_scene, s->slist, s->status + mpm::ST_SCOUNT,
-                                                  s->total_tiles, s->tile_lb, s->chunk_of_slot, s->part_cap, s->srec,
-                                                  s->stream));
-        // previous slot of every new slot: the sorted slots spread over cells
-        // inside each chunk, or the reference order's ids mapped to slots
-        if (by_slot)
-            HIP_TRY(s, mpm::launch_chunk_spread(s->d_scenes, s->schunks, s->status + mpm::ST_NCHUNKS,
-                                                s->max_schunks, s->ps[s->ps_cur], s->cap, s->vals, s->src_slot,
-                                                s->keys, CHUNK * s->chunk_ppt, s->stream));
-        else
-            HIP_TRY(s, mpm::launch_reorder_index(s->vals, s->slot_of_id, s->src_slot, s->n, s->stream));
-        HIP_TRY(s, mpm::launch_reorder(s->ps[s->ps_cur], s->ps[other], s->cap, s->src_slot, s->n, s->stream));
-        HIP_TRY(s, mpm::launch_index_slots(s->ps[other], s->cap, s->slot_of_id, s->n, s->stream));
-        s->ps_cur = other;
-        s->sorted = true;
-        s->since_sort = 0;
-        s->sorts++;
+    uint32_t* n_chunks = s->status + mpm::ST_NCHUNKS;
+    if (!reorder) {
+        HIP_TRY(s, mpm::launch_tile_keys(a, mpm::radix_input(s->keys, s->n, bits, s->sort_scratch), 0, s->stream));
+        HIP_TRY(s, mpm::radix_sort_pairs(s->keys, s->vals, s->n, bits, s->sort_scratch, nullptr, 0, nullptr,
+                                         s->stream));
+        return MPM_OK;
     }
+    // several particles per thread only for the shader model's fused layout
+    // (the differentiable model and its adjoint take one)
+    s->chunk_ppt = (by_slot && s->sh[0].model == MPM_MODEL_SHADER) ? s->ppt : 1u;
+    const uint32_t chunk_cap = CHUNK * s->chunk_ppt;
+    mpm::LayoutArgs q{};
+    q.scenes = s->d_scenes;
+    q.tile_scene = s->tile_scene;
+    q.tile_flag = s->tile_flag;
+    q.slist = s->slist;
+    q.scount = s->status + mpm::ST_SCOUNT;
+    q.tile_lb = s->tile_lb;
+    q.keys = s->keys;
+    q.src = by_slot ? s->vals : s->src_slot;
+    q.chunks = s->schunks;
+    q.n_chunks = n_chunks;
+    q.n = s->n;
+    q.total_tiles = s->total_tiles;
+    q.max_W = s->max_W;
+    if (mpm::layout_fits_one(s->n, s->total_tiles)) {
+        HIP_TRY(s, mpm::launch_layout_one(a, s->n_scenes, q, chunk_cap, s->seg_tiles, bits,
+                                          by_slot ? nullptr : s->slot_of_id, s->stream));
+    } else {
+        bool lb_done = false;
+        HIP_TRY(s, mpm::launch_tile_keys(a, mpm::radix_input(s->keys, s->n, bits, s->sort_scratch), by_slot ? 1 : 0,
+                                         s->stream));
+        HIP_TRY(s, mpm::radix_sort_pairs(s->keys, s->vals, s->n, bits, s->sort_scratch, s->tile_lb, s->total_tiles,
+                                         &lb_done, s->stream));
+        HIP_TRY(s, mpm::launch_layout(q, lb_done, chunk_cap, s->seg_tiles, s->lscan, s->stream));
+        if (!by_slot) HIP_TRY(s, mpm::launch_reorder_index(s->vals, s->slot_of_id, s->src_slot, s->n, s->stream));
+    }
+    // the sorted slots spread over cells inside each chunk; the reference
+    // order keeps its slots
+    if (by_slot)
+        HIP_TRY(s, mpm::launch_chunk_spread(s->d_scenes, s->schunks, n_chunks, chunk_bound(s), s->ps[s->ps_cur],
+                                            s->cap, s->vals, s->src_slot, s->keys, s->chunk_of_slot, chunk_cap,
+                                            s->stream));
+    else
+        HIP_TRY(s, mpm::launch_chunk_slots(s->schunks, n_chunks, chunk_bound(s), s->chunk_of_slot, s->stream));
+    const int other = 1 - s->ps_cur;
+    const mpm::RecordArgs rec{s->d_scenes, s->tile_scene, s->slist, s->status + mpm::ST_SCOUNT, s->total_tiles,
+                              s->tile_lb, s->chunk_of_slot, s->part_cap, s->srec};
+    HIP_TRY(s, mpm::launch_reorder(s->ps[s->ps_cur], s->ps[other], s->cap, s->src_slot, s->n,
+                                   by_slot ? nullptr : s->slot_of_id, rec, s->stream));
+    s->srec_valid = s->srec != nullptr;
+    s->index_valid = !by_slot;
+    s->ps_cur = other;
+    s->sorted = true;
+    s->since_sort = 0;
+    s->sorts++;
     return MPM_OK;
 }
 
@@ -547,7 +572,7 @@ int sort_particles(mpm_sim* s, bool reorder) {
 void use_sorted_chunks(mpm_sim* s, mpm::StepArgs& a, int& blocks) {
     a.chunks = s->schunks;
     a.n_chunks_dev = s->status + mpm::ST_NCHUNKS;
-    a.n_chunks = std::min<uint32_t>(s->max_schunks, s->n / 256 + s->n / 64 + s->n_scenes + 64);
+    a.n_chunks = chunk_bound(s);
     blocks = s->pblocks ? int(s->pblocks) : int(std::min<uint32_t>(a.n_chunks, 4096u));
 }
 
@@ -758,6 +783,7 @@ int create(const mpm_scene_config* cfgs, uint32_t n_scenes, mpm_sim** out) {
         uint64_t W = (cfgs[i].grid_size + 3u) / 4u;
         s->sh.push_back(make_scene(cfgs[i], uint32_t(tiles), i * MPM_MAX_MATERIALS));
         tiles += W * W * W;
+        s->max_W = std::max(s->max_W, uint32_t(W));
         s->pbase.push_back(uint32_t(cap));
         cap += cfgs[i].max_particles;
     }
@@ -850,8 +876,10 @@ int set_particles(mpm_sim* s, const uint32_t* counts, const float* pos, const fl
     }
     HIP_TRY(s, put(mpm::CID));
     s->ps_cur = 0;
-    HIP_TRY(s, mpm::launch_index_slots(s->ps[0], s->cap, s->slot_of_id, s->n, s->stream));
-    int rc = build_chunks(s);
+    s->index_valid = false;
+    int rc = ensure_index(s);
+    if (rc != MPM_OK) return rc;
+    rc = build_chunks(s);
     if (rc != MPM_OK) return rc;
     rc = upload_scenes(s);
     if (rc != MPM_OK) return rc;
@@ -1364,7 +1392,7 @@ int autotune(mpm_sim* s, float dt, uint32_t trial, uint32_t* out_pb, uint32_t* o
         if (r != MPM_OK) return r;
         HIP_TRY(s, hipMemcpyAsync(s->ps[0], backup, words * 4, hipMemcpyDeviceToDevice, s->stream));
         s->ps_cur = 0;
-        HIP_TRY(s, mpm::launch_index_slots(s->ps[0], s->cap, s->slot_of_id, s->n, s->stream));
+        s->index_valid = false;
         s->sorted = false;
         return MPM_OK;
     };
@@ -1472,15 +1500,13 @@ int autotune(mpm_sim* s, float dt, uint32_t trial, uint32_t* out_pb, uint32_t* o
 //
 // The radix sort of mpm_sort_keys_noalloc works in `scratch`, a static device
 // array sized by radix_scratch_words(MPM_NOALLOC_MAX_PARTICLES): ping-pong
-// keys and ids (2 n words), the per-block digit histogram and its scan
-// (2 x 256 x n/4096 words) and the scan's block sums.  Every GPU the library
+// keys and ids (2 n words), the digit histograms of the blocks (at most 2^18
+// words up to that count) and the digit totals.  Every GPU the library
 // runs on holds its own copy until the process ends.  In host code `scratch`
 // names a host-side stand-in; its device address comes from
 // hipGetSymbolAddress, once per device (noalloc_scratch), and only that
 // address is ever handed to a kernel or a copy.
-constexpr size_t NOALLOC_HIST = 256u * ((MPM_NOALLOC_MAX_PARTICLES + 4095u) / 4096u);
-constexpr size_t NOALLOC_WORDS =
-    2u * size_t(MPM_NOALLOC_MAX_PARTICLES) + 2u * NOALLOC_HIST + NOALLOC_HIST / 1024u + 1024u + 256u;
+constexpr size_t NOALLOC_WORDS = 2u * size_t(MPM_NOALLOC_MAX_PARTICLES) + (1u << 18) + (1u << 12) + 64u;
 static __device__ __align__(256) uint32_t scratch[NOALLOC_WORDS];
 
 namespace {
@@ -1504,26 +1530,16 @@ int noalloc_scratch(mpm_sim* s, uint32_t** out) {
     return MPM_OK;
 }
 
-// Scene-local tile key and id of every particle of one scene (the scene's
-// slots are [pbase, pbase + cnt) in any layout), written at the local id so a
-// stable sort over ids 0..cnt-1 gives the reference order.  Same key formula
-// as k_tile_keys (mpm_particle_order.wgsl:13-25), without the tile base.
+// Scene-local tile key of every particle of one scene (the scene's slots are
+// [pbase, pbase + cnt) in any layout), written at the local id so a stable
+// sort over ids 0..cnt-1 gives the reference order.
 __global__ void k_scene_keys(const float* __restrict__ ps, uint32_t cap, const SceneDev* __restrict__ scenes,
-                             uint32_t scene, uint32_t pbase, uint32_t cnt, uint32_t* __restrict__ keys,
-                             uint32_t* __restrict__ ids) {
+                             uint32_t scene, uint32_t pbase, uint32_t cnt, uint32_t* __restrict__ keys) {
     const SceneDev& sc = scenes[scene];
     for (uint32_t j = blockIdx.x * blockDim.x + threadIdx.x; j < cnt; j += gridDim.x * blockDim.x) {
         const uint32_t slot = pbase + j;
-        uint32_t t[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-            const float c = floorf((ps[(size_t)(mpm::CX + k) * cap + slot] - sc.origin[k]) * sc.inv_dx);
-            const int ci = min(max(int(c) - sc.window[k], 0), int(sc.G) - 1);
-            t[k] = uint32_t(ci) >> 2;
-        }
         const uint32_t id = __float_as_uint(ps[(size_t)mpm::CID * cap + slot]) - pbase;
-        keys[id] = t[0] + sc.W * (t[1] + sc.W * t[2]);
-        ids[id] = id;
+        keys[id] = mpm::tile_key(sc, ps, cap, slot) - sc.tile_base;
     }
 }
 
@@ -1764,7 +1780,7 @@ int mpm_step_n_graph(mpm_sim* sim, float dt, uint32_t substeps) {
     GraphKey key{dtb, substeps, uint32_t(sim->p2g_mode), uint32_t(sim->ps_cur), uint32_t(sim->list_cur),
                  uint32_t(sim->grid_dirty), uint32_t(sort_start) | (sim->since_sort << 1), uint32_t(sim->write_vc),
                  sim->pblocks, sim->gblocks, sim->sort_every, uint32_t(sim->has_E),
-                 sim->ppt | (sim->seg_tiles << 4) | (sim->chunk_ppt << 8)};
+                 sim->ppt | (sim->seg_tiles << 4) | (sim->chunk_ppt << 8) | (uint32_t(sim->index_valid) << 12)};
     auto it = sim->graphs.find(key);
     if (it == sim->graphs.end()) {
         // Lazily allocated tables must exist before capture.
@@ -2008,9 +2024,9 @@ int mpm_sort_keys_noalloc(mpm_sim* sim, uint32_t scene, uint32_t capacity, uint3
     if (cnt > 0) {
         const unsigned blocks = std::min<uint32_t>((cnt + 255) / 256, 8192u);
         hipLaunchKernelGGL(k_scene_keys, dim3(blocks), dim3(256), 0, sim->stream, sim->ps[sim->ps_cur], sim->cap,
-                           sim->d_scenes, scene, sim->pbase[scene], cnt, keys_dev, ids_dev);
+                           sim->d_scenes, scene, sim->pbase[scene], cnt, mpm::radix_input(keys_dev, cnt, bits, scr));
         HIP_TRY(sim, hipGetLastError());
-        HIP_TRY(sim, mpm::radix_sort_pairs(keys_dev, ids_dev, cnt, bits, scr, sim->stream));
+        HIP_TRY(sim, mpm::radix_sort_pairs(keys_dev, ids_dev, cnt, bits, scr, nullptr, 0, nullptr, sim->stream));
     }
     if (capacity > cnt) {
         const unsigned blocks = std::min<uint32_t>((capacity - cnt + 255) / 256, 8192u);
@@ -2258,6 +2274,7 @@ int mpm_checkpoint_capture(mpm_sim* sim, uint32_t* words, uint32_t n) {
         return fail(sim, MPM_ERR_FAULT,
                     "MPM soil checkpoint: latched grid fault; incomplete state cannot be archived");
     if (n == 0) return MPM_OK;
+    if ((rc = ensure_index(sim)) != MPM_OK) return rc;
     TempWords d;
     const size_t nw = (size_t)MPM_SOIL_WORDS_PER_PARTICLE * n;
     HIP_TRY(sim, dalloc(&d.p, nw));
@@ -2318,7 +2335,7 @@ int mpm_checkpoint_restore(mpm_sim* sim, const mpm_soil_meta* meta, const uint32
     sim->counts.assign(1, n);
     sim->pbase.assign(1, 0);
     sim->ps_cur = 0;
-    HIP_TRY(sim, mpm::launch_index_slots(sim->ps[0], sim->cap, sim->slot_of_id, n, sim->stream));
+    sim->index_valid = false;
     if ((rc = build_chunks(sim)) != MPM_OK) return rc;
     if ((rc = upload_scenes(sim)) != MPM_OK) return rc;
     if (sim->gmp && (rc = clear_grid(sim)) != MPM_OK) return rc;

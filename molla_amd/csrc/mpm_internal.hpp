@@ -216,26 +216,33 @@ hipError_t launch_set_u32(uint32_t* p, uint32_t v, hipStream_t s);
 hipError_t launch_snap_counters(const uint32_t* status, uint32_t* dst, hipStream_t s);
 hipError_t launch_copy_u32(const uint32_t* src, uint32_t* dst, hipStream_t s);
 hipError_t launch_sum_pairs(const double* v, const uint32_t* count, uint32_t cap, double* out, hipStream_t s);
-// Static active list of a sort: the 3x3x3 dilation of occupied tiles, in
-// ascending tile order (mark/pos: total_tiles u32 each; scan_scratch:
-// scan_scratch_words(total_tiles)).  Also builds the tile lower-bound table.
-hipError_t launch_static_rebuild(const SceneDev* scenes, const uint32_t* tile_scene,
-                                 uint32_t* tile_flag, uint32_t* slist, uint32_t* scount,
-                                 const uint32_t* sorted_keys, uint32_t n, uint32_t* tile_lb,
-                                 uint32_t total_tiles, uint32_t* mark, uint32_t* pos, uint32_t* scan_scratch,
-                                 hipStream_t s);
-hipError_t launch_fill_u32(uint32_t* p, uint32_t v, size_t n, hipStream_t s);
-// The static tiles' records (GridDev::srec) for the sorted chunk list:
-// max_static bounds the static count (read on the device).
-hipError_t launch_static_records(const SceneDev* scenes, const uint32_t* tile_scene, const uint32_t* slist,
-                                 const uint32_t* scount, uint32_t max_static, const uint32_t* tile_lb,
-                                 const uint32_t* chunk_of_slot, uint32_t part_capacity, int* srec, hipStream_t s);
 hipError_t launch_tile_keys(const StepArgs& a, uint32_t* keys_out, int by_slot, hipStream_t s);
+// Spreads each chunk's particles over cells (src_in -> src_out and the keys,
+// in place) and writes chunk_of_slot.
 hipError_t launch_chunk_spread(const SceneDev* scenes, const Chunk* chunks, const uint32_t* n_chunks,
                                uint32_t max_chunks, const float* ps, uint32_t cap, const uint32_t* src_in,
-                               uint32_t* src_out, uint32_t* keys, uint32_t chunk_cap, hipStream_t s);
-hipError_t launch_reorder(const float* src, float* dst, uint32_t cap, const uint32_t* src_slot,
-                          uint32_t n, hipStream_t s);
+                               uint32_t* src_out, uint32_t* keys, uint32_t* chunk_of_slot, uint32_t chunk_cap,
+                               hipStream_t s);
+// chunk_of_slot alone (layouts whose order inside a chunk is fixed).
+hipError_t launch_chunk_slots(const Chunk* chunks, const uint32_t* n_chunks, uint32_t max_chunks,
+                              uint32_t* chunk_of_slot, hipStream_t s);
+// The static tiles' records (GridDev::srec) of a sorted chunk list:
+// max_static bounds the static count (read on the device).
+struct RecordArgs {
+    const SceneDev* scenes;
+    const uint32_t* tile_scene;
+    const uint32_t* slist;
+    const uint32_t* scount;
+    uint32_t max_static;
+    const uint32_t* tile_lb;
+    const uint32_t* chunk_of_slot;
+    uint32_t part_capacity;
+    int* srec;  // null: no records
+};
+// Gathers every plane into the new slot order; slot_of_id (may be null)
+// receives the new index; the records are written by blocks of the same launch.
+hipError_t launch_reorder(const float* src, float* dst, uint32_t cap, const uint32_t* src_slot, uint32_t n,
+                          uint32_t* slot_of_id, const RecordArgs& rec, hipStream_t s);
 hipError_t launch_index_slots(const float* ps, uint32_t cap, uint32_t* slot_of_id, uint32_t n,
                               hipStream_t s);
 // `ncomp` (1, 3 or 9) planes <-> n x ncomp words in original order; ids: the
@@ -291,21 +298,54 @@ hipError_t launch_adj_p2g(const AdjArgs& q, int blocks, hipStream_t s);
 hipError_t launch_adj_fused(const AdjArgs& q, const float* ps_prev, const float4* gv_prev, int blocks,
                             hipStream_t s);
 
-// ---- scans and the sorted chunk list (mpm_scan.hip) ----
-size_t scan_scratch_words(size_t n);
-hipError_t exclusive_scan_u32(const uint32_t* in, uint32_t* out, size_t n, uint32_t* scratch,
-                              uint32_t** total, hipStream_t s);
-hipError_t build_sorted_chunks(const SceneDev* scenes, const uint32_t* tile_scene, const uint32_t* keys,
-                               const uint32_t* lb, uint32_t n, uint32_t* flags, uint32_t* excl,
-                               uint32_t* scan_scratch, Chunk* chunks, uint32_t* n_chunks,
-                               uint32_t* chunk_of_slot, uint32_t chunk_cap, uint32_t seg_tiles, uint32_t total_tiles,
-                               hipStream_t s);
+// ---- tables of the sorted layout (mpm_scan.hip) ----
+struct LayoutArgs {
+    const SceneDev* scenes;
+    const uint32_t* tile_scene;
+    uint32_t* tile_flag;  // the static bit is rewritten
+    uint32_t* slist;      // static active list, ascending tiles
+    uint32_t* scount;
+    uint32_t* tile_lb;    // first sorted slot of every tile key, and n (total_tiles + 1)
+    uint32_t* keys;       // sorted tile keys
+    uint32_t* src;        // launch_layout_one: previous slot of every sorted slot
+    Chunk* chunks;
+    uint32_t* n_chunks;
+    uint32_t n, total_tiles, max_W;  // max_W: tiles of the longest tile row
+};
+size_t layout_scratch_words(uint32_t total_tiles);  // u64 words
+bool layout_fits_one(uint32_t n, uint32_t total_tiles);
+// Keys, sort, table and lists of a small layout in one launch.  slot_of_id
+// null: ties by current slot; else by original id.
+hipError_t launch_layout_one(const StepArgs& a, uint32_t n_scenes, const LayoutArgs& q, uint32_t chunk_cap,
+                             uint32_t seg_tiles, int bits, const uint32_t* slot_of_id, hipStream_t s);
+// Table and lists of sorted keys (lb_done: the table is there already).
+hipError_t launch_layout(const LayoutArgs& q, bool lb_done, uint32_t chunk_cap, uint32_t seg_tiles, uint64_t* scratch,
+                         hipStream_t s);
 
 // ---- radix sort (mpm_sort.hip) ----
 size_t radix_scratch_words(uint32_t n);
-// Stable LSD sort of (key, value) pairs on the low `bits` bits of the keys.
-// keys/vals are sorted in place; scratch holds radix_scratch_words(n) u32.
-hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, int bits,
-                            uint32_t* scratch, hipStream_t s);
+// Where the keys of a sort of n keys of `bits` bits have to be written:
+// `keys` itself or a part of the scratch.
+uint32_t* radix_input(uint32_t* keys, uint32_t n, int bits, uint32_t* scratch);
+// Stable LSD sort on the low `bits` bits: sorted keys in `keys`, the input
+// index of each in `vals`; scratch holds radix_scratch_words(n) u32.  lb (may
+// be null): where the sort finds the first position of every key in [0, n_lb]
+// by the way, it is written there and *lb_done set.
+hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, int bits, uint32_t* scratch, uint32_t* lb,
+                            uint32_t n_lb, bool* lb_done, hipStream_t s);
+
+// Tile key (shaders/mpm_particle_order.wgsl:13-25) of the particle in `slot`:
+// cell = floor((x - o) * inv_dx) - window, clamped to [0, G-1], /4, linearised
+// x-fastest, plus the scene's tile base.
+__device__ __forceinline__ uint32_t tile_key(const SceneDev& sc, const float* ps, uint32_t cap, uint32_t slot) {
+    uint32_t t[3];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float c = floorf((ps[(size_t)(CX + k) * cap + slot] - sc.origin[k]) * sc.inv_dx);
+        const int ci = min(max(int(c) - sc.window[k], 0), int(sc.G) - 1);
+        t[k] = uint32_t(ci) >> 2;
+    }
+    return sc.tile_base + t[0] + sc.W * (t[1] + sc.W * t[2]);
+}
 
 }  // namespace mpm

@@ -1,134 +1,279 @@
-// mpm_sort.hip -- stable LSD radix sort of (u32 key, u32 value) pairs.
+// mpm_sort.hip -- stable LSD radix sort of u32 keys with their input index.
 //
 // Same contract as molla's RadixSortKernel (molla-compute-primitives/src/
-// radix_sort.rs:1-30): 8-bit digits, stable, so ties keep their input
-// order.  Only the key bits that can be non-zero are sorted (ceil(bits/8)
-// passes).  Each pass is three launches:
-//   k_hist    per-block digit histogram (blocks of 4096 elements, LDS atomics)
-//   scan      device-wide exclusive scan of the digit-major histogram
-//   k_scatter stable scatter: within a block, elements are ranked in index
-//             order with 64-lane ballots (8 ballots give the lanes that share
-//             a digit), per-wave digit counts combined in LDS.
+// radix_sort.rs:1-30): stable, so ties keep their input order; the values are
+// the input indices 0..n-1, which is what every caller sorts.  Only the key
+// bits that can be non-zero are sorted, in equal digits of at most
+// radix_plan's width.  Each pass is three launches:
+//   k_radix_hist     per-block digit histogram (blocks of 4096 keys, LDS atomics)
+//   k_radix_rows     per digit: exclusive scan of the blocks' counts, total
+//   k_radix_scatter  the digits' bases from the totals, then a stable scatter:
+//                    each wave ranks its 1024 consecutive keys in 16 rounds of
+//                    64 with ballots (the lanes that share a digit) and digit
+//                    counters of its own, with no barrier between the rounds,
+//                    and the block's keys leave through LDS in digit order.
+// What bounds a pass at 2 M keys is the scatter: a block's latency (its loads,
+// the ballots, whose rounds overlap bit by bit, the stage) with two blocks per
+// CU.  Wide digits trade passes for counters: 18 key bits (a 256^3 grid) are
+// two passes of 9 bits.  A key query of 2 M random particles takes 73 us
+// (scatter 18, histogram 5, rows 5 us per pass); three passes of 8 bits with
+// barriers in every round, unstaged stores and a three-launch scan took 154.
+#include <algorithm>
+
 #include "mpm_internal.hpp"
+#include "mpm_blockscan.hpp"
 
 namespace mpm {
 
 constexpr int SORT_THREADS = 256;
+constexpr int SORT_WAVES = SORT_THREADS / 64;
 constexpr int SORT_ITEMS = 16;
 constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;  // 4096
-constexpr int RADIX = 256;
+constexpr int MAX_DIGIT = 12;
 
 static inline uint32_t sort_blocks(uint32_t n) { return (n + SORT_TILE - 1) / SORT_TILE; }
 
-size_t radix_scratch_words(uint32_t n) {
-    // ping-pong keys + values, histogram (RADIX * blocks), its scan scratch
-    const size_t h = (size_t)RADIX * sort_blocks(n);
-    return 2 * (size_t)n + 2 * h + scan_scratch_words(h) + 64;
+// Digit width limit: the histogram table (2^width x blocks words, written and
+// read once per pass) stays within 1 MB up to 512 blocks (2 M keys); beyond,
+// 11 bits, because another pass over the keys costs more than the table.
+static inline int max_digit(uint32_t nb) {
+    return nb <= 64 ? MAX_DIGIT : (nb <= 128 ? 11 : (nb <= 256 ? 10 : (nb <= 512 ? 9 : 11)));
 }
 
-__global__ __launch_bounds__(SORT_THREADS) void k_hist(const uint32_t* __restrict__ keys, uint32_t n,
-                                                       int shift, uint32_t nblocks,
-                                                       uint32_t* __restrict__ hist) {
-    __shared__ uint32_t h[RADIX];
-    h[threadIdx.x] = 0u;
+struct RadixPlan {
+    int passes, width;
+};
+static inline RadixPlan radix_plan(uint32_t n, int bits) {
+    const int w = max_digit(sort_blocks(n)), b = std::max(bits, 1);
+    const int passes = (b + w - 1) / w;
+    return {passes, (b + passes - 1) / passes};
+}
+
+size_t radix_scratch_words(uint32_t n) {
+    // ping-pong keys + values, histogram table, digit totals
+    const uint32_t nb = sort_blocks(n);
+    return 2 * (size_t)n + ((size_t)nb << max_digit(nb)) + (1u << MAX_DIGIT) + 64;
+}
+
+uint32_t* radix_input(uint32_t* keys, uint32_t n, int bits, uint32_t* scratch) {
+    return radix_plan(n, bits).passes % 2 ? scratch : keys;
+}
+
+__global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
+                                                             int width, uint32_t* __restrict__ hist) {
+    extern __shared__ uint32_t lds[];
+    const uint32_t R = 1u << width;
+    for (uint32_t d = threadIdx.x; d < R; d += SORT_THREADS) lds[d] = 0u;
     __syncthreads();
     const uint32_t base = blockIdx.x * SORT_TILE;
+    uint32_t k[SORT_ITEMS];
+#pragma unroll
     for (int r = 0; r < SORT_ITEMS; ++r) {
-        uint32_t i = base + r * SORT_THREADS + threadIdx.x;
-        if (i < n) atomicAdd(&h[(keys[i] >> shift) & 0xffu], 1u);
+        const uint32_t i = base + r * SORT_THREADS + threadIdx.x;
+        k[r] = i < n ? keys[i] : 0u;
+    }
+    // keys in nearly sorted order put a wave on one digit, whose 64 adds to
+    // one word would run one after the other: such a wave adds once
+#pragma unroll
+    for (int r = 0; r < SORT_ITEMS; ++r) {
+        const uint32_t d = (k[r] >> shift) & (R - 1u);
+        const bool valid = base + r * SORT_THREADS + threadIdx.x < n;
+        const uint64_t all = __ballot(valid);
+        if (__ballot(valid && d == (uint32_t)__builtin_amdgcn_readfirstlane(int(d))) == all) {
+            if (valid && (threadIdx.x & 63u) == 0u) atomicAdd(&lds[d], (uint32_t)__popcll(all));
+        } else if (valid) {
+            atomicAdd(&lds[d], 1u);
+        }
     }
     __syncthreads();
-    hist[(size_t)threadIdx.x * nblocks + blockIdx.x] = h[threadIdx.x];
+    for (uint32_t d = threadIdx.x; d < R; d += SORT_THREADS) hist[(size_t)blockIdx.x * R + d] = lds[d];
 }
 
-__global__ __launch_bounds__(SORT_THREADS) void k_scatter(const uint32_t* __restrict__ kin,
-                                                          const uint32_t* __restrict__ vin,
-                                                          uint32_t* __restrict__ kout,
-                                                          uint32_t* __restrict__ vout, uint32_t n,
-                                                          int shift, uint32_t nblocks,
-                                                          const uint32_t* __restrict__ offs) {
-    constexpr int W = SORT_THREADS / 64;
-    __shared__ uint32_t base[RADIX];
-    __shared__ uint32_t cnt[W][RADIX];
+// hist is block-major ([block][digit], so that the kernels around this one
+// move whole rows): each digit's exclusive sum over the blocks in place, and
+// its total.  A block takes ROW_DIGITS digits; its threads split the blocks
+// into ROW_SEGS segments, whose sums one wave per digit scans.
+constexpr int ROW_DIGITS = 16;
+constexpr int ROW_SEGS = 64;
+__global__ __launch_bounds__(ROW_DIGITS * ROW_SEGS) void k_radix_rows(uint32_t* __restrict__ hist, uint32_t nblocks,
+                                                                      uint32_t R, uint32_t* __restrict__ total) {
+    __shared__ uint32_t part[ROW_SEGS][ROW_DIGITS + 1];
+    const uint32_t c = threadIdx.x % ROW_DIGITS, seg = threadIdx.x / ROW_DIGITS;
+    const uint32_t d = blockIdx.x * ROW_DIGITS + c;
+    const uint32_t len = (nblocks + ROW_SEGS - 1u) / ROW_SEGS;
+    const uint32_t b0 = min(seg * len, nblocks), b1 = min(b0 + len, nblocks);
+    uint32_t sum = 0u;
+    if (d < R)
+#pragma unroll 8
+        for (uint32_t b = b0; b < b1; ++b) sum += hist[(size_t)b * R + d];
+    part[seg][c] = sum;
+    __syncthreads();
+    const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;  // wave w scans digit w
+    {
+        const uint32_t v = part[lane][wave], incl = wave_incl_scan(v);
+        part[lane][wave] = incl - v;
+        if (lane == 63u && blockIdx.x * ROW_DIGITS + wave < R) total[blockIdx.x * ROW_DIGITS + wave] = incl;
+    }
+    __syncthreads();
+    if (d >= R) return;
+    uint32_t run = part[seg][c];
+#pragma unroll 8
+    for (uint32_t b = b0; b < b1; ++b) {
+        const uint32_t v = hist[(size_t)b * R + d];
+        hist[(size_t)b * R + d] = run;
+        run += v;
+    }
+}
+static_assert(ROW_SEGS == 64, "one lane per segment");
+
+// vin null: the values are the indices.  lb (may be null; single-pass sorts
+// only): receives the first position of every key in [0, n_lb].
+__global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* __restrict__ kin,
+                                                                const uint32_t* __restrict__ vin,
+                                                                uint32_t* __restrict__ kout,
+                                                                uint32_t* __restrict__ vout, uint32_t n, int shift,
+                                                                int width, const uint32_t* __restrict__ hist,
+                                                                const uint32_t* __restrict__ total,
+                                                                uint32_t* __restrict__ lb, uint32_t n_lb) {
+    extern __shared__ uint32_t lds[];
+    __shared__ uint32_t s_wave[64];
+    const uint32_t R = 1u << width;
+    uint32_t* base = lds;  // R words: where the block's keys of a digit go, less their place in the stage
+    uint16_t* cnt = reinterpret_cast<uint16_t*>(lds + R);  // [digit][wave]
+    uint32_t *skey = lds + R, *sval = skey + SORT_TILE;                      // the stage, once cnt is done with
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    base[tid] = offs[(size_t)tid * nblocks + blockIdx.x];
-    const uint64_t lt = (lane == 0) ? 0ull : (~0ull >> (64 - lane));
-    const uint32_t blk = blockIdx.x * SORT_TILE;
+    const uint32_t first = blockIdx.x * SORT_TILE + uint32_t(wave) * (SORT_ITEMS * 64);
+    uint32_t key[SORT_ITEMS], val[SORT_ITEMS];
+#pragma unroll
     for (int r = 0; r < SORT_ITEMS; ++r) {
+        const uint32_t i = first + r * 64 + lane;
+        key[r] = i < n ? kin[i] : 0u;
+        val[r] = vin && i < n ? vin[i] : i;
+    }
+    for (uint32_t i = tid; i < R * SORT_WAVES / 2; i += SORT_THREADS) lds[R + i] = 0u;
+    // thread t holds the R / 256 digits from t R / 256 on
+    constexpr uint32_t PER = (1u << MAX_DIGIT) / SORT_THREADS;
+    const uint32_t per = R > uint32_t(SORT_THREADS) ? R / SORT_THREADS : 1u, d0 = uint32_t(tid) * per;
+    uint32_t tot[PER], at[PER];
+    uint32_t sum = 0u;
 #pragma unroll
-        for (int w = 0; w < W; ++w) cnt[w][tid] = 0u;
-        __syncthreads();
-        const uint32_t i = blk + r * SORT_THREADS + tid;
-        const bool valid = i < n;
-        uint32_t key = 0u, val = 0u, d = 0u;
-        if (valid) {
-            key = kin[i];
-            val = vin[i];
-            d = (key >> shift) & 0xffu;
-        }
-        uint64_t same = __ballot(valid);
+    for (uint32_t q = 0; q < PER; ++q) {
+        const bool on = q < per && d0 + q < R;
+        tot[q] = on ? total[d0 + q] : 0u;
+        at[q] = on ? hist[(size_t)blockIdx.x * R + d0 + q] : 0u;
+        sum += tot[q];
+    }
+    uint32_t run = block_excl_scan(sum, s_wave, (uint32_t*)nullptr);
 #pragma unroll
-        for (int bit = 0; bit < 8; ++bit) {
-            const bool on = (d >> bit) & 1u;
+    for (uint32_t q = 0; q < PER; ++q) {
+        if (q >= per || d0 + q >= R) continue;
+        if (lb && blockIdx.x == 0 && d0 + q <= n_lb) lb[d0 + q] = run;
+        at[q] += run;
+        run += tot[q];
+    }
+    if (lb && blockIdx.x == 0 && tid == 0 && n_lb >= R) lb[R] = n;
+    // the lanes of each round that share a digit: one bit of all rounds at a
+    // time, so that the rounds' ballots overlap
+    const uint64_t lt = (1ull << lane) - 1ull;
+    uint64_t same[SORT_ITEMS];
+#pragma unroll
+    for (int r = 0; r < SORT_ITEMS; ++r) same[r] = __ballot(first + r * 64 + lane < n);
+    for (int bit = shift; bit < shift + width; ++bit)
+#pragma unroll
+        for (int r = 0; r < SORT_ITEMS; ++r) {
+            const bool on = (key[r] >> bit) & 1u;
             const uint64_t m = __ballot(on);
-            same &= on ? m : ~m;
+            same[r] &= on ? m : ~m;
         }
-        const uint32_t rank = (uint32_t)__popcll(same & lt);
-        const bool leader = valid && (same & lt) == 0ull;
-        if (leader) cnt[wave][d] = (uint32_t)__popcll(same);
-        __syncthreads();
-        uint32_t pos = 0;
-        if (valid) {
-            uint32_t before = 0;
-            for (int w = 0; w < wave; ++w) before += cnt[w][d];
-            pos = base[d] + before + rank;
-        }
-        __syncthreads();
-        {
-            uint32_t tot = 0;
+    uint32_t rank[SORT_ITEMS];
 #pragma unroll
-            for (int w = 0; w < W; ++w) tot += cnt[w][tid];
-            base[tid] += tot;
+    for (int r = 0; r < SORT_ITEMS; ++r) {
+        rank[r] = 0u;
+        if (first + r * 64 + lane < n) {
+            // the wave's LDS accesses stay in program order: a round reads
+            // the counts that the rounds before it wrote
+            volatile uint16_t* c = &cnt[((key[r] >> shift) & (R - 1u)) * SORT_WAVES + uint32_t(wave)];
+            const uint32_t before = *c;
+            rank[r] = before + (uint32_t)__popcll(same[r] & lt);
+            if ((same[r] & lt) == 0ull) *c = uint16_t(before + (uint32_t)__popcll(same[r]));
         }
-        if (valid) {
-            kout[pos] = key;
-            vout[pos] = val;
+    }
+    __syncthreads();
+    // places in the stage: digits ascending, the waves' keys of a digit in order
+    static_assert(SORT_WAVES == 4, "four counters of a digit are one word");
+    uint64_t* cnt4 = reinterpret_cast<uint64_t*>(cnt);
+    uint64_t c4[PER];
+    uint32_t mine = 0u;
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) {
+        c4[q] = q < per && d0 + q < R ? cnt4[d0 + q] : 0ull;
+        mine += uint32_t(c4[q] & 0xffffu) + uint32_t((c4[q] >> 16) & 0xffffu) + uint32_t((c4[q] >> 32) & 0xffffu) +
+                uint32_t(c4[q] >> 48);
+    }
+    uint32_t place = block_excl_scan(mine, s_wave, (uint32_t*)nullptr);
+#pragma unroll
+    for (uint32_t q = 0; q < PER; ++q) {
+        if (q >= per || d0 + q >= R) continue;
+        base[d0 + q] = at[q] - place;
+        uint64_t out = 0ull;
+#pragma unroll
+        for (int w = 0; w < SORT_WAVES; ++w) {
+            out |= uint64_t(place) << (16 * w);
+            place += uint32_t(c4[q] >> (16 * w)) & 0xffffu;
         }
-        __syncthreads();
+        cnt4[d0 + q] = out;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < SORT_ITEMS; ++r)
+        rank[r] += cnt[((key[r] >> shift) & (R - 1u)) * SORT_WAVES + uint32_t(wave)];
+    __syncthreads();  // the stage overwrites the counters
+#pragma unroll
+    for (int r = 0; r < SORT_ITEMS; ++r) {
+        if (first + r * 64 + lane >= n) continue;
+        skey[rank[r]] = key[r];
+        sval[rank[r]] = val[r];
+    }
+    __syncthreads();
+    // staged order: a digit's keys leave as one run
+    const uint32_t held = min(n - blockIdx.x * SORT_TILE, uint32_t(SORT_TILE));
+#pragma unroll
+    for (int r = 0; r < SORT_ITEMS; ++r) {
+        const uint32_t i = r * SORT_THREADS + tid;
+        if (i >= held) continue;
+        const uint32_t k = skey[i], pos = base[(k >> shift) & (R - 1u)] + i;
+        kout[pos] = k;
+        vout[pos] = sval[i];
     }
 }
 
-hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, int bits,
-                            uint32_t* scratch, hipStream_t s) {
-    if (n <= 1 || bits <= 0) return hipSuccess;
+hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, int bits, uint32_t* scratch, uint32_t* lb,
+                            uint32_t n_lb, bool* lb_done, hipStream_t s) {
+    if (lb_done) *lb_done = false;
+    if (n == 0) return hipSuccess;
     const uint32_t nb = sort_blocks(n);
+    const RadixPlan plan = radix_plan(n, bits);
+    const uint32_t R = 1u << plan.width;
     uint32_t* k2 = scratch;
     uint32_t* v2 = scratch + n;
     uint32_t* hist = scratch + 2 * (size_t)n;
-    uint32_t* offs = hist + (size_t)RADIX * nb;
-    uint32_t* sscr = offs + (size_t)RADIX * nb;
-    const int passes = (bits + 7) / 8;
-    uint32_t *ka = keys, *va = vals, *kb = k2, *vb = v2;
-    for (int p = 0; p < passes; ++p) {
-        const int shift = 8 * p;
-        hipLaunchKernelGGL(k_hist, dim3(nb), dim3(SORT_THREADS), 0, s, ka, n, shift, nb, hist);
-        hipError_t e = exclusive_scan_u32(hist, offs, (size_t)RADIX * nb, sscr, nullptr, s);
-        if (e != hipSuccess) return e;
-        hipLaunchKernelGGL(k_scatter, dim3(nb), dim3(SORT_THREADS), 0, s, ka, va, kb, vb, n, shift, nb,
-                           offs);
-        uint32_t* t = ka;
-        ka = kb;
-        kb = t;
-        t = va;
-        va = vb;
-        vb = t;
+    uint32_t* total = hist + (size_t)R * nb;
+    const uint32_t* kin = radix_input(keys, n, bits, scratch);
+    const uint32_t* vin = nullptr;  // the first pass's values are the indices
+    const bool with_lb = lb && plan.passes == 1;
+    for (int p = 0; p < plan.passes; ++p) {
+        const int shift = plan.width * p;
+        uint32_t *kout = kin == keys ? k2 : keys, *vout = kin == keys ? v2 : vals;
+        hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(SORT_THREADS), R * 4, s, kin, n, shift, plan.width, hist);
+        hipLaunchKernelGGL(k_radix_rows, dim3((R + ROW_DIGITS - 1) / ROW_DIGITS), dim3(ROW_DIGITS * ROW_SEGS), 0, s, hist,
+                           nb, R, total);
+        hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(SORT_THREADS),
+                           R * 4 + std::max<uint32_t>(R * SORT_WAVES * 2, 2 * SORT_TILE * 4), s, kin, vin, kout,
+                           vout, n, shift, plan.width, hist, total, with_lb ? lb : nullptr, n_lb);
+        kin = kout;
+        vin = vout;
     }
-    if (ka != keys) {
-        hipError_t e = hipMemcpyAsync(keys, ka, (size_t)n * 4, hipMemcpyDeviceToDevice, s);
-        if (e != hipSuccess) return e;
-        e = hipMemcpyAsync(vals, va, (size_t)n * 4, hipMemcpyDeviceToDevice, s);
-        if (e != hipSuccess) return e;
-    }
+    if (lb_done) *lb_done = with_lb;
     return hipGetLastError();
 }
 
