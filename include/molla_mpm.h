@@ -203,7 +203,9 @@ int mpm_set_launch(mpm_sim* sim, uint32_t particle_blocks, uint32_t grid_blocks)
  *   particles_per_thread          1 or 2: particles each thread of the fused
  *                                 pass takes per chunk of the sorted layout
  *                                 (a chunk holds 256 x this many; shader
- *                                 model only, MPM_MODEL_CPUDIFF handles run 1);
+ *                                 model only, MPM_MODEL_CPUDIFF handles run 1;
+ *                                 until a configuration is set or tuned, a
+ *                                 handle of up to 131,072 particles runs 1);
  *   segment_tiles                 the chunk rule of the sorted layout; all
  *                                 keep a chunk inside one tile row, which
  *                                 bounds the LDS box of its scatter.  4 or

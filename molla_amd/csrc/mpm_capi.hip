@@ -120,6 +120,7 @@ struct mpm_sim {
     uint32_t pblocks = 0;
     uint32_t gblocks = 0;
     uint32_t ppt = 2;         // particles per thread asked for (shader model)
+    bool ppt_set = false;     // ... by the caller or the autotuner; else layout_ppt() may take one
     uint32_t seg_tiles = 6;   // chunk rule: 4 or 6 greedy rows of at most that many tiles, 8 aligned segments
     uint32_t chunk_ppt = 1;   // particles per thread of the current sorted chunk list
     // profiling
@@ -475,6 +476,19 @@ int clear_grid(mpm_sim* s) {
     return MPM_OK;
 }
 
+// Particles per thread of the fused layout (shader model).  Two share a
+// chunk's fixed costs, but a thread runs them one after the other, so a scene
+// whose chunks of two would leave CUs idle is faster with one: up to one chunk
+// of 512 per CU (256 CUs).  A frame alone, two against one: 6,001 particles
+// 295 / 206 us (4 substeps and host copies), 8,192 599 / 447 us (20
+// substeps), 50,000 567 / 457, 100,000 627 / 556 us (16); above the line
+// 200,003 759 / 851, 400,000 1125 / 1142 us.
+constexpr uint32_t ONE_PER_THREAD = 256u * 512u;
+uint32_t layout_ppt(const mpm_sim* s) {
+    if (s->sh[0].model != MPM_MODEL_SHADER) return 1u;
+    return !s->ppt_set && s->n <= ONE_PER_THREAD ? 1u : s->ppt;
+}
+
 // slot_of_id of the current slots, where a sort since has left it behind.
 int ensure_index(mpm_sim* s) {
     if (s->index_valid) return MPM_OK;
@@ -496,6 +510,9 @@ int sort_particles(mpm_sim* s, bool reorder) {
         int rc = ensure_index(s);
         if (rc != MPM_OK) return rc;
     }
+    // several particles per thread only for the shader model's fused layout
+    // (the differentiable model and its adjoint take one)
+    if (reorder) s->chunk_ppt = by_slot ? layout_ppt(s) : 1u;
     if (s->dry) {
         if (reorder) {
             s->ps_cur = 1 - s->ps_cur;
@@ -516,9 +533,6 @@ int sort_particles(mpm_sim* s, bool reorder) {
                                          s->stream));
         return MPM_OK;
     }
-    // several particles per thread only for the shader model's fused layout
-    // (the differentiable model and its adjoint take one)
-    s->chunk_ppt = (by_slot && s->sh[0].model == MPM_MODEL_SHADER) ? s->ppt : 1u;
     const uint32_t chunk_cap = CHUNK * s->chunk_ppt;
     mpm::LayoutArgs q{};
     q.scenes = s->d_scenes;
@@ -1424,6 +1438,7 @@ int autotune(mpm_sim* s, float dt, uint32_t trial, uint32_t* out_pb, uint32_t* o
     const uint32_t ses[] = {8u, 16u, 32u, 64u, 128u};
     const uint32_t gb0 = best_gb, se0 = best_se ? best_se : 16u;
     if (s->sh[0].model == MPM_MODEL_SHADER && s->p2g_mode == MPM_P2G_FUSED) {
+        s->ppt_set = true;
         for (uint32_t pp : {1u, 2u})
             for (uint32_t sg : {4u, 6u, 8u}) {
                 if (rc != MPM_OK) break;
@@ -1725,9 +1740,12 @@ int mpm_set_launch_config(mpm_sim* sim, const mpm_launch_config* cfg) {
     sim->pblocks = cfg->particle_blocks;
     sim->gblocks = cfg->grid_blocks;
     sim->sort_every = cfg->sort_every;
-    if (cfg->particles_per_thread != sim->ppt || cfg->segment_tiles != sim->seg_tiles) {
+    const uint32_t ppt0 = layout_ppt(sim);
+    const bool asked = cfg->particles_per_thread != sim->ppt;
+    sim->ppt = cfg->particles_per_thread;
+    sim->ppt_set = true;
+    if (asked || ppt0 != layout_ppt(sim) || cfg->segment_tiles != sim->seg_tiles) {
         // a new chunk list at the next step (a taped forward is not reversible after it)
-        sim->ppt = cfg->particles_per_thread;
         sim->seg_tiles = cfg->segment_tiles;
         if (sim->sorted) {
             sim->sorted = false;
@@ -1780,7 +1798,7 @@ int mpm_step_n_graph(mpm_sim* sim, float dt, uint32_t substeps) {
     GraphKey key{dtb, substeps, uint32_t(sim->p2g_mode), uint32_t(sim->ps_cur), uint32_t(sim->list_cur),
                  uint32_t(sim->grid_dirty), uint32_t(sort_start) | (sim->since_sort << 1), uint32_t(sim->write_vc),
                  sim->pblocks, sim->gblocks, sim->sort_every, uint32_t(sim->has_E),
-                 sim->ppt | (sim->seg_tiles << 4) | (sim->chunk_ppt << 8) | (uint32_t(sim->index_valid) << 12)};
+                 sim->ppt | (uint32_t(sim->ppt_set) << 2) | (sim->seg_tiles << 4) | (sim->chunk_ppt << 8) | (uint32_t(sim->index_valid) << 12)};
     auto it = sim->graphs.find(key);
     if (it == sim->graphs.end()) {
         // Lazily allocated tables must exist before capture.

@@ -68,3 +68,26 @@ def test_layout_shapes(sizes):
         log(f"{sizes} segment_tiles {seg}: {st['chunks']} chunks, x {e[0]:.1e} v {e[1]:.1e}")
         assert e[0] <= 1e-6 and e[1] <= 2e-5
         s.close()
+
+
+@pytest.mark.parametrize("n,G,cap", [(8192, 32, 256), (131072, 64, 256), (131073, 64, 512)])
+def test_default_chunk_size_follows_the_particle_count(n, G, cap):
+    # one particle per thread up to 131,072 particles, two beyond; a
+    # configuration that is set holds, and takes effect at the next step
+    scene = _scene(n, G, 3)
+    s = MpmSimulation(scene[0])
+    s.set_particles(scene[1])
+    s.step_n(1e-5, 1)
+    assert s.read_status()["chunks"] == _chunks([scene], cap, 6)
+    s.set_launch_config(particles_per_thread=2)
+    s.step_n(1e-5, 1)
+    st = s.read_status()
+    x = s.read_positions()
+    s.close()
+    assert abs(st["chunks"] - _chunks([scene], 512, 6)) <= 2  # the particles have moved a little
+    t = MpmSimulation(scene[0])
+    t.set_particles(scene[1])
+    t.set_launch_config(particles_per_thread=2)
+    t.step_n(1e-5, 2)
+    assert rel_err(x, t.read_positions()) <= 1e-6
+    t.close()
