@@ -324,6 +324,7 @@ mpm::GridDev griddev(mpm_sim* s) {
         g.slot_tile = s->slot_tile;
         g.pool_count = s->status + mpm::ST_POOL;
         g.pool_capacity = s->pool_cap;
+        g.defer_count = s->status + mpm::ST_DEFER;
     }
     return g;
 }
@@ -630,18 +631,21 @@ int grid_update(mpm_sim* s, float dt, bool zero_after, bool react = false) {
     const int parts = s->p2g_mode == MPM_P2G_FUSED ? 1 : 0;
     if (s->jacobi_iters > 0) {
         // Semi-implicit step (mpm.rs:2515-2530): the sweeps need this substep's
-        // tile flags, so the grid update keeps them and the clear follows.
-        HIP_TRY(s, mpm::launch_grid_update(s->d_scenes, g, s->list[s->list_cur], cur_count, nullptr, dt, 0, parts,
-                                           grid_blocks(s), s->stream, nullptr, rigid ? &rg : nullptr, grid_split(s)));
+        // dynamic-tile marks, so the grid update keeps them and the last sweep
+        // launch takes them off.
+        mpm::GridDev g0 = g;
+        g0.gv = mpm::implicit_first(s->gv, s->gv2, s->jacobi_iters);
+        HIP_TRY(s, mpm::launch_grid_update(s->d_scenes, g0, s->list[s->list_cur], cur_count,
+                                           zero_after ? s->status + mpm::ST_COUNT0 + nxt : nullptr, dt,
+                                           zero_after ? 2 : 0, parts, grid_blocks(s), s->stream, nullptr,
+                                           rigid ? &rg : nullptr, grid_split(s)));
         HIP_TRY(s, mpm::launch_implicit_sweeps(s->d_scenes, g, s->gv2, s->jacobi_iters, s->list[s->list_cur],
-                                               cur_count, dt, grid_blocks(s), s->stream, rigid ? &rg : nullptr));
+                                               cur_count, dt, grid_blocks(s),
+                                               zero_after ? s->status + mpm::ST_TICKET : nullptr, s->stream,
+                                               rigid ? &rg : nullptr));
         if (rg.wrench && !s->prescribed)
             HIP_TRY(s, mpm::launch_rigid_shell(s->d_scenes, g, s->list[s->list_cur], cur_count, dt, rg,
                                                grid_blocks(s), s->stream));
-        if (zero_after) {
-            HIP_TRY(s, mpm::launch_clear_tiles(g, s->list[s->list_cur], cur_count, grid_blocks(s), s->stream));
-            HIP_TRY(s, mpm::launch_set_u32(s->status + mpm::ST_COUNT0 + nxt, 0u, s->stream));
-        }
         return MPM_OK;
     }
     HIP_TRY(s, mpm::launch_grid_update(s->d_scenes, g, s->list[s->list_cur], cur_count,

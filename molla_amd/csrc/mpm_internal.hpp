@@ -42,10 +42,11 @@ constexpr uint32_t FAULT_NUMERICAL = 2u;
 // ST_COUNT0/1: the two dynamic active-tile lists; ST_SCOUNT: the static list.
 // Sparse tile pool: ST_POOL the tiles marked by the last substep (slots in
 // use, or the demand that overflowed the pool), ST_DEFER the particles whose
-// global-atomic scatter waits for the slots.
+// global-atomic scatter waits for the slots.  ST_TICKET: blocks of the last
+// sweep launch that are done (zero between launches).
 enum StatusWord : int {
     ST_FAULT = 0, ST_GATHERS = 1, ST_COUNT0 = 2, ST_COUNT1 = 3, ST_SCOUNT = 4, ST_ESCAPES = 5, ST_NCHUNKS = 6,
-    ST_FALLBACK = 7, ST_POOL = 8, ST_DEFER = 9, ST_WORDS = 10
+    ST_FALLBACK = 7, ST_POOL = 8, ST_DEFER = 9, ST_TICKET = 10, ST_WORDS = 11
 };
 
 struct SceneDev {
@@ -124,6 +125,7 @@ struct GridDev {
     const uint32_t* slot_tile;
     const uint32_t* pool_count;
     uint32_t pool_capacity;
+    uint32_t* defer_count;  // status[ST_DEFER], cleared by the grid update
     float4* gmp;          // atomic accumulation / final P2G kept for readback
     float4* gv;           // grid velocity (vx, vy, vz, m)
     uint32_t* tile_flag;  // FLAG_* bits
@@ -179,13 +181,15 @@ struct RigidDev;  // rigid bodies on the grid (mpm_rigid.hpp)
 
 // ---- sparse tile pool (mpm_kernels.hip) ----
 // Slots for the marked tiles (marks cleared), in arrival order; more marked
-// tiles than `capacity` latch FAULT_OVERFLOW.  status[ST_POOL] = marked tiles.
+// tiles than `capacity` latch FAULT_OVERFLOW.  status[ST_POOL] = marked tiles
+// (counted from the zero that the scattering pass before it leaves there).
 hipError_t launch_pool_compact(uint32_t* tile_mark, uint32_t total_tiles, uint32_t* tile_slot, uint32_t* slot_tile,
                                uint32_t capacity, uint32_t* status, hipStream_t s);
 // Marks of legacy rigid spheres (mark_rigids, mpm_active_tiles.wgsl:108-124).
 hipError_t launch_mark_spheres(const SceneDev* scenes, const RigidDev& rg, uint32_t* tile_mark, uint32_t capacity,
                                uint32_t* status, hipStream_t s);
-// The deferred global-atomic P2G of the particles listed in a.defer_list.
+// The deferred global-atomic P2G of the particles listed in a.defer_list
+// (status[ST_DEFER] of them; the grid update that follows clears the count).
 hipError_t launch_deferred_p2g(const StepArgs& a, int model, hipStream_t s);
 // Mass and momentum of the first `cells` storage cells (pool order).
 hipError_t launch_storage_to_host_layout(const float4* gmp, uint32_t cells, float* mass, float* mom, hipStream_t s);
@@ -193,6 +197,8 @@ hipError_t launch_storage_to_host_layout(const float4* gmp, uint32_t cells, floa
 // ---- launchers (mpm_kernels.hip) ----
 hipError_t launch_particle_pass(int mode, int model, const StepArgs& a, int ppt, int blocks,
                                 hipStream_t s);
+// zero_after: 0 keep the P2G total in gmp; 1 clear gmp and the flags but the
+// static bit; 2 as 1, but keep FLAG_DYN (the implicit sweeps read it).
 // keep (may be null): per-cell copy of the P2G total (m, p) of the listed tiles.
 // split: four waves per tile instead of one (same results; for scenes with no
 // more active tiles than blocks).
@@ -206,11 +212,14 @@ hipError_t launch_rigid_shell(const SceneDev* scenes, const GridDev& g, const ui
 hipError_t launch_zero_f64(double* p, uint32_t n, hipStream_t s);
 hipError_t launch_clear_tiles(const GridDev& g, const uint32_t* dlist, uint32_t* dcount, int blocks,
                               hipStream_t s, float4* also = nullptr);
-// `iters` semi-implicit Jacobi sweeps of g.gv over the active tiles (scratch:
-// a second cell buffer); the result is left in g.gv.  Tile flags must still
-// mark this substep's dynamic tiles (FLAG_DYN).
+// `iters` > 0 semi-implicit Jacobi sweeps over the active tiles: they start
+// from the buffer implicit_first() names (g.gv or the second cell buffer
+// `scratch`), where the grid update has to leave its velocities, and end in
+// g.gv.  Tile flags must still mark this substep's dynamic tiles (FLAG_DYN);
+// `ticket` (a zero word, or null) takes those marks off at the end.
+float4* implicit_first(float4* gv, float4* scratch, uint32_t iters);
 hipError_t launch_implicit_sweeps(const SceneDev* scenes, const GridDev& g, float4* scratch, uint32_t iters,
-                                  const uint32_t* dlist, const uint32_t* dcount, float dt, int blocks,
+                                  const uint32_t* dlist, const uint32_t* dcount, float dt, int blocks, uint32_t* ticket,
                                   hipStream_t s, const RigidDev* rigid = nullptr);
 hipError_t launch_set_u32(uint32_t* p, uint32_t v, hipStream_t s);
 hipError_t launch_snap_counters(const uint32_t* status, uint32_t* dst, hipStream_t s);
