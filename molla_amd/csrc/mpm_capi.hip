@@ -219,6 +219,8 @@ SceneDev make_scene(const mpm_scene_config& c, uint32_t tile_base, uint32_t mat_
     d.model = c.model;
     d.mat_base = mat_base;
     d.n_mat = c.n_materials;
+    d.pmass = c.particle_mass;
+    d.pvol = c.particle_volume;
     return d;
 }
 
@@ -858,49 +860,19 @@ int set_particles(mpm_sim* s, const uint32_t* counts, const float* pos, const fl
         s->pbase.push_back(acc);
         acc += counts[i];
     }
-    // host-built planes [0, n) of every component
-    std::vector<float> plane(std::max<size_t>(s->n, 1));
-    float* ps = s->ps[0];
-    auto put = [&](int comp) -> hipError_t {
-        return hipMemcpy(ps + (size_t)comp * s->cap, plane.data(), (size_t)s->n * 4, hipMemcpyHostToDevice);
-    };
-    for (int k = 0; k < 3; ++k) {
-        for (uint32_t p = 0; p < s->n; ++p) plane[p] = pos[3 * (size_t)p + k];
-        HIP_TRY(s, put(mpm::CX + k));
-        for (uint32_t p = 0; p < s->n; ++p) plane[p] = vel ? vel[3 * (size_t)p + k] : 0.0f;
-        HIP_TRY(s, put(mpm::CV + k));
-    }
-    std::fill(plane.begin(), plane.end(), 0.0f);
-    for (int k = 0; k < 9; ++k) HIP_TRY(s, put(mpm::CC + k));
-    HIP_TRY(s, put(mpm::CJP));
-    HIP_TRY(s, put(mpm::CMAT));
-    for (int k = 0; k < 9; ++k) {
-        std::fill(plane.begin(), plane.end(), (k % 4 == 0) ? 1.0f : 0.0f);
-        HIP_TRY(s, put(mpm::CF + k));
-    }
-    auto per_scene = [&](auto getter) {
-        for (uint32_t sc = 0; sc < s->n_scenes; ++sc)
-            for (uint32_t p = 0; p < counts[sc]; ++p) plane[s->pbase[sc] + p] = getter(s->cfg[sc]);
-    };
-    per_scene([](const mpm_scene_config& c) { return c.particle_mass; });
-    HIP_TRY(s, put(mpm::CMASS));
-    per_scene([](const mpm_scene_config& c) { return c.particle_volume; });
-    HIP_TRY(s, put(mpm::CVOL));
-    per_scene([](const mpm_scene_config& c) { return c.youngs; });
-    HIP_TRY(s, put(mpm::CE));
-    for (uint32_t p = 0; p < s->n; ++p) {
-        uint32_t id = p;
-        std::memcpy(&plane[p], &id, 4);
-    }
-    HIP_TRY(s, put(mpm::CID));
+    // positions and velocities go up as they are; a kernel makes the planes
+    float* dpos = s->staging;
+    float* dvel = s->staging + 3 * (size_t)s->n;
+    if (s->n) HIP_TRY(s, hipMemcpyAsync(dpos, pos, (size_t)s->n * 12, hipMemcpyHostToDevice, s->stream));
+    if (s->n && vel) HIP_TRY(s, hipMemcpyAsync(dvel, vel, (size_t)s->n * 12, hipMemcpyHostToDevice, s->stream));
     s->ps_cur = 0;
-    s->index_valid = false;
-    int rc = ensure_index(s);
-    if (rc != MPM_OK) return rc;
-    rc = build_chunks(s);
+    int rc = build_chunks(s);
     if (rc != MPM_OK) return rc;
     rc = upload_scenes(s);
     if (rc != MPM_OK) return rc;
+    HIP_TRY(s, mpm::launch_init_particles(s->d_scenes, s->d_chunks, s->n_chunks, dpos, vel ? dvel : nullptr, s->ps[0],
+                                          s->cap, s->slot_of_id, s->stream));
+    s->index_valid = true;
     s->has_E = 0;
     s->sorted = false;
     s->diff_steps = 0;

@@ -71,6 +71,8 @@ struct SceneDev {
     uint32_t pbase;
     uint32_t n;
     uint32_t cbase;  // first chunk of the scene
+    float pmass;     // particle mass and volume of set_particles
+    float pvol;
 };
 
 // A contiguous run of particle slots of one scene, processed by one block.
@@ -252,6 +254,11 @@ struct RecordArgs {
 // receives the new index; the records are written by blocks of the same launch.
 hipError_t launch_reorder(const float* src, float* dst, uint32_t cap, const uint32_t* src_slot, uint32_t n,
                           uint32_t* slot_of_id, const RecordArgs& rec, hipStream_t s);
+// Every plane of a new particle set, slot = id: positions and velocities (null:
+// zero) as n x 3 words, F = I, C = 0, jp = 0, material 0, the scene's mass,
+// volume and E; and its slot_of_id.  chunks: the unsorted list.
+hipError_t launch_init_particles(const SceneDev* scenes, const Chunk* chunks, uint32_t n_chunks, const float* pos,
+                                 const float* vel, float* ps, uint32_t cap, uint32_t* slot_of_id, hipStream_t s);
 hipError_t launch_index_slots(const float* ps, uint32_t cap, uint32_t* slot_of_id, uint32_t n,
                               hipStream_t s);
 // `ncomp` (1, 3 or 9) planes <-> n x ncomp words in original order; ids: the
