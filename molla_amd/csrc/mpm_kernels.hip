@@ -18,6 +18,7 @@
 // f32 atomics instead.
 #include <algorithm>
 
+#include "mpm_blockscan.hpp"
 #include "mpm_rigid.hpp"
 #include "mpm_scatter.hpp"
 
@@ -1502,20 +1503,23 @@ hipError_t launch_gather_prepare(const StepArgs& a, float* affine, int blocks, h
 //      order, in an LDS list.
 //   2. In batches of GATHER_RECS the listed particles' weights, node offsets
 //      and momentum rows go to LDS, one particle per thread.
-//   3. Four waves sum the batch: wave z takes the tile's cells of one z, 16
-//      cells x (m, px, py, pz), and walks the records that reach that z.
+//   3. Each of the block's 16 waves takes one x-row of the tile (4 cells x
+//      (m, px, py, pz) = 16 lanes) and the records that reach its row; its
+//      four groups of 16 lanes form the terms of four records at once, which
+//      the first group then adds in list order.
 // A cell's sum is one serial chain, so what bounds the kernel is the length of
 // that chain and the time of each link, not bytes or flops.  One wave per tile
 // that walked every particle of the 27 tiles through dependent global loads
-// took 2,352 us on 16,384 sand particles in a 32^3 grid; here a link is a few
-// LDS reads issued GATHER_FLY records ahead of their sums, only the ~1/16 of
-// the candidates that reach a wave's cells are links, and the same launch
-// takes 115 us (163 us with two records in flight and separate x and y
-// weights; 132 us with four).
-constexpr int GATHER_THREADS = 512;
-constexpr int GATHER_PER = 4;
-constexpr int GATHER_FLY = 8;
-constexpr int GATHER_RECS = 256;
+// took 2,352 us on 16,384 sand particles in a 32^3 grid, one wave per z with
+// eight records' LDS reads in flight 115 us; here a link is an add, its terms
+// come 16 at a time, only the ~1/32 of the candidates that reach a wave's row
+// are links, and the same launch takes 62 us.
+constexpr int GATHER_THREADS = 1024;
+constexpr int GATHER_WAVES = GATHER_THREADS / 64;
+constexpr int GATHER_PER = 2;
+constexpr int GATHER_FLY = 4;  // records per lane group and step
+constexpr int GATHER_STEP = 4 * GATHER_FLY;
+constexpr int GATHER_RECS = 512;
 constexpr int GATHER_LIST = 4096;
 
 // A particle relative to a tile: the weight product of the tile's 4 x 4 cell
@@ -1529,48 +1533,23 @@ struct GatherRec {
     float4 row[4];
 };
 
-// A group of GATHER_FLY records as one lane (cell and channel) sees them.
-struct GatherLink {
-    float w[GATHER_FLY], dx[GATHER_FLY], dy[GATHER_FLY];
-    float2 z[GATHER_FLY];
-    float4 r[GATHER_FLY];
-    __device__ __forceinline__ void fetch(const GatherRec* rec, const uint16_t* at, int cx, int cy, int cz, int ch) {
-#pragma unroll
-        for (int u = 0; u < GATHER_FLY; ++u) {
-            const GatherRec& q = rec[at[u]];
-            w[u] = q.wxy[cx + 4 * cy];
-            dx[u] = q.dx[cx];
-            dy[u] = q.dy[cy];
-            z[u] = q.z[cz];
-            r[u] = q.row[ch];
-        }
-    }
-    __device__ __forceinline__ float add(float acc) const {
-#pragma unroll
-        for (int u = 0; u < GATHER_FLY; ++u) {
-            const float v = acc + w[u] * z[u].x * (r[u].x + r[u].y * dx[u] + r[u].z * dy[u] + r[u].w * z[u].y);
-            acc = w[u] < 0.f ? acc : v;
-        }
-        return acc;
-    }
-};
-
 __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const uint32_t* __restrict__ tile_scene,
                                                                const uint32_t* __restrict__ lb,
                                                                const float* __restrict__ aff,
                                                                const uint32_t* __restrict__ list,
                                                                const uint32_t* __restrict__ count) {
     __shared__ GatherRec rec[GATHER_RECS + 1];  // the last one reaches no cell
-    __shared__ uint32_t zmask[GATHER_RECS];  // bit z: the record reaches the tile's cells of that z
-    __shared__ uint16_t zlist[4][GATHER_RECS + GATHER_FLY];
+    __shared__ uint16_t rows[GATHER_RECS];      // bit y + 4 z: the record reaches that x-row of the tile
+    __shared__ uint16_t wlist[GATHER_WAVES][GATHER_RECS + GATHER_STEP];
     __shared__ uint32_t slots[GATHER_LIST];
     __shared__ uint32_t rbeg[9], roff[10];
-    __shared__ uint32_t wcnt[GATHER_PER][GATHER_THREADS / 64];
+    __shared__ uint32_t wcnt[64];  // [GATHER_PER][GATHER_WAVES]
+    static_assert(GATHER_PER * GATHER_WAVES <= 64, "one lane per count");
     const uint32_t n = *count;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const uint32_t cap = a.cap;
-    // wave z < 4 sums cells (lane >> 2 & 3, lane >> 4, z), channel lane & 3
-    const int ch = lane & 3, cx = (lane >> 2) & 3, cy = lane >> 4, cz = wave & 3;
+    // lane: channel, cell of the wave's row, record of a step's four
+    const int ch = lane & 3, cx = (lane >> 2) & 3, grp = lane >> 4, cy = wave & 3, cz = wave >> 2;
     if (tid < int(sizeof(GatherRec) / 4)) reinterpret_cast<float*>(&rec[GATHER_RECS])[tid] = tid < 16 ? -1.f : 0.f;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const uint32_t t = list[i];
@@ -1634,17 +1613,17 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                     for (int k = 0; k < 3; ++k) hit[u] = hit[u] && r[k] >= -3 && r[k] <= 2;
                 }
                 m[u] = __ballot(hit[u]);
-                if (lane == 0) wcnt[u][wave] = uint32_t(__popcll(m[u]));
+                if (lane == 0) wcnt[u * GATHER_WAVES + wave] = uint32_t(__popcll(m[u]));
             }
             __syncthreads();
-            uint32_t at = held;
+            // places after the slots held: candidates ascend over (u, wave, lane)
+            const uint32_t c = lane < GATHER_PER * GATHER_WAVES ? wcnt[lane] : 0u, incl = wave_incl_scan(c);
 #pragma unroll
-            for (int u = 0; u < GATHER_PER; ++u)
-                for (int w = 0; w < GATHER_THREADS / 64; ++w) {
-                    if (w == wave && hit[u]) slots[at + uint32_t(__popcll(m[u] & ((1ull << lane) - 1ull)))] = slot[u];
-                    at += wcnt[u][w];
-                }
-            held = at;
+            for (int u = 0; u < GATHER_PER; ++u) {
+                const uint32_t at = held + (uint32_t)__shfl(int(incl - c), u * GATHER_WAVES + wave, 64);
+                if (hit[u]) slots[at + uint32_t(__popcll(m[u] & ((1ull << lane) - 1ull)))] = slot[u];
+            }
+            held += (uint32_t)__shfl(int(incl), 63, 64);
             __syncthreads();
             // sum the list when another round might not fit, and at the end
             const bool last = c0 + GATHER_THREADS * GATHER_PER >= total;
@@ -1652,7 +1631,7 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
             for (uint32_t b0 = 0; b0 < held; b0 += GATHER_RECS) {
                 const uint32_t cnt = min(held - b0, uint32_t(GATHER_RECS));
                 if (tid < GATHER_RECS) {
-                    uint32_t zm = 0u;
+                    uint32_t rm = 0u;
                     if (uint32_t(tid) < cnt) {
                         const uint32_t j = slots[b0 + uint32_t(tid)];
                         int r[3];
@@ -1664,59 +1643,72 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                         const float mass = a.ps[(size_t)CMASS * cap + j];
                         GatherRec& q = rec[tid];
                         float w[3][4], d[3][4];  // weight (-1: none) and node offset of the tile's cells
+                        uint32_t in[3] = {0u, 0u, 0u};
 #pragma unroll
                         for (int k = 0; k < 3; ++k) {
                             float wk[3];
                             quad_weights(fx[k], wk);
 #pragma unroll
-                            for (int c = 0; c < 4; ++c) {
-                                const int off = r[k] + c;
-                                w[k][c] = off == 0 ? wk[0] : (off == 1 ? wk[1] : (off == 2 ? wk[2] : -1.0f));
-                                d[k][c] = (float(off) - fx[k]) * sc.dx;
-                                if (k == 2 && off >= 0 && off <= 2) zm |= 1u << c;
+                            for (int c2 = 0; c2 < 4; ++c2) {
+                                const int off = r[k] + c2;
+                                w[k][c2] = off == 0 ? wk[0] : (off == 1 ? wk[1] : (off == 2 ? wk[2] : -1.0f));
+                                d[k][c2] = (float(off) - fx[k]) * sc.dx;
+                                if (off >= 0 && off <= 2) in[k] |= 1u << c2;
                             }
                         }
 #pragma unroll
-                        for (int c = 0; c < 4; ++c) {
+                        for (int z = 0; z < 4; ++z)
+                            if (in[2] & (1u << z)) rm |= in[1] << (4 * z);
 #pragma unroll
-                            for (int b = 0; b < 4; ++b)
-                                q.wxy[c + 4 * b] = w[0][c] < 0.f || w[1][b] < 0.f ? -1.0f : w[0][c] * w[1][b];
-                            q.dx[c] = d[0][c];
-                            q.dy[c] = d[1][c];
-                            q.z[c] = make_float2(w[2][c], d[2][c]);
+                        for (int c2 = 0; c2 < 4; ++c2) {
+#pragma unroll
+                            for (int y = 0; y < 4; ++y)
+                                q.wxy[c2 + 4 * y] = w[0][c2] < 0.f || w[1][y] < 0.f ? -1.0f : w[0][c2] * w[1][y];
+                            q.dx[c2] = d[0][c2];
+                            q.dy[c2] = d[1][c2];
+                            q.z[c2] = make_float2(w[2][c2], d[2][c2]);
                         }
                         q.row[0] = make_float4(mass, 0.f, 0.f, 0.f);
 #pragma unroll
                         for (int k = 0; k < 3; ++k)
                             q.row[1 + k] = make_float4(A[9 + k], A[3 * k], A[3 * k + 1], A[3 * k + 2]);
                     }
-                    zmask[tid] = zm;
+                    rows[tid] = uint16_t(rm);
                 }
                 __syncthreads();
-                if (wave < 4) {
-                    // the wave's own list: records reaching its z, in order,
-                    // filled up to whole groups with the record that adds nothing
-                    uint32_t len = 0u;
-                    for (uint32_t g = 0; g < cnt; g += 64) {
-                        const bool on = (zmask[g + uint32_t(lane)] >> cz) & 1u;
-                        const uint64_t m = __ballot(on);
-                        if (on) zlist[wave][len + uint32_t(__popcll(m & ((1ull << lane) - 1ull)))] = uint16_t(g + lane);
-                        len += uint32_t(__popcll(m));
+                // the wave's own list: records reaching its row, in order,
+                // filled up to a whole step with the record that adds nothing
+                uint32_t len = 0u;
+                for (uint32_t g = 0; g < cnt; g += 64) {
+                    const bool on = (rows[g + uint32_t(lane)] >> wave) & 1u;
+                    const uint64_t mm = __ballot(on);
+                    if (on) wlist[wave][len + uint32_t(__popcll(mm & ((1ull << lane) - 1ull)))] = uint16_t(g + lane);
+                    len += uint32_t(__popcll(mm));
+                }
+                if (lane < GATHER_STEP) wlist[wave][len + uint32_t(lane)] = uint16_t(GATHER_RECS);
+                __builtin_amdgcn_wave_barrier();
+                for (uint32_t g = 0; g < len; g += GATHER_STEP) {
+                    float v[GATHER_FLY];
+#pragma unroll
+                    for (int f = 0; f < GATHER_FLY; ++f) {
+                        const GatherRec& q = rec[wlist[wave][g + uint32_t(4 * f + grp)]];
+                        const float w = q.wxy[cx + 4 * cy];
+                        const float2 z = q.z[cz];
+                        const float4 r = q.row[ch];
+                        const float p = w * z.x * (r.x + r.y * q.dx[cx] + r.z * q.dy[cy] + r.w * z.y);
+                        v[f] = w < 0.f ? 0.f : p;
                     }
-                    if (lane < GATHER_FLY) zlist[wave][len + uint32_t(lane)] = uint16_t(GATHER_RECS);
-                    __builtin_amdgcn_wave_barrier();
-                    for (uint32_t g = 0; g < len; g += GATHER_FLY) {
-                        GatherLink q;
-                        q.fetch(rec, zlist[wave] + g, cx, cy, cz, ch);
-                        __builtin_amdgcn_sched_barrier(0);  // all of the group's reads before its sums
-                        acc = q.add(acc);
-                    }
+                    // the four groups' terms, in list order, to the first group
+#pragma unroll
+                    for (int f = 0; f < GATHER_FLY; ++f)
+#pragma unroll
+                        for (int h = 0; h < 4; ++h) acc += h == 0 ? v[f] : __shfl_down(v[f], 16 * h, 64);
                 }
                 __syncthreads();
             }
             held = 0u;
         }
-        if (wave < 4) {
+        if (grp == 0) {
             const int G = int(sc.G);
             const bool valid = 4 * tc[0] + cx < G && 4 * tc[1] + cy < G && 4 * tc[2] + cz < G;
             const uint32_t c = (t << 6) | uint32_t(cx | (cy << 2) | (cz << 4));

@@ -17,7 +17,8 @@ pytestmark = pytest.mark.gpu
 @pytest.mark.parametrize("n,G,lo,hi,window", [
     (1, 16, 6.2, 6.3, 0),
     (5003, 16, 7.0, 9.0, 0),      # more stencils on a tile than the slot list holds
-    (257, 16, 6.0, 7.5, 0),       # one record more than a batch
+    (257, 16, 6.0, 7.5, 0),       # half a batch and one record
+    (513, 16, 7.0, 8.9, 0),       # one record more than a batch
     (3001, 19, 2.6, 15.9, 0),     # ragged grid: the last tile has three cells
     (2048, 18, 4.0, 13.0, 5),     # window: grid indices start at cell 5
 ])
