@@ -56,13 +56,238 @@ __device__ __forceinline__ double warp_sum(double v) {
 
 }  // namespace
 
+// A block's box of grid cells in LDS for the gathers of its particles: the
+// bounding box of their stencils, cells outside the grid as zeros (which add
+// nothing to any of the gathers' sums).  `cells` null: not staged.
+struct Staged {
+    const float4* cells;
+    int o[3], d[3];
+    // index of the node (0, 0, 0) of a stencil at b, or -1 when not inside
+    __device__ __forceinline__ int find(const int* b) const {
+        bool in = cells != nullptr;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) in = in && b[k] >= o[k] && b[k] + 2 < o[k] + d[k];
+        return in ? (b[0] - o[0]) + d[0] * ((b[1] - o[1]) + d[1] * (b[2] - o[2])) : -1;
+    }
+};
+
+// Stencil base of the particle in `slot` of planes ps; `on`: the particle is
+// the block's and its stencil has not left its sorted neighbourhood (an
+// escaped one reads global memory and would blow up the box).
+__device__ __forceinline__ bool staged_base(const StepArgs& a, const SceneDev& sc, const Chunk& ch, const float* ps,
+                                            uint32_t slot, bool active, int* b) {
+    b[0] = b[1] = b[2] = 0;
+    if (!active) return false;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+        b[k] = int(floorf(fmaf(ps[(size_t)(CX + k) * a.cap + slot] - sc.origin[k], sc.inv_dx, -0.5f)));
+    return !stencil_escapes(sc, ch, a.sorted_keys[slot], b);
+}
+
+// Joins the waves' stencil boxes (min and max base per axis) of up to two
+// gathers through `red`.  Every thread calls it.
+constexpr int NO_BASE = 0x3fffffff;
+template <int N>
+__device__ __forceinline__ void block_boxes(const bool (&on)[N], const int (&b)[N][3], int (*red)[WAVES][6],
+                                            int (&lo)[N][3], int (&hi)[N][3]) {
+    const int lane = threadIdx.x & 63, wave = wave_id();
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const int l = wave_min(on[n] ? b[n][k] : NO_BASE), h = wave_max(on[n] ? b[n][k] : -NO_BASE);
+            if (lane == 0) {
+                red[n][wave][k] = l;
+                red[n][wave][3 + k] = h;
+            }
+        }
+    __syncthreads();
+#pragma unroll
+    for (int n = 0; n < N; ++n)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            lo[n][k] = red[n][0][k];
+            hi[n][k] = red[n][0][3 + k];
+#pragma unroll
+            for (int w = 1; w < WAVES; ++w) {
+                lo[n][k] = min(lo[n][k], red[n][w][k]);
+                hi[n][k] = max(hi[n][k], red[n][w][3 + k]);
+            }
+            lo[n][k] = __builtin_amdgcn_readfirstlane(lo[n][k]);
+            hi[n][k] = __builtin_amdgcn_readfirstlane(hi[n][k]);
+        }
+}
+
+// Loads the cells of stencils with bases lo .. hi into `to` (LDS_CELLS); the
+// caller puts a barrier before the first read.
+__device__ __forceinline__ Staged stage_box(const SceneDev& sc, const float4* __restrict__ grid, const int* lo,
+                                            const int* hi, float4* to) {
+    Staged s;
+    s.cells = nullptr;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        s.o[k] = lo[k];
+        s.d[k] = hi[k] - lo[k] + 3;
+    }
+    // no base at all (hi < lo), or a box that cannot fit
+    if (s.d[0] < 3 || s.d[1] < 3 || s.d[2] < 3 || s.d[0] > LDS_CELLS || s.d[1] > LDS_CELLS || s.d[2] > LDS_CELLS ||
+        s.d[0] * s.d[1] > LDS_CELLS || s.d[0] * s.d[1] * s.d[2] > LDS_CELLS)
+        return s;
+    const int vol = s.d[0] * s.d[1] * s.d[2];
+    const float inv_x = 1.0f / float(s.d[0]), inv_y = 1.0f / float(s.d[1]);
+    constexpr int PER = 4;  // loads in flight per thread
+#pragma unroll 1
+    for (int i0 = 0; i0 < vol; i0 += PER * BLOCK) {
+        float4 v[PER];
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const int i = i0 + int(threadIdx.x) + u * BLOCK;
+            v[u] = make_float4(0.f, 0.f, 0.f, 0.f);
+            // exact for the box's small integers, as in stage_gather_box
+            const int r = int((float(i) + 0.5f) * inv_x), z = int((float(r) + 0.5f) * inv_y);
+            const int ix = s.o[0] + (i - r * s.d[0]), iy = s.o[1] + (r - z * s.d[1]), iz = s.o[2] + z;
+            if (i < vol && in_grid(sc, ix, iy, iz)) v[u] = grid[cell_index(sc, ix, iy, iz)];
+        }
+#pragma unroll
+        for (int u = 0; u < PER; ++u) {
+            const int i = i0 + int(threadIdx.x) + u * BLOCK;
+            if (i < vol) to[i] = v[u];
+        }
+    }
+    s.cells = to;
+    return s;
+}
+
+// The gathers' arithmetic is written out with its fused operations (and the
+// compiler's own fusing switched off): a gradient's last bits depend on which
+// products are rounded, and as the compiler fuses within a basic block only,
+// they would change with every change of the code around the sums.
+__device__ __forceinline__ float dot3(float a0, float b0, float a1, float b1, float a2, float b2) {
+#pragma clang fp contract(off)
+    return fmaf(a2, b2, fmaf(a0, b0, a1 * b1));
+}
+
+// Quadratic stencil of a position: first node, offset, weights, derivatives.
+struct AdjStencil {
+    int b[3];
+    float fx[3], w[3][3], dw[3][3];
+    __device__ __forceinline__ AdjStencil(const SceneDev& sc, const float* x) {
+#pragma clang fp contract(off)
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+            const float r = x[k] - sc.origin[k];
+            const float bf = floorf(fmaf(r, sc.inv_dx, -0.5f));
+            b[k] = int(bf);
+            fx[k] = fmaf(r, sc.inv_dx, -bf);
+            const float p = 1.5f - fx[k], q = fx[k] - 1.0f, s = fx[k] - 0.5f;
+            w[k][0] = 0.5f * p * p;
+            w[k][1] = fmaf(-q, q, 0.75f);
+            w[k][2] = 0.5f * s * s;
+            dw[k][0] = -p;
+            dw[k][1] = -2.0f * q;
+            dw[k][2] = s;
+        }
+    }
+};
+
+// One z-plane of the sums over a stencil's nodes g, row by row (fixed j, k):
+// with the node term
+// u_jk + i c0, u_jk = u0 + j c1 + k c2, and h = (MASS ? m g.x : 0) + G . u,
+// G the node's vector (MASS: g.yzw, else g.xyz),
+//   S = sum w G,  M = sum w G (i, j, k)^T,
+//   acc = (sum w1 w2 Sdw, sum dw1 w2 Sw, sum w1 dw2 Sw),
+// Sw = sum_i w0 h, Sdw = sum_i dw0 h.  fetch(i, j, k) gives a node, zero
+// outside the grid.
+template <bool MASS, class Fetch>
+__device__ __forceinline__ void adj_plane(int k, float wk, float dwk, const AdjStencil& st, float m, const float* u0,
+                                          const float* c0, const float* c1, const float* c2, Fetch fetch, float* S,
+                                          float* M, float* acc) {
+#pragma clang fp contract(off)
+    const float wi[3] = {0.f, st.w[0][1], 2.0f * st.w[0][2]};
+#pragma unroll
+    for (int j = 0; j < 3; ++j) {
+        const float wjk = st.w[1][j] * wk;
+        float u[3], rs[3] = {0.f, 0.f, 0.f}, ri[3] = {0.f, 0.f, 0.f}, Sw = 0.f, Sdw = 0.f;
+#pragma unroll
+        for (int r = 0; r < 3; ++r) u[r] = fmaf(float(k), c2[r], fmaf(float(j), c1[r], u0[r]));
+#pragma unroll
+        for (int i = 0; i < 3; ++i) {
+            const float4 g = fetch(i, j, k);
+            const float G[3] = {MASS ? g.y : g.x, MASS ? g.z : g.y, MASS ? g.w : g.z};
+            float v[3], h;
+#pragma unroll
+            for (int r = 0; r < 3; ++r) v[r] = fmaf(float(i), c0[r], u[r]);
+            if (!MASS) {
+                h = dot3(v[0], G[0], v[1], G[1], v[2], G[2]);
+            } else {
+                h = i == 0 ? fmaf(m, g.x, v[0] * G[0]) : fmaf(v[0], G[0], m * g.x);
+                h = fmaf(v[2], G[2], fmaf(v[1], G[1], h));
+            }
+            Sw = fmaf(st.w[0][i], h, Sw);
+            Sdw = fmaf(st.dw[0][i], h, Sdw);
+#pragma unroll
+            for (int r = 0; r < 3; ++r) {
+                rs[r] = fmaf(st.w[0][i], G[r], rs[r]);
+                if (i > 0) ri[r] = fmaf(wi[i], G[r], ri[r]);
+            }
+        }
+#pragma unroll
+        for (int r = 0; r < 3; ++r) {
+            S[r] = fmaf(wjk, rs[r], S[r]);
+            M[3 * r] = fmaf(wjk, ri[r], M[3 * r]);
+            M[3 * r + 1] = fmaf(float(j) * wjk, rs[r], M[3 * r + 1]);
+            M[3 * r + 2] = fmaf(float(k) * wjk, rs[r], M[3 * r + 2]);
+        }
+        acc[0] = fmaf(wjk, Sdw, acc[0]);
+        acc[1] = fmaf(st.dw[1][j] * wk, Sw, acc[1]);
+        acc[2] = fmaf(st.w[1][j] * dwk, Sw, acc[2]);
+    }
+}
+
+// The sums over a stencil from the block's staged cells, or from global memory
+// for waves with a stencil outside them (rolled: it is rare, and 27 nodes of
+// code twice crowd the instruction cache: 340 us of k_adj_fused instead of 367;
+// the common one rolled as well costs 26 instead of 13 us of k_adj_p2g on one
+// scene of 65,536 particles).
+template <bool MASS>
+__device__ __forceinline__ void adj_gather(const SceneDev& sc, const float4* __restrict__ grid, const Staged& box,
+                                           const AdjStencil& st, float m, const float* u0, const float* c0,
+                                           const float* c1, const float* c2, float* S, float* M, float* acc) {
+#pragma unroll
+    for (int r = 0; r < 3; ++r) S[r] = acc[r] = M[3 * r] = M[3 * r + 1] = M[3 * r + 2] = 0.f;
+    const int at = box.find(st.b);
+    if (__all(at >= 0)) {
+        const int dx = box.d[0], dxy = box.d[0] * box.d[1];
+        const auto fetch = [&](int i, int j, int k) { return box.cells[at + i + dx * j + dxy * k]; };
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+            adj_plane<MASS>(k, st.w[2][k], st.dw[2][k], st, m, u0, c0, c1, c2, fetch, S, M, acc);
+    } else {
+        const auto fetch = [&](int i, int j, int k) {
+            const int ix = st.b[0] + i, iy = st.b[1] + j, iz = st.b[2] + k;
+            return in_grid(sc, ix, iy, iz) ? grid[cell_index(sc, ix, iy, iz)] : make_float4(0.f, 0.f, 0.f, 0.f);
+        };
+        float w0 = st.w[2][0], w1 = st.w[2][1], d0 = st.dw[2][0], d1 = st.dw[2][1];
+#pragma unroll 1
+        for (int k = 0; k < 3; ++k) {
+            adj_plane<MASS>(k, w0, d0, st, m, u0, c0, c1, c2, fetch, S, M, acc);
+            w0 = w1;
+            d0 = d1;
+            w1 = st.w[2][2];
+            d1 = st.dw[2][2];
+        }
+    }
+}
+
 // Reverse of G2P and of the x/F advance for the particle in `slot` of the
 // pre-state a.ps with grid velocity a.gv (mpm_adjoint.rs:196-305).  On entry
 // gx, gv, gC, gF are dJ/d(post-state); on return gx holds the G2P part of
 // dJ/dx (plus the pass-through), gF = (I + dt C')^T dJ/dF', and sp the
 // scatter of dJ/d(grid v).
 __device__ __forceinline__ void adj_g2p_particle(const StepArgs& a, const SceneDev& sc, const Chunk& ch, uint32_t slot,
-                                                 float* gx, const float* gv, const float* gC, float* gF, Scatter& sp) {
+                                                 float* gx, const float* gv, const float* gC, float* gF, Scatter& sp,
+                                                 const Staged& box) {
+#pragma clang fp contract(off)
     const uint32_t cap = a.cap;
     const float* __restrict__ ps = a.ps;
     const float dt = a.dt;
@@ -76,103 +301,51 @@ __device__ __forceinline__ void adj_g2p_particle(const StepArgs& a, const SceneD
     float gvp[3], B[9];
     const float s4 = 4.0f * sc.inv_dx * sc.inv_dx;
 #pragma unroll
-    for (int k = 0; k < 3; ++k) gvp[k] = gx[k] * dt + gv[k];
+    for (int k = 0; k < 3; ++k) gvp[k] = fmaf(gx[k], dt, gv[k]);
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-            B[3 * i + j] = s4 * (gC[3 * i + j] + dt * (gF[3 * i] * F[3 * j] + gF[3 * i + 1] * F[3 * j + 1] +
-                                                       gF[3 * i + 2] * F[3 * j + 2]));
-    float xp[3], fx[3], w[3][3], dw[3][3];
-    int b[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        xp[k] = (x[k] - sc.origin[k]) * sc.inv_dx;
-        const float bf = floorf(xp[k] - 0.5f);
-        b[k] = int(bf);
-        fx[k] = xp[k] - bf;
-        quad_weights(fx[k], w[k]);
-        dw[k][0] = -(1.5f - fx[k]);
-        dw[k][1] = -2.0f * (fx[k] - 1.0f);
-        dw[k][2] = fx[k] - 0.5f;
-    }
+            B[3 * i + j] = s4 * fmaf(dt, dot3(gF[3 * i], F[3 * j], gF[3 * i + 1], F[3 * j + 1], gF[3 * i + 2],
+                                              F[3 * j + 2]),
+                                     gC[3 * i + j]);
+    const AdjStencil st(sc, x);
     // G2P reverse (mpm_adjoint.rs:249-305): with B = 4/dx^2 dJ/dC',
-    //   dJ/dx += sum grad(w) (v_i . (dJ/dv' + B d)) - B^T sum w v_i,
-    // summed row by row (fixed j, k): with d = ((i, j, k) - fx) dx the node
-    // term is u_jk + i b0 (b0 = dx B[:, 0]); with Sw = sum_i w0 h and
-    // Sdw = sum_i dw0 h the gradient sum is
-    //   idx (sum w1 w2 Sdw, sum dw1 w2 Sw, sum w1 dw2 Sw),
-    // and C' = 4/dx^2 sum w v_i d^T = 4/dx (Mv - vn fx^T), Mv = sum w v_i (i, j, k)^T.
+    //   dJ/dx += sum grad(w) (v_i . (dJ/dv' + B d)) - B^T sum w v_i
+    // in adj_gather's rows: d = ((i, j, k) - fx) dx, the gradient sum is
+    // idx acc, and C' = 4/dx^2 sum w v_i d^T = 4/dx (M - S fx^T).
     const float dx = sc.dx, idx = sc.inv_dx;
-    float b0[3], u0[3];
+    float c0[3], c1[3], c2[3], u0[3];
 #pragma unroll
     for (int r = 0; r < 3; ++r) {
-        b0[r] = dx * B[3 * r];
-        u0[r] = gvp[r] - (b0[r] * fx[0] + dx * B[3 * r + 1] * fx[1] + dx * B[3 * r + 2] * fx[2]);
+        c0[r] = dx * B[3 * r];
+        c1[r] = dx * B[3 * r + 1];
+        c2[r] = dx * B[3 * r + 2];
+        u0[r] = gvp[r] - dot3(c0[r], st.fx[0], c1[r], st.fx[1], c2[r], st.fx[2]);
     }
-    const float wi[3] = {0.f, w[0][1], 2.0f * w[0][2]};
-    float vn[3] = {0.f, 0.f, 0.f}, Mv[9], acc[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < 9; ++k) Mv[k] = 0.f;
-    for (int k = 0; k < 3; ++k)
-        for (int j = 0; j < 3; ++j) {
-            const float wjk = w[1][j] * w[2][k];
-            float u[3], rs[3] = {0.f, 0.f, 0.f}, ri[3] = {0.f, 0.f, 0.f}, Sw = 0.f, Sdw = 0.f;
-#pragma unroll
-            for (int r = 0; r < 3; ++r) u[r] = u0[r] + float(j) * (dx * B[3 * r + 1]) + float(k) * (dx * B[3 * r + 2]);
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const int ix = b[0] + i, iy = b[1] + j, iz = b[2] + k;
-                if (!in_grid(sc, ix, iy, iz)) continue;
-                const float4 g = a.gv[cell_index(sc, ix, iy, iz)];
-                const float h = g.x * (u[0] + float(i) * b0[0]) + g.y * (u[1] + float(i) * b0[1]) +
-                                g.z * (u[2] + float(i) * b0[2]);
-                Sw += w[0][i] * h;
-                Sdw += dw[0][i] * h;
-                rs[0] += w[0][i] * g.x;
-                rs[1] += w[0][i] * g.y;
-                rs[2] += w[0][i] * g.z;
-                if (i > 0) {
-                    ri[0] += wi[i] * g.x;
-                    ri[1] += wi[i] * g.y;
-                    ri[2] += wi[i] * g.z;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                vn[r] += wjk * rs[r];
-                Mv[3 * r] += wjk * ri[r];
-                Mv[3 * r + 1] += float(j) * wjk * rs[r];
-                Mv[3 * r + 2] += float(k) * wjk * rs[r];
-            }
-            acc[0] += wjk * Sdw;
-            acc[1] += dw[1][j] * w[2][k] * Sw;
-            acc[2] += w[1][j] * dw[2][k] * Sw;
-        }
+    float vn[3], Mv[9], acc[3];
+    adj_gather<false>(sc, a.gv, box, st, 0.f, u0, c0, c1, c2, vn, Mv, acc);
     float Cn[9];
 #pragma unroll
     for (int r = 0; r < 3; ++r)
 #pragma unroll
-        for (int c = 0; c < 3; ++c) Cn[3 * r + c] = s4 * dx * (Mv[3 * r + c] - vn[r] * fx[c]);
+        for (int c = 0; c < 3; ++c) Cn[3 * r + c] = s4 * dx * fmaf(-vn[r], st.fx[c], Mv[3 * r + c]);
 #pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        acc[k] = acc[k] * idx - (B[k] * vn[0] + B[3 + k] * vn[1] + B[6 + k] * vn[2]);
-        gx[k] += acc[k];
-    }
+    for (int k = 0; k < 3; ++k) gx[k] += fmaf(acc[k], idx, -dot3(B[k], vn[0], B[3 + k], vn[1], B[6 + k], vn[2]));
     // dJ/dF (pre) = (I + dt C')^T dJ/dF'
     float nF[9];
 #pragma unroll
     for (int i = 0; i < 3; ++i)
 #pragma unroll
         for (int j = 0; j < 3; ++j)
-            nF[3 * i + j] = gF[3 * i + j] + dt * (Cn[i] * gF[j] + Cn[3 + i] * gF[3 + j] + Cn[6 + i] * gF[6 + j]);
+            nF[3 * i + j] = fmaf(dt, dot3(Cn[i], gF[j], Cn[3 + i], gF[3 + j], Cn[6 + i], gF[6 + j]), gF[3 * i + j]);
 #pragma unroll
     for (int k = 0; k < 9; ++k) gF[k] = nF[k];
     // dJ/d(grid v_i) += w (dJ/dv' + B d): the P2G form with m = 0
 #pragma unroll
     for (int k = 0; k < 3; ++k) {
-        sp.b[k] = b[k];
-        sp.fx[k] = fx[k];
+        sp.b[k] = st.b[k];
+        sp.fx[k] = st.fx[k];
         sp.mv[k] = gvp[k];
     }
 #pragma unroll
@@ -182,9 +355,51 @@ __device__ __forceinline__ void adj_g2p_particle(const StepArgs& a, const SceneD
     sp.esc = stencil_escapes(sc, ch, a.sorted_keys[slot], sp.b);
 }
 
+// P2G reverse (mpm_adjoint.rs:389-487): with gw = sum w dJ/dp_i and
+// T = sum w dJ/dp_i d^T:  dJ/dv = m gw, dJ/dC = m T, dJ/dstress = 4/dx^2 T,
+// dJ/dx = sum grad(w) (dJ/dp_i . (m v + A d) + m dJ/dm_i) - A^T gw, in
+// adj_gather's rows with T = dx (M - gw fx^T).  A = m C + 4/dx^2 stress
+// (stress = -dt vol P F^T) as the forward scattered it: the tape holds it in
+// the planes `aff`, so the FP64 SVD is not live across the gather.
+__device__ __forceinline__ void adj_p2g_gather(const StepArgs& a, const float4* __restrict__ gadj,
+                                               const float* __restrict__ aff, const SceneDev& sc, uint32_t slot, float m,
+                                               float* gx, float* gv, float* T, const Staged& box) {
+#pragma clang fp contract(off)
+    const uint32_t cap = a.cap;
+    const float* __restrict__ ps = a.ps;
+    float x[3], v[3], A[9];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        x[k] = ps[(size_t)(CX + k) * cap + slot];
+        v[k] = ps[(size_t)(CV + k) * cap + slot];
+    }
+#pragma unroll
+    for (int k = 0; k < 9; ++k) A[k] = aff[(size_t)k * cap + slot];
+    const AdjStencil st(sc, x);
+    const float dx = sc.dx, idx = sc.inv_dx;
+    float c0[3], c1[3], c2[3], u0[3];
+#pragma unroll
+    for (int r = 0; r < 3; ++r) {
+        c0[r] = dx * A[3 * r];
+        c1[r] = dx * A[3 * r + 1];
+        c2[r] = dx * A[3 * r + 2];
+        u0[r] = fmaf(v[r], m, -dot3(c0[r], st.fx[0], c1[r], st.fx[1], c2[r], st.fx[2]));
+    }
+    float gw[3], Mt[9], acc[3];
+    adj_gather<true>(sc, gadj, box, st, m, u0, c0, c1, c2, gw, Mt, acc);
+#pragma unroll
+    for (int r = 0; r < 3; ++r)
+#pragma unroll
+        for (int c = 0; c < 3; ++c) T[3 * r + c] = dx * fmaf(-gw[r], st.fx[c], Mt[3 * r + c]);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        gx[k] += fmaf(acc[k], idx, -dot3(A[k], gw[0], A[3 + k], gw[1], A[6 + k], gw[2]));
+        gv[k] = m * gw[k];
+    }
+}
+
 // Reverse of P2G, of the stress and of the SVD for the particle in `slot`
-// of the pre-state a.ps, with the P2G affine A the forward scattered (the
-// planes `aff`), gathering (dJ/dm, dJ/dp) from gadj
+// of the pre-state a.ps, gathering (dJ/dm, dJ/dp) from gadj
 // (mpm_adjoint.rs:389-487, mpm_cpu_diff.rs:330-379, dense3.rs:321-372).  On
 // entry gx, gF hold the reverse G2P's output; on return gx, gv, gC, gF are
 // dJ/d(pre-state), gE has dJ/dE_p added, and (amu, alam) are the particle's
@@ -192,97 +407,13 @@ __device__ __forceinline__ void adj_g2p_particle(const StepArgs& a, const SceneD
 __device__ __forceinline__ void adj_p2g_particle(const StepArgs& a, const float4* __restrict__ gadj,
                                                  const float* __restrict__ aff, const SceneDev& sc, uint32_t slot,
                                                  float* gx, float* gF, float* gv, float* gC, float& gE, double& amu,
-                                                 double& alam) {
+                                                 double& alam, const Staged& box) {
     const uint32_t cap = a.cap;
     const float* __restrict__ ps = a.ps;
     const float dt = a.dt;
-    float x[3], v[3], A[9];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        x[k] = ps[(size_t)(CX + k) * cap + slot];
-        v[k] = ps[(size_t)(CV + k) * cap + slot];
-    }
-    // A = m C + 4/dx^2 stress (stress = -dt vol P F^T) as the forward scattered
-    // it: the tape holds it, so the FP64 SVD is not live across the gather
-#pragma unroll
-    for (int k = 0; k < 9; ++k) A[k] = aff[(size_t)k * cap + slot];
     const float m = ps[(size_t)CMASS * cap + slot];
-    float mv[3] = {m * v[0], m * v[1], m * v[2]};
-    float xp[3], fx[3], w[3][3], dw[3][3];
-    int b[3];
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        xp[k] = (x[k] - sc.origin[k]) * sc.inv_dx;
-        const float bf = floorf(xp[k] - 0.5f);
-        b[k] = int(bf);
-        fx[k] = xp[k] - bf;
-        quad_weights(fx[k], w[k]);
-        dw[k][0] = -(1.5f - fx[k]);
-        dw[k][1] = -2.0f * (fx[k] - 1.0f);
-        dw[k][2] = fx[k] - 0.5f;
-    }
-    // P2G reverse (mpm_adjoint.rs:389-487): with gw = sum w dJ/dp_i and
-    // T = sum w dJ/dp_i d^T:  dJ/dv = m gw, dJ/dC = m T, dJ/dstress = 4/dx^2 T,
-    // dJ/dx = sum grad(w) (dJ/dp_i . (m v + A d) + m dJ/dm_i) - A^T gw,
-    // summed row by row as in the reverse G2P (A d = u_jk - m v + i a0,
-    // a0 = dx A[:, 0]) with T = dx (Mt - gw fx^T), Mt = sum w dJ/dp_i (i, j, k)^T.
-    const float dx = sc.dx, idx = sc.inv_dx;
-    float a0[3], u0[3];
-#pragma unroll
-    for (int r = 0; r < 3; ++r) {
-        a0[r] = dx * A[3 * r];
-        u0[r] = mv[r] - (a0[r] * fx[0] + dx * A[3 * r + 1] * fx[1] + dx * A[3 * r + 2] * fx[2]);
-    }
-    const float wi[3] = {0.f, w[0][1], 2.0f * w[0][2]};
-    float gw[3] = {0.f, 0.f, 0.f}, Mt[9], gpos[3] = {0.f, 0.f, 0.f};
-#pragma unroll
-    for (int k = 0; k < 9; ++k) Mt[k] = 0.f;
-    for (int k = 0; k < 3; ++k)
-        for (int j = 0; j < 3; ++j) {
-            const float wjk = w[1][j] * w[2][k];
-            float u[3], rs[3] = {0.f, 0.f, 0.f}, ri[3] = {0.f, 0.f, 0.f}, Sw = 0.f, Sdw = 0.f;
-#pragma unroll
-            for (int r = 0; r < 3; ++r) u[r] = u0[r] + float(j) * (dx * A[3 * r + 1]) + float(k) * (dx * A[3 * r + 2]);
-#pragma unroll
-            for (int i = 0; i < 3; ++i) {
-                const int ix = b[0] + i, iy = b[1] + j, iz = b[2] + k;
-                if (!in_grid(sc, ix, iy, iz)) continue;
-                const float4 g = gadj[cell_index(sc, ix, iy, iz)];
-                const float h = m * g.x + g.y * (u[0] + float(i) * a0[0]) + g.z * (u[1] + float(i) * a0[1]) +
-                                g.w * (u[2] + float(i) * a0[2]);
-                Sw += w[0][i] * h;
-                Sdw += dw[0][i] * h;
-                rs[0] += w[0][i] * g.y;
-                rs[1] += w[0][i] * g.z;
-                rs[2] += w[0][i] * g.w;
-                if (i > 0) {
-                    ri[0] += wi[i] * g.y;
-                    ri[1] += wi[i] * g.z;
-                    ri[2] += wi[i] * g.w;
-                }
-            }
-#pragma unroll
-            for (int r = 0; r < 3; ++r) {
-                gw[r] += wjk * rs[r];
-                Mt[3 * r] += wjk * ri[r];
-                Mt[3 * r + 1] += float(j) * wjk * rs[r];
-                Mt[3 * r + 2] += float(k) * wjk * rs[r];
-            }
-            gpos[0] += wjk * Sdw;
-            gpos[1] += dw[1][j] * w[2][k] * Sw;
-            gpos[2] += w[1][j] * dw[2][k] * Sw;
-        }
     float T[9];
-#pragma unroll
-    for (int r = 0; r < 3; ++r)
-#pragma unroll
-        for (int c = 0; c < 3; ++c) T[3 * r + c] = dx * (Mt[3 * r + c] - gw[r] * fx[c]);
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-        gpos[k] = gpos[k] * idx - (A[k] * gw[0] + A[3 + k] * gw[1] + A[6 + k] * gw[2]);
-        gx[k] += gpos[k];
-        gv[k] = m * gw[k];
-    }
+    adj_p2g_gather(a, gadj, aff, sc, slot, m, gx, gv, T, box);
     // corotated-SVK PK1 from the FP64 SVD (mpm_cpu_diff.rs:279-287)
     float F[9];
 #pragma unroll
@@ -425,8 +556,9 @@ __device__ __forceinline__ void add_chunk_mu_lambda(double* gml, uint32_t ci, do
 }
 
 // ---------------------------------------------------------------------------
-__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3))) void k_adj_g2p(AdjArgs q) {
+__global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_g2p(AdjArgs q) {
     __shared__ ScatterLdsT<true> L;
+    __shared__ int red[1][WAVES][6];
     const StepArgs& a = q.a;
     const uint32_t cap = a.cap;
     float* __restrict__ adj = q.adj;
@@ -436,6 +568,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3))) v
         const Chunk ch = a.chunks[ci];
         const SceneDev sc = a.scenes[ch.scene];
         const uint32_t slot = ch.start + threadIdx.x;
+        int b[1][3], lo[1][3], hi[1][3];
+        const bool on[1] = {staged_base(a, sc, ch, a.ps, slot, threadIdx.x < ch.count, b[0])};
+        block_boxes<1>(on, b, red, lo, hi);
+        const Staged st = stage_box(sc, a.gv, lo[0], hi[0], reinterpret_cast<float4*>(&L.acc[0][0]));
+        __syncthreads();
         Scatter sp;
         sp.on = false;
         sp.esc = false;
@@ -451,7 +588,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3))) v
                 gC[k] = adj[(size_t)(AC + k) * cap + slot];
                 gF[k] = adj[(size_t)(AF + k) * cap + slot];
             }
-            adj_g2p_particle(a, sc, ch, slot, gx, gv, gC, gF, sp);
+            adj_g2p_particle(a, sc, ch, slot, gx, gv, gC, gF, sp, st);
 #pragma unroll
             for (int k = 0; k < 3; ++k) adj[(size_t)(AX + k) * cap + slot] = gx[k];
 #pragma unroll
@@ -529,6 +666,8 @@ __global__ __launch_bounds__(256) void k_adj_grid(const SceneDev* __restrict__ s
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_p2g(AdjArgs q) {
     __shared__ double red[2][WAVES];
+    __shared__ float4 cells[LDS_CELLS];
+    __shared__ int bred[1][WAVES][6];
     const StepArgs& a = q.a;
     const uint32_t cap = a.cap;
     float* __restrict__ adj = q.adj;
@@ -538,6 +677,11 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         const Chunk ch = a.chunks[ci];
         const SceneDev sc = a.scenes[ch.scene];
         const uint32_t slot = ch.start + threadIdx.x;
+        int b[1][3], lo[1][3], hi[1][3];
+        const bool on[1] = {staged_base(a, sc, ch, a.ps, slot, threadIdx.x < ch.count, b[0])};
+        block_boxes<1>(on, b, bred, lo, hi);
+        const Staged st = stage_box(sc, q.gadj, lo[0], hi[0], cells);
+        __syncthreads();
         double amu = 0.0, alam = 0.0;
         if (threadIdx.x < ch.count) {
             float gx[3], gv[3], gC[9], gF[9];
@@ -546,7 +690,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 #pragma unroll
             for (int k = 0; k < 9; ++k) gF[k] = adj[(size_t)(AF + k) * cap + slot];
             float gE = adj[(size_t)AE * cap + slot];
-            adj_p2g_particle(a, q.gadj, q.aff, sc, slot, gx, gF, gv, gC, gE, amu, alam);
+            adj_p2g_particle(a, q.gadj, q.aff, sc, slot, gx, gF, gv, gC, gE, amu, alam, st);
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
                 adj[(size_t)(AX + k) * cap + slot] = gx[k];
@@ -567,9 +711,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 // the same particle: dJ/d(state k) stays in registers.  Valid when no
 // particle of either substep scatters with global atomics (the host checks
 // the recompute's escape and fallback counters), so gadj is only read here.
+// The FP64 SVD's registers leave two waves per SIMD, too few to hide 54
+// dependent 16-byte gathers from L2 per particle, so both gathers' boxes are
+// staged in the scatter's LDS first, with a round of coalesced loads: 128
+// scenes of 4 k to 32 k particles 440 us before, 340 now, one of 65,536
+// particles 29.7 and 24.3.  What is left is the FP64 arithmetic.
 __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) void k_adj_fused(AdjArgs q, const float* ps_prev, const float4* gv_prev) {
     __shared__ ScatterLdsT<true> L;
     __shared__ double red[2][WAVES];
+    __shared__ int bred[2][WAVES][6];
+    static_assert(sizeof(L.acc) >= 2 * LDS_CELLS * sizeof(float4), "two boxes of grid cells before the scatter");
     const StepArgs& a = q.a;
     StepArgs ap = q.a;
     ap.ps = ap.ps_out = const_cast<float*>(ps_prev);
@@ -583,6 +734,16 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         const SceneDev sc = a.scenes[ch.scene];
         const uint32_t slot = ch.start + threadIdx.x;
         const bool active = threadIdx.x < ch.count;
+        // both gathers' boxes (dJ/d grid of this substep, grid velocity of the
+        // previous one) in the scatter's space, loaded at once
+        int b[2][3], lo[2][3], hi[2][3];
+        const bool on[2] = {staged_base(a, sc, ch, a.ps, slot, active, b[0]),
+                            staged_base(a, sc, ch, ap.ps, slot, active, b[1])};
+        block_boxes<2>(on, b, bred, lo, hi);
+        float4* cells = reinterpret_cast<float4*>(&L.acc[0][0]);
+        const Staged st = stage_box(sc, q.gadj, lo[0], hi[0], cells);
+        const Staged stp = stage_box(sc, ap.gv, lo[1], hi[1], cells + LDS_CELLS);
+        __syncthreads();
         double amu = 0.0, alam = 0.0;
         float gx[3], gv[3], gC[9], gF[9];
         if (active) {
@@ -591,7 +752,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
 #pragma unroll
             for (int k = 0; k < 9; ++k) gF[k] = adj[(size_t)(AF + k) * cap + slot];
             float gE = adj[(size_t)AE * cap + slot];
-            adj_p2g_particle(a, q.gadj, q.aff, sc, slot, gx, gF, gv, gC, gE, amu, alam);
+            adj_p2g_particle(a, q.gadj, q.aff, sc, slot, gx, gF, gv, gC, gE, amu, alam, st);
             adj[(size_t)AE * cap + slot] = gE;
         }
         add_chunk_mu_lambda(q.gml, ci, amu, alam, red);
@@ -599,7 +760,7 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(2, 2))) v
         sp.on = false;
         sp.esc = false;
         if (active) {
-            adj_g2p_particle(ap, sc, ch, slot, gx, gv, gC, gF, sp);
+            adj_g2p_particle(ap, sc, ch, slot, gx, gv, gC, gF, sp, stp);
 #pragma unroll
             for (int k = 0; k < 3; ++k) adj[(size_t)(AX + k) * cap + slot] = gx[k];
 #pragma unroll
