@@ -1493,44 +1493,50 @@ hipError_t launch_gather_prepare(const StepArgs& a, float* affine, int blocks, h
     return hipGetLastError();
 }
 
-// One block per active tile.  For each cell, particles of the 27 neighbour
-// tiles are summed in tile order dx + 3 dy + 9 dz, then in ascending sorted
-// slot (mpm_deterministic_p2g.wgsl:100-144): a fixed order, so the result is
-// bitwise repeatable.  The 27 tiles are nine x-rows of consecutive keys, i.e.
-// nine slot ranges of the tile lower-bound table, already in that order.
+// One block per active tile.  For each cell, the particles of the 27 neighbour
+// tiles are listed in tile order dx + 3 dy + 9 dz, then in ascending sorted
+// slot (mpm_deterministic_p2g.wgsl:100-144), and summed in a fixed order, so
+// the result is bitwise repeatable: 16 sums of every 16th particle, then a
+// tree, which rounds less than one serial sum (5,003 particles over a few
+// tiles: momentum 2.0e-7 off instead of 1.7e-6).  The 27 tiles are nine x-rows
+// of consecutive keys, i.e. nine slot ranges of the tile lower-bound table,
+// already in that order.
 //   1. The block tests the ranges' particles, GATHER_PER per thread at once,
 //      and keeps the slots whose stencil reaches the tile (about 1 in 8), in
 //      order, in an LDS list.
 //   2. In batches of GATHER_RECS the listed particles' weights, node offsets
 //      and momentum rows go to LDS, one particle per thread.
-//   3. Each of the block's 16 waves takes one x-row of the tile (4 cells x
-//      (m, px, py, pz) = 16 lanes) and the records that reach its row; its
-//      four groups of 16 lanes form the terms of four records at once, which
-//      the first group then adds in list order.
-// A cell's sum is one serial chain, so what bounds the kernel is the length of
-// that chain and the time of each link, not bytes or flops.  One wave per tile
-// that walked every particle of the 27 tiles through dependent global loads
-// took 2,352 us on 16,384 sand particles in a 32^3 grid, one wave per z with
-// eight records' LDS reads in flight 115 us; here a link is an add, its terms
-// come 16 at a time, only the ~1/32 of the candidates that reach a wave's row
-// are links, and the same launch takes 62 us.
+//   3. Each of the block's 16 waves takes one x-row of the tile and the records
+//      that reach its row, 16 at a time: a lane sums one channel of the row's
+//      four cells over every 16th record, and the 16 partial sums are added in
+//      a fixed tree at the end.
+// One wave per tile that walked every particle of the 27 tiles through
+// dependent global loads took 2,352 us on 16,384 sand particles in a 32^3 grid.
+// With the records in LDS, reading them is what counts: one wave per z with a
+// lane per cell and channel 115 us, a wave per row with 16 lanes per record
+// 62 us (36 LDS instructions per 16 records, 12 of them to bring the terms to
+// one serial sum); a lane per record and channel reads each record once for
+// four cells, 6 LDS instructions per 16 records: 38 us, and 35 with a batch's
+// loads issued before the sums of the one before.
 constexpr int GATHER_THREADS = 1024;
 constexpr int GATHER_WAVES = GATHER_THREADS / 64;
-constexpr int GATHER_PER = 2;
-constexpr int GATHER_FLY = 4;  // records per lane group and step
-constexpr int GATHER_STEP = 4 * GATHER_FLY;
+constexpr int GATHER_PER = 4;
+constexpr int GATHER_FLY = 2;  // records per lane in flight
+constexpr int GATHER_STEP = 16 * GATHER_FLY;
 constexpr int GATHER_RECS = 512;
-constexpr int GATHER_LIST = 4096;
+constexpr int GATHER_LIST = 8192;
 
-// A particle relative to a tile: the weight product of the tile's 4 x 4 cell
-// columns in x and y (-1: the stencil misses the column), the weights in z,
-// the node offsets per axis and cell, and the four channels as
-// c + r0 d0 + r1 d1 + r2 d2 (mass: r = 0).
-struct GatherRec {
-    float wxy[16];
-    float dx[4], dy[4];
-    float2 z[4];
+// A particle relative to a tile: the four channels as c + r0 d0 + r1 d1 + r2 d2
+// (mass: r = 0), the weight product of the tile's 4 x 4 cell columns in x and y
+// (-1: the stencil misses the column), weight and node offset in z, node offset
+// in y, and in x the first cell's offset in cells and the fraction.
+struct alignas(16) GatherRec {
     float4 row[4];
+    float4 wxy[4];
+    float2 z[4];
+    float4 dy;
+    float2 x;
+    float pad[6];  // 52 words: 16 records' rows lie in different LDS banks
 };
 
 __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const uint32_t* __restrict__ tile_scene,
@@ -1548,9 +1554,10 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
     const uint32_t n = *count;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const uint32_t cap = a.cap;
-    // lane: channel, cell of the wave's row, record of a step's four
-    const int ch = lane & 3, cx = (lane >> 2) & 3, grp = lane >> 4, cy = wave & 3, cz = wave >> 2;
-    if (tid < int(sizeof(GatherRec) / 4)) reinterpret_cast<float*>(&rec[GATHER_RECS])[tid] = tid < 16 ? -1.f : 0.f;
+    // lane: channel, record of a step's 16; wave: the tile's row
+    const int ch = lane & 3, grp = lane >> 2, cy = wave & 3, cz = wave >> 2;
+    if (tid < int(sizeof(GatherRec) / 4))
+        reinterpret_cast<float*>(&rec[GATHER_RECS])[tid] = tid >= 16 && tid < 32 ? -1.f : 0.f;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const uint32_t t = list[i];
         const SceneDev sc = a.scenes[tile_scene[t]];
@@ -1575,17 +1582,17 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
         }
         __syncthreads();
         const uint32_t total = roff[9];
-        // base cell and fractional offset of a slot's particle on each axis
-        auto stencil = [&](uint32_t slot, int* r, float* fx) {
+        // base cell relative to the tile and fractional offset of a position
+        auto stencil = [&](const float* x, int* r, float* fx) {
 #pragma unroll
             for (int k = 0; k < 3; ++k) {
-                const float xp = (a.ps[(size_t)(CX + k) * cap + slot] - sc.origin[k]) * sc.inv_dx;
+                const float xp = (x[k] - sc.origin[k]) * sc.inv_dx;
                 const float bf = floorf(xp - 0.5f);
                 fx[k] = xp - bf;
                 r[k] = 4 * tc[k] - (int(bf) - sc.window[k]);  // offset of the tile's first cell
             }
         };
-        float acc = 0.f;
+        float acc[4] = {0.f, 0.f, 0.f, 0.f};
         uint32_t held = 0u;  // slots in the list (block-uniform)
         for (uint32_t c0 = 0; c0 < total; c0 += GATHER_THREADS * GATHER_PER) {
             uint32_t slot[GATHER_PER];
@@ -1608,7 +1615,9 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                 int r[3];
                 float fx[3];
                 if (hit[u]) {
-                    stencil(slot[u], r, fx);
+                    const float x[3] = {a.ps[(size_t)CX * cap + slot[u]], a.ps[(size_t)(CX + 1) * cap + slot[u]],
+                                        a.ps[(size_t)(CX + 2) * cap + slot[u]]};
+                    stencil(x, r, fx);
 #pragma unroll
                     for (int k = 0; k < 3; ++k) hit[u] = hit[u] && r[k] >= -3 && r[k] <= 2;
                 }
@@ -1628,19 +1637,24 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
             // sum the list when another round might not fit, and at the end
             const bool last = c0 + GATHER_THREADS * GATHER_PER >= total;
             if (!last && held + GATHER_THREADS * GATHER_PER <= GATHER_LIST) continue;
+            // a batch's loads are issued before the sums of the batch before it
+            float px[3], A[12], mass = 0.f;
+            auto load = [&](uint32_t j) __attribute__((always_inline)) {
+#pragma unroll
+                for (int k = 0; k < 3; ++k) px[k] = a.ps[(size_t)(CX + k) * cap + j];
+#pragma unroll
+                for (int k = 0; k < 12; ++k) A[k] = aff[(size_t)k * cap + j];
+                mass = a.ps[(size_t)CMASS * cap + j];
+            };
+            if (tid < GATHER_RECS && uint32_t(tid) < held) load(slots[tid]);
             for (uint32_t b0 = 0; b0 < held; b0 += GATHER_RECS) {
                 const uint32_t cnt = min(held - b0, uint32_t(GATHER_RECS));
                 if (tid < GATHER_RECS) {
                     uint32_t rm = 0u;
                     if (uint32_t(tid) < cnt) {
-                        const uint32_t j = slots[b0 + uint32_t(tid)];
                         int r[3];
                         float fx[3];
-                        stencil(j, r, fx);
-                        float A[12];
-#pragma unroll
-                        for (int k = 0; k < 12; ++k) A[k] = aff[(size_t)k * cap + j];
-                        const float mass = a.ps[(size_t)CMASS * cap + j];
+                        stencil(px, r, fx);
                         GatherRec& q = rec[tid];
                         float w[3][4], d[3][4];  // weight (-1: none) and node offset of the tile's cells
                         uint32_t in[3] = {0u, 0u, 0u};
@@ -1660,14 +1674,16 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                         for (int z = 0; z < 4; ++z)
                             if (in[2] & (1u << z)) rm |= in[1] << (4 * z);
 #pragma unroll
-                        for (int c2 = 0; c2 < 4; ++c2) {
+                        for (int y = 0; y < 4; ++y) {
+                            float v[4];
 #pragma unroll
-                            for (int y = 0; y < 4; ++y)
-                                q.wxy[c2 + 4 * y] = w[0][c2] < 0.f || w[1][y] < 0.f ? -1.0f : w[0][c2] * w[1][y];
-                            q.dx[c2] = d[0][c2];
-                            q.dy[c2] = d[1][c2];
-                            q.z[c2] = make_float2(w[2][c2], d[2][c2]);
+                            for (int c2 = 0; c2 < 4; ++c2)
+                                v[c2] = w[0][c2] < 0.f || w[1][y] < 0.f ? -1.0f : w[0][c2] * w[1][y];
+                            q.wxy[y] = make_float4(v[0], v[1], v[2], v[3]);
+                            q.z[y] = make_float2(w[2][y], d[2][y]);
                         }
+                        q.dy = make_float4(d[1][0], d[1][1], d[1][2], d[1][3]);
+                        q.x = make_float2(float(r[0]), fx[0]);
                         q.row[0] = make_float4(mass, 0.f, 0.f, 0.f);
 #pragma unroll
                         for (int k = 0; k < 3; ++k)
@@ -1676,6 +1692,8 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                     rows[tid] = uint16_t(rm);
                 }
                 __syncthreads();
+                if (tid < GATHER_RECS && b0 + GATHER_RECS + uint32_t(tid) < held)
+                    load(slots[b0 + GATHER_RECS + uint32_t(tid)]);
                 // the wave's own list: records reaching its row, in order,
                 // filled up to a whole step with the record that adds nothing
                 uint32_t len = 0u;
@@ -1688,31 +1706,34 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                 if (lane < GATHER_STEP) wlist[wave][len + uint32_t(lane)] = uint16_t(GATHER_RECS);
                 __builtin_amdgcn_wave_barrier();
                 for (uint32_t g = 0; g < len; g += GATHER_STEP) {
-                    float v[GATHER_FLY];
 #pragma unroll
                     for (int f = 0; f < GATHER_FLY; ++f) {
-                        const GatherRec& q = rec[wlist[wave][g + uint32_t(4 * f + grp)]];
-                        const float w = q.wxy[cx + 4 * cy];
-                        const float2 z = q.z[cz];
-                        const float4 r = q.row[ch];
-                        const float p = w * z.x * (r.x + r.y * q.dx[cx] + r.z * q.dy[cy] + r.w * z.y);
-                        v[f] = w < 0.f ? 0.f : p;
+                        const GatherRec& q = rec[wlist[wave][g + uint32_t(16 * f + grp)]];
+                        const float4 r = q.row[ch], wv = q.wxy[cy];
+                        const float2 z = q.z[cz], qx = q.x;
+                        const float base = r.x + r.z * reinterpret_cast<const float*>(&q.dy)[cy] + r.w * z.y;
+                        const float w[4] = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+                        for (int c2 = 0; c2 < 4; ++c2) {
+                            const float t = w[c2] * z.x * (base + r.y * ((qx.x + float(c2) - qx.y) * sc.dx));
+                            acc[c2] += w[c2] < 0.f ? 0.f : t;
+                        }
                     }
-                    // the four groups' terms, in list order, to the first group
-#pragma unroll
-                    for (int f = 0; f < GATHER_FLY; ++f)
-#pragma unroll
-                        for (int h = 0; h < 4; ++h) acc += h == 0 ? v[f] : __shfl_down(v[f], 16 * h, 64);
                 }
                 __syncthreads();
             }
             held = 0u;
         }
-        if (grp == 0) {
+#pragma unroll
+        for (int c2 = 0; c2 < 4; ++c2)
+#pragma unroll
+            for (int o = 4; o < 64; o *= 2) acc[c2] += __shfl_xor(acc[c2], o, 64);
+        if (grp < 4) {  // lane's cell of the row
             const int G = int(sc.G);
-            const bool valid = 4 * tc[0] + cx < G && 4 * tc[1] + cy < G && 4 * tc[2] + cz < G;
-            const uint32_t c = (t << 6) | uint32_t(cx | (cy << 2) | (cz << 4));
-            reinterpret_cast<float*>(a.gmp)[4 * (size_t)c + ch] = valid ? acc : 0.f;
+            const bool valid = 4 * tc[0] + grp < G && 4 * tc[1] + cy < G && 4 * tc[2] + cz < G;
+            const uint32_t c = (t << 6) | uint32_t(grp | (cy << 2) | (cz << 4));
+            const float v = grp == 0 ? acc[0] : (grp == 1 ? acc[1] : (grp == 2 ? acc[2] : acc[3]));
+            reinterpret_cast<float*>(a.gmp)[4 * (size_t)c + ch] = valid ? v : 0.f;
         }
         if (tid == 0) a.tile_flag[t] |= FLAG_GMP;
         __syncthreads();  // rbeg, roff and the records are reused by the next tile
