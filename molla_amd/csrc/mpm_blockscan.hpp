@@ -45,4 +45,21 @@ __device__ __forceinline__ T block_excl_scan(T v, T* s_wave, T* total) {
     return r;
 }
 
+// Counter `i` of a table of u16 counters goes up by the lanes of `same` (the
+// wave's lanes with this counter) and every one of them gets the word that
+// holds it after that; counter_half takes it out.  The wave's LDS accesses
+// stay in program order, so rounds can be issued one after the other without
+// waiting for the words.
+__device__ __forceinline__ uint32_t counter_add(uint16_t* table, uint32_t i, uint64_t same, uint64_t lt) {
+    uint32_t* w = reinterpret_cast<uint32_t*>(table) + i / 2u;
+    if ((same & lt) == 0ull)
+        __hip_atomic_fetch_add(w, (uint32_t)__popcll(same) << (16u * (i & 1u)), __ATOMIC_RELAXED,
+                               __HIP_MEMORY_SCOPE_WORKGROUP);
+    __builtin_amdgcn_wave_barrier();
+    return __hip_atomic_load(w, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+}
+__device__ __forceinline__ uint32_t counter_half(uint32_t word, uint32_t i) {
+    return (word >> (16u * (i & 1u))) & 0xffffu;
+}
+
 }  // namespace mpm

@@ -553,7 +553,8 @@ int sort_particles(mpm_sim* s, bool reorder) {
     q.max_W = s->max_W;
     if (mpm::layout_fits_one(s->n, s->total_tiles)) {
         HIP_TRY(s, mpm::launch_layout_one(a, s->n_scenes, q, chunk_cap, s->seg_tiles, bits,
-                                          by_slot ? nullptr : s->slot_of_id, s->stream));
+                                          by_slot ? nullptr : reinterpret_cast<const uint32_t*>(id_plane(s)),
+                                          s->stream));
     } else {
         bool lb_done = false;
         HIP_TRY(s, mpm::launch_tile_keys(a, mpm::radix_input(s->keys, s->n, bits, s->sort_scratch), by_slot ? 1 : 0,

@@ -330,10 +330,10 @@ struct LayoutArgs {
 };
 size_t layout_scratch_words(uint32_t total_tiles);  // u64 words
 bool layout_fits_one(uint32_t n, uint32_t total_tiles);
-// Keys, sort, table and lists of a small layout in one launch.  slot_of_id
-// null: ties by current slot; else by original id.
+// Keys, sort, table and lists of a small layout in one launch.  ids null: ties
+// by current slot; else by original id (ids: the slots' ids).
 hipError_t launch_layout_one(const StepArgs& a, uint32_t n_scenes, const LayoutArgs& q, uint32_t chunk_cap,
-                             uint32_t seg_tiles, int bits, const uint32_t* slot_of_id, hipStream_t s);
+                             uint32_t seg_tiles, int bits, const uint32_t* ids, hipStream_t s);
 // Table and lists of sorted keys (lb_done: the table is there already).
 hipError_t launch_layout(const LayoutArgs& q, bool lb_done, uint32_t chunk_cap, uint32_t seg_tiles, uint64_t* scratch,
                          hipStream_t s);

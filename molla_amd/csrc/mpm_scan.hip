@@ -27,10 +27,10 @@
 //   k_layout_block  up to LAYOUT_TILES tiles: table and lists in one block;
 //   the rest        one launch per step, the prefix sum in three.
 // With the chunk spread and the reorder, a sort of 8,192 particles in a 32^3
-// grid is 3 launches (37 us of kernels in a trace), of 200,003 in 61^3 7 (73
+// grid is 3 launches (36 us of kernels in a trace), of 200,003 in 61^3 7 (73
 // us), of 2 M in 256^3 15 (290 us); lists built from per-particle flags took
 // 27 to 32 launches and about 130, 190 and 480 us.  The lines: k_layout_one
-// still beats the separate launches at its 16,384 particles (49 us against
+// still beats the separate launches at its 16,384 particles (36 us against
 // ~60), where its LDS ends; one block walks 8,192 tiles in 15 us, as long as
 // the four launches it saves.
 #include <algorithm>
@@ -182,49 +182,49 @@ __global__ __launch_bounds__(LAYOUT_THREADS) void k_layout_block(LayoutArgs q, C
     layout_lists([&](uint32_t t) { return s_lb[t]; }, q, rule, s_wave);
 }
 
-// Keys, sort and lists of a small layout.  A key (13 bits) and its index (14
+// Keys, sort and lists of a small layout.  A key (13 bits) and its slot (14
 // bits) share a word, so a pass of the sort moves one word per particle; the
 // passes rank as k_radix_scatter does, 16 waves of up to 1024 keys.
 constexpr uint32_t ONE_WAVES = LAYOUT_THREADS / 64;
 constexpr uint32_t ONE_ITEMS = LAYOUT_ONE / LAYOUT_THREADS;
+constexpr uint32_t ONE_FLY = 8;    // rounds of counters in flight
 constexpr uint32_t ONE_DIGIT = 9;  // 512 tiles (a 32^3 grid) in one pass
 
 __global__ __launch_bounds__(LAYOUT_THREADS) void k_layout_one(StepArgs a, uint32_t n_scenes, LayoutArgs q,
                                                                ChunkRule rule, int bits,
-                                                               const uint32_t* __restrict__ slot_of_id) {
+                                                               const uint32_t* __restrict__ ids) {
     __shared__ uint32_t s_key[LAYOUT_ONE];
-    __shared__ uint16_t s_cnt[ONE_WAVES << ONE_DIGIT];
+    __shared__ alignas(4) uint16_t s_cnt[ONE_WAVES << ONE_DIGIT];
     __shared__ uint32_t s_base[1 << ONE_DIGIT];
     __shared__ uint16_t s_lb[LAYOUT_TILES + 1];
     __shared__ uint64_t s_wave[64];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6, n = q.n;
     // four particles' loads in flight per thread: their latency, not their
-    // number, is what counts in one block
+    // number, is what counts in one block.  Slots are read in order, also where
+    // the keys go in the order of the ids: a gather through the ids' slots
+    // took 22 instead of 13 us for 16,384 particles
     for (uint32_t i0 = tid; i0 < n; i0 += 4u * LAYOUT_THREADS) {
-        uint32_t slot[4], key[4];
+        uint32_t at[4], key[4];
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) {
             const uint32_t i = min(i0 + u * LAYOUT_THREADS, n - 1u);
-            slot[u] = slot_of_id ? slot_of_id[i] : i;
-        }
-#pragma unroll
-        for (uint32_t u = 0; u < 4u; ++u) {
+            at[u] = ids ? min(ids[i], n - 1u) : i;
             if (n_scenes == 1u) {  // the scene in scalar registers
-                key[u] = tile_key(a.scenes[0], a.ps, a.cap, slot[u]);
+                key[u] = tile_key(a.scenes[0], a.ps, a.cap, i);
                 continue;
             }
             uint32_t lo = 0u, hi = n_scenes;  // the last scene starting at or before the slot
             while (hi - lo > 1u) {
                 const uint32_t mid = (lo + hi) / 2u;
-                if (a.scenes[mid].pbase <= slot[u]) lo = mid;
+                if (a.scenes[mid].pbase <= i) lo = mid;
                 else hi = mid;
             }
-            key[u] = tile_key(a.scenes[lo], a.ps, a.cap, slot[u]);
+            key[u] = tile_key(a.scenes[lo], a.ps, a.cap, i);
         }
 #pragma unroll
         for (uint32_t u = 0; u < 4u; ++u) {
             const uint32_t i = i0 + u * LAYOUT_THREADS;
-            if (i < n) s_key[i] = key[u] << 14 | i;
+            if (i < n) s_key[at[u]] = key[u] << 14 | i;
         }
     }
     // rounds of 64 keys per wave: a wave's keys are consecutive
@@ -255,16 +255,18 @@ __global__ __launch_bounds__(LAYOUT_THREADS) void k_layout_one(StepArgs a, uint3
                 const uint64_t m = __ballot(on);
                 same[r] &= on ? m : ~m;
             }
+        auto counter = [&](uint32_t r) { return (wave << width) + ((key[r] >> shift) & (R - 1u)); };
 #pragma unroll
-        for (uint32_t r = 0; r < ONE_ITEMS; ++r) {
-            pos[r] = 0u;
-            if (r < rounds && first + r * 64u < n) {
-                // in program order: a round reads the counts of those before it
-                volatile uint16_t* c = &s_cnt[(wave << width) + ((key[r] >> shift) & (R - 1u))];
-                const uint32_t before = *c;
-                pos[r] = before + (uint32_t)__popcll(same[r] & lt);
-                if ((same[r] & lt) == 0ull) *c = uint16_t(before + (uint32_t)__popcll(same[r]));
+        for (uint32_t h = 0; h < ONE_ITEMS; h += ONE_FLY) {
+#pragma unroll
+            for (uint32_t r = h; r < h + ONE_FLY; ++r) {
+                pos[r] = 0u;
+                if (r < rounds && first + r * 64u < n) pos[r] = counter_add(s_cnt, counter(r), same[r], lt);
             }
+#pragma unroll
+            for (uint32_t r = h; r < h + ONE_FLY; ++r)
+                pos[r] = counter_half(pos[r], counter(r)) - (uint32_t)__popcll(same[r] & ~lt);
+            __builtin_amdgcn_sched_barrier(0);  // more in flight does not fit the registers
         }
         __syncthreads();
         uint32_t mine = 0u;  // keys of digit tid (R <= 512 <= threads)
@@ -294,9 +296,8 @@ __global__ __launch_bounds__(LAYOUT_THREADS) void k_layout_one(StepArgs a, uint3
     }
 #pragma unroll 4
     for (uint32_t j = tid; j < n; j += LAYOUT_THREADS) {
-        const uint32_t i = s_key[j] & (LAYOUT_ONE - 1u);
         q.keys[j] = s_key[j] >> 14;
-        q.src[j] = slot_of_id ? slot_of_id[i] : i;
+        q.src[j] = s_key[j] & (LAYOUT_ONE - 1u);
     }
     for (uint32_t t = tid; t <= q.total_tiles; t += LAYOUT_THREADS) {
         uint32_t lo = 0u, hi = n;
@@ -434,11 +435,11 @@ static bool chunk_rule(uint32_t cap, uint32_t seg_tiles, ChunkRule& rule) {
 }
 
 hipError_t launch_layout_one(const StepArgs& a, uint32_t n_scenes, const LayoutArgs& q, uint32_t chunk_cap,
-                             uint32_t seg_tiles, int bits, const uint32_t* slot_of_id, hipStream_t s) {
+                             uint32_t seg_tiles, int bits, const uint32_t* ids, hipStream_t s) {
     ChunkRule rule;
     if (!chunk_rule(chunk_cap, seg_tiles, rule) || !layout_fits_one(q.n, q.total_tiles)) return hipErrorInvalidValue;
     hipLaunchKernelGGL(k_layout_one, dim3(1), dim3(LAYOUT_THREADS), 0, s, a, n_scenes, q, rule, std::max(bits, 1),
-                       slot_of_id);
+                       ids);
     return hipGetLastError();
 }
 

@@ -186,18 +186,15 @@ __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* 
             same[r] &= on ? m : ~m;
         }
     uint32_t rank[SORT_ITEMS];
+    auto counter = [&](int r) { return ((key[r] >> shift) & (R - 1u)) * SORT_WAVES + uint32_t(wave); };
 #pragma unroll
     for (int r = 0; r < SORT_ITEMS; ++r) {
         rank[r] = 0u;
-        if (first + r * 64 + lane < n) {
-            // the wave's LDS accesses stay in program order: a round reads
-            // the counts that the rounds before it wrote
-            volatile uint16_t* c = &cnt[((key[r] >> shift) & (R - 1u)) * SORT_WAVES + uint32_t(wave)];
-            const uint32_t before = *c;
-            rank[r] = before + (uint32_t)__popcll(same[r] & lt);
-            if ((same[r] & lt) == 0ull) *c = uint16_t(before + (uint32_t)__popcll(same[r]));
-        }
+        if (first + r * 64 + lane < n) rank[r] = counter_add(cnt, counter(r), same[r], lt);
     }
+#pragma unroll
+    for (int r = 0; r < SORT_ITEMS; ++r)
+        rank[r] = counter_half(rank[r], counter(r)) - (uint32_t)__popcll(same[r] & ~lt);
     __syncthreads();
     // places in the stage: digits ascending, the waves' keys of a digit in order
     static_assert(SORT_WAVES == 4, "four counters of a digit are one word");
