@@ -474,7 +474,7 @@ int clear_grid(mpm_sim* s) {
         return MPM_OK;
     }
     HIP_TRY(s, mpm::launch_clear_tiles(griddev(s), s->list[s->list_cur], s->status + mpm::ST_COUNT0 + s->list_cur,
-                                       grid_blocks(s), s->stream));
+                                       s->status + mpm::ST_TICKET, grid_blocks(s), s->stream));
     s->grid_dirty = false;
     return MPM_OK;
 }
@@ -1199,7 +1199,7 @@ int diff_backward_pass(mpm_sim* s, bool has_gv, bool checked, Stage& span) {
             }
             mpm::GridDev gc = g;
             gc.gmp = s->gadj;
-            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), gb, s->stream));
+            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), s->status + mpm::ST_TICKET, gb, s->stream));
             L = R;
             continue;
         }
@@ -1218,7 +1218,7 @@ int diff_backward_pass(mpm_sim* s, bool has_gv, bool checked, Stage& span) {
             HIP_TRY(s, mpm::launch_adj_p2g(q, blocks, s->stream));
             mpm::GridDev gc = g;
             gc.gmp = s->gadj;
-            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), gb, s->stream));
+            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), s->status + mpm::ST_TICKET, gb, s->stream));
         }
         L = R;
     }

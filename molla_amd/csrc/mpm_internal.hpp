@@ -42,8 +42,8 @@ constexpr uint32_t FAULT_NUMERICAL = 2u;
 // ST_COUNT0/1: the two dynamic active-tile lists; ST_SCOUNT: the static list.
 // Sparse tile pool: ST_POOL the tiles marked by the last substep (slots in
 // use, or the demand that overflowed the pool), ST_DEFER the particles whose
-// global-atomic scatter waits for the slots.  ST_TICKET: blocks of the last
-// sweep launch that are done (zero between launches).
+// global-atomic scatter waits for the slots.  ST_TICKET: blocks of a clear or
+// of the last sweep launch that are done (zero between launches).
 enum StatusWord : int {
     ST_FAULT = 0, ST_GATHERS = 1, ST_COUNT0 = 2, ST_COUNT1 = 3, ST_SCOUNT = 4, ST_ESCAPES = 5, ST_NCHUNKS = 6,
     ST_FALLBACK = 7, ST_POOL = 8, ST_DEFER = 9, ST_TICKET = 10, ST_WORDS = 11
@@ -212,7 +212,7 @@ hipError_t launch_grid_update(const SceneDev* scenes, const GridDev& g, const ui
 hipError_t launch_rigid_shell(const SceneDev* scenes, const GridDev& g, const uint32_t* dlist,
                               const uint32_t* dcount, float dt, const RigidDev& rg, int blocks, hipStream_t s);
 hipError_t launch_zero_f64(double* p, uint32_t n, hipStream_t s);
-hipError_t launch_clear_tiles(const GridDev& g, const uint32_t* dlist, uint32_t* dcount, int blocks,
+hipError_t launch_clear_tiles(const GridDev& g, const uint32_t* dlist, uint32_t* dcount, uint32_t* ticket, int blocks,
                               hipStream_t s, float4* also = nullptr);
 // `iters` > 0 semi-implicit Jacobi sweeps over the active tiles: they start
 // from the buffer implicit_first() names (g.gv or the second cell buffer
