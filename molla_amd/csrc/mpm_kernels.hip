@@ -100,8 +100,8 @@ __global__ __launch_bounds__(BLOCK) __attribute__((amdgpu_waves_per_eu(3, 3))) v
     const uint32_t nch = a.n_chunks_dev ? *a.n_chunks_dev : a.n_chunks;
     for (ChunkWalk w = chunk_walk(nch); w.ci < w.end; w.ci += w.step) {
         const uint32_t ci = w.ci;
-        const Chunk ch = a.chunks[ci];
-        const SceneDev sc = a.scenes[ch.scene];
+        const Chunk ch = const_load(a.chunks + ci);
+        const SceneDev sc = const_load(a.scenes + ch.scene);
         // Gather staging: the chunk's P2G box of the previous pass holds every
         // stencil this gather reads (same particles, same positions), so the
         // block loads that box of grid velocities into LDS once and the 27
@@ -591,7 +591,7 @@ __global__ __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(RIGID ? 4 :
             walk.at(g, dlist, i, t, st);
             scene = g.tile_scene[t];
         }
-        const SceneDev sc = scenes[scene];
+        const SceneDev sc = const_load(scenes + scene);
         int tx, ty, tz, ix, iy, iz;
         tile_cell(sc, t, lane, tx, ty, tz, ix, iy, iz);
         const uint32_t c = (st << 6) | uint32_t(lane);
@@ -1468,9 +1468,9 @@ __global__ __launch_bounds__(256) void k_gather_prepare(StepArgs a, float* __res
     const uint32_t cap = a.cap;
     const float* ps = a.ps;
     for (uint32_t ci = blockIdx.x; ci < a.n_chunks; ci += gridDim.x) {
-        const Chunk ch = a.chunks[ci];
+        const Chunk ch = const_load(a.chunks + ci);
         if (threadIdx.x >= ch.count) continue;
-        const SceneDev sc = a.scenes[ch.scene];
+        const SceneDev sc = const_load(a.scenes + ch.scene);
         const uint32_t slot = ch.start + threadIdx.x;
         float F[9], C[9];
         for (int k = 0; k < 9; ++k) {
@@ -1572,7 +1572,7 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
         reinterpret_cast<float*>(&rec[GATHER_RECS])[tid] = tid >= 16 && tid < 32 ? -1.f : 0.f;
     for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
         const uint32_t t = list[i];
-        const SceneDev sc = a.scenes[tile_scene[t]];
+        const SceneDev sc = const_load(a.scenes + tile_scene[t]);
         const uint32_t tl = t - sc.tile_base;
         const int W = int(sc.W);
         const int tc[3] = {int(tl % sc.W), int((tl / sc.W) % sc.W), int(tl / (sc.W * sc.W))};
@@ -1845,7 +1845,7 @@ __global__ __launch_bounds__(256) void k_deferred_p2g(StepArgs a) {
     if (a.status[ST_FAULT] != 0u) return;
     const uint32_t n = a.status[ST_DEFER], cap = a.cap;
     const float* ps = a.ps;
-    const SceneDev sc = a.scenes[0];
+    const SceneDev sc = const_load(a.scenes);
     for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < n; i += gridDim.x * blockDim.x) {
         const uint32_t slot = a.defer_list[i], boff = 4u * slot;
         float x[3], v[3], C[9], F[9];
