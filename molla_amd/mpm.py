@@ -349,7 +349,7 @@ class MpmSimulation:
     def read_field(self, name: str) -> np.ndarray:
         fid, nc = FIELDS[name]
         dt = np.uint32 if name == "material" else np.float32
-        out = np.zeros((self.n, nc) if nc > 1 else (self.n,), dt)
+        out = np.empty((self.n, nc) if nc > 1 else (self.n,), dt)
         self._check(lib().mpm_read_field(self._h, fid, _ptr(out), self.n))
         if nc == 9:
             return out.reshape(self.n, 3, 3)
