@@ -8,15 +8,15 @@
 //   k_radix_hist     per-block digit histogram (blocks of 4096 keys, LDS atomics)
 //   k_radix_rows     per digit: exclusive scan of the blocks' counts, total
 //   k_radix_scatter  the digits' bases from the totals, then a stable scatter:
-//                    each wave ranks its 1024 consecutive keys in 16 rounds of
-//                    64 with ballots (the lanes that share a digit) and digit
+//                    each wave ranks its 512 (wide digits: 1024) consecutive
+//                    keys in rounds of 64 with ballots (the lanes that share a digit) and digit
 //                    counters of its own, with no barrier between the rounds,
 //                    and the block's keys leave through LDS in digit order.
 // What bounds a pass at 2 M keys is the scatter: a block's latency (its loads,
 // the ballots, whose rounds overlap bit by bit, the stage) with two blocks per
 // CU.  Wide digits trade passes for counters: 18 key bits (a 256^3 grid) are
-// two passes of 9 bits.  A key query of 2 M random particles takes 73 us
-// (scatter 18, histogram 5, rows 5 us per pass); three passes of 8 bits with
+// two passes of 9 bits.  A key query of 2 M random particles takes 67 us
+// (scatter 15, histogram 5, rows 4 us per pass); three passes of 8 bits with
 // barriers in every round, unstaged stores and a three-launch scan took 154.
 #include <algorithm>
 
@@ -25,11 +25,20 @@
 
 namespace mpm {
 
-constexpr int SORT_THREADS = 256;
-constexpr int SORT_WAVES = SORT_THREADS / 64;
-constexpr int SORT_ITEMS = 16;
-constexpr int SORT_TILE = SORT_THREADS * SORT_ITEMS;  // 4096
+constexpr int SORT_TILE = 4096;  // keys per block
 constexpr int MAX_DIGIT = 12;
+// Threads of a block, by its digits: eight waves rank 512 keys each in half
+// the rounds of four, but hold twice the counters, whose clear and sums come
+// to outweigh the rounds at 4096 digits.  A key query, four waves / eight: of
+// 20,000 keys in one pass of 12 bits 41.8 / 46.2 us, of 60,000 in two of 7
+// 49.8 / 43.3, of 400,000 in two of 8 54.8 / 48.2, of 2 M in two of 9 71.6 /
+// 66.8 us.  Sixteen waves gain another 1 us at 60,000 and nothing at 2 M.
+constexpr int MANY_DIGIT = 10;  // eight waves up to this width
+template <int THREADS>
+struct SortShape {
+    static constexpr int WAVES = THREADS / 64, ITEMS = SORT_TILE / THREADS;
+    static constexpr int PER = (1 << (THREADS == 512 ? MANY_DIGIT : MAX_DIGIT)) / THREADS;  // digits per thread
+};
 
 static inline uint32_t sort_blocks(uint32_t n) { return (n + SORT_TILE - 1) / SORT_TILE; }
 
@@ -59,8 +68,10 @@ uint32_t* radix_input(uint32_t* keys, uint32_t n, int bits, uint32_t* scratch) {
     return radix_plan(n, bits).passes % 2 ? scratch : keys;
 }
 
+template <int SORT_THREADS>
 __global__ __launch_bounds__(SORT_THREADS) void k_radix_hist(const uint32_t* __restrict__ keys, uint32_t n, int shift,
                                                              int width, uint32_t* __restrict__ hist) {
+    constexpr int SORT_ITEMS = SortShape<SORT_THREADS>::ITEMS;
     extern __shared__ uint32_t lds[];
     const uint32_t R = 1u << width;
     for (uint32_t d = threadIdx.x; d < R; d += SORT_THREADS) lds[d] = 0u;
@@ -128,6 +139,7 @@ static_assert(ROW_SEGS == 64, "one lane per segment");
 
 // vin null: the values are the indices.  lb (may be null; single-pass sorts
 // only): receives the first position of every key in [0, n_lb].
+template <int SORT_THREADS>
 __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* __restrict__ kin,
                                                                 const uint32_t* __restrict__ vin,
                                                                 uint32_t* __restrict__ kout,
@@ -135,6 +147,8 @@ __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* 
                                                                 int width, const uint32_t* __restrict__ hist,
                                                                 const uint32_t* __restrict__ total,
                                                                 uint32_t* __restrict__ lb, uint32_t n_lb) {
+    constexpr int SORT_WAVES = SortShape<SORT_THREADS>::WAVES, SORT_ITEMS = SortShape<SORT_THREADS>::ITEMS;
+    constexpr uint32_t PER = SortShape<SORT_THREADS>::PER;
     extern __shared__ uint32_t lds[];
     __shared__ uint32_t s_wave[64];
     const uint32_t R = 1u << width;
@@ -151,8 +165,7 @@ __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* 
         val[r] = vin && i < n ? vin[i] : i;
     }
     for (uint32_t i = tid; i < R * SORT_WAVES / 2; i += SORT_THREADS) lds[R + i] = 0u;
-    // thread t holds the R / 256 digits from t R / 256 on
-    constexpr uint32_t PER = (1u << MAX_DIGIT) / SORT_THREADS;
+    // a thread holds R / threads digits in a row (one where R is less)
     const uint32_t per = R > uint32_t(SORT_THREADS) ? R / SORT_THREADS : 1u, d0 = uint32_t(tid) * per;
     uint32_t tot[PER], at[PER];
     uint32_t sum = 0u;
@@ -197,28 +210,35 @@ __global__ __launch_bounds__(SORT_THREADS) void k_radix_scatter(const uint32_t* 
         rank[r] = counter_half(rank[r], counter(r)) - (uint32_t)__popcll(same[r] & ~lt);
     __syncthreads();
     // places in the stage: digits ascending, the waves' keys of a digit in order
-    static_assert(SORT_WAVES == 4, "four counters of a digit are one word");
+    static_assert(SORT_WAVES % 4 == 0, "four counters of a digit are one word");
+    constexpr int CW = SORT_WAVES / 4;
     uint64_t* cnt4 = reinterpret_cast<uint64_t*>(cnt);
-    uint64_t c4[PER];
+    uint64_t c4[PER][CW];
     uint32_t mine = 0u;
 #pragma unroll
-    for (uint32_t q = 0; q < PER; ++q) {
-        c4[q] = q < per && d0 + q < R ? cnt4[d0 + q] : 0ull;
-        mine += uint32_t(c4[q] & 0xffffu) + uint32_t((c4[q] >> 16) & 0xffffu) + uint32_t((c4[q] >> 32) & 0xffffu) +
-                uint32_t(c4[q] >> 48);
-    }
+    for (uint32_t q = 0; q < PER; ++q)
+#pragma unroll
+        for (int w = 0; w < CW; ++w) {
+            const uint64_t c = q < per && d0 + q < R ? cnt4[(d0 + q) * CW + w] : 0ull;
+            mine += uint32_t(c & 0xffffu) + uint32_t((c >> 16) & 0xffffu) + uint32_t((c >> 32) & 0xffffu) +
+                    uint32_t(c >> 48);
+            c4[q][w] = c;
+        }
     uint32_t place = block_excl_scan(mine, s_wave, (uint32_t*)nullptr);
 #pragma unroll
     for (uint32_t q = 0; q < PER; ++q) {
         if (q >= per || d0 + q >= R) continue;
         base[d0 + q] = at[q] - place;
-        uint64_t out = 0ull;
 #pragma unroll
-        for (int w = 0; w < SORT_WAVES; ++w) {
-            out |= uint64_t(place) << (16 * w);
-            place += uint32_t(c4[q] >> (16 * w)) & 0xffffu;
+        for (int w = 0; w < CW; ++w) {
+            uint64_t out = 0ull;
+#pragma unroll
+            for (int k = 0; k < 4; ++k) {
+                out |= uint64_t(place) << (16 * k);
+                place += uint32_t(c4[q][w] >> (16 * k)) & 0xffffu;
+            }
+            cnt4[(d0 + q) * CW + w] = out;
         }
-        cnt4[d0 + q] = out;
     }
     __syncthreads();
 #pragma unroll
@@ -261,11 +281,15 @@ hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, int bits
     for (int p = 0; p < plan.passes; ++p) {
         const int shift = plan.width * p;
         uint32_t *kout = kin == keys ? k2 : keys, *vout = kin == keys ? v2 : vals;
-        hipLaunchKernelGGL(k_radix_hist, dim3(nb), dim3(SORT_THREADS), R * 4, s, kin, n, shift, plan.width, hist);
+        const bool many = plan.width <= MANY_DIGIT;
+        const dim3 threads(many ? 512 : 256);
+        auto* khist = many ? k_radix_hist<512> : k_radix_hist<256>;
+        auto* kscatter = many ? k_radix_scatter<512> : k_radix_scatter<256>;
+        hipLaunchKernelGGL(khist, dim3(nb), threads, R * 4, s, kin, n, shift, plan.width, hist);
         hipLaunchKernelGGL(k_radix_rows, dim3((R + ROW_DIGITS - 1) / ROW_DIGITS), dim3(ROW_DIGITS * ROW_SEGS), 0, s, hist,
                            nb, R, total);
-        hipLaunchKernelGGL(k_radix_scatter, dim3(nb), dim3(SORT_THREADS),
-                           R * 4 + std::max<uint32_t>(R * SORT_WAVES * 2, 2 * SORT_TILE * 4), s, kin, vin, kout,
+        hipLaunchKernelGGL(kscatter, dim3(nb), threads,
+                           R * 4 + std::max<uint32_t>(R * (threads.x / 64) * 2, 2 * SORT_TILE * 4), s, kin, vin, kout,
                            vout, n, shift, plan.width, hist, total, with_lb ? lb : nullptr, n_lb);
         kin = kout;
         vin = vout;
