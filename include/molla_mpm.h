@@ -247,6 +247,8 @@ int mpm_autotune(mpm_sim* sim, float dt, uint32_t trial_substeps, uint32_t* part
 int mpm_autotune_config(mpm_sim* sim, float dt, uint32_t trial_substeps, mpm_launch_config* out);
 
 /* ---- stepping (step / step_n, mpm.rs:2232-2272) ---- */
+/* Small scenes' repeated calls replay a captured graph, with the same bits
+ * (the fused mode, 8 substeps or more, up to 131,072 particles). */
 int mpm_step_n(mpm_sim* sim, float dt, uint32_t substeps);
 /* Capture step_n(dt, substeps) into a hipGraph once and replay it
  * (PreparedMpmStep / MpmCommandBatch, mpm_command_batch.rs:10-235). */
