@@ -19,6 +19,7 @@
 
 #include "../../include/molla_mpm.h"
 #include "mpm_internal.hpp"
+#include "mpm_radix_plan.hpp"
 #include "mpm_rigid.hpp"
 
 using mpm::Chunk;
@@ -1576,7 +1577,7 @@ int autotune(mpm_sim* s, float dt, uint32_t trial, uint32_t* out_pb, uint32_t* o
 // names a host-side stand-in; its device address comes from
 // hipGetSymbolAddress, once per device (noalloc_scratch), and only that
 // address is ever handed to a kernel or a copy.
-constexpr size_t NOALLOC_WORDS = 2u * size_t(MPM_NOALLOC_MAX_PARTICLES) + (1u << 18) + (1u << 12) + 64u;
+constexpr size_t NOALLOC_WORDS = mpm::radix_scratch_words(MPM_NOALLOC_MAX_PARTICLES);
 static __device__ __align__(256) uint32_t scratch[NOALLOC_WORDS];
 
 namespace {
@@ -2088,8 +2089,6 @@ int mpm_sort_keys_noalloc(mpm_sim* sim, uint32_t scene, uint32_t capacity, uint3
                         std::to_string(MPM_NOALLOC_MAX_PARTICLES));
     const uint32_t W = sim->sh[scene].W;
     const int bits = int(ceil_log2(std::max(W * W * W, 2u)));
-    if (mpm::radix_scratch_words(cnt) > NOALLOC_WORDS)
-        return fail(sim, MPM_ERR_INVALID, "mpm_sort_keys_noalloc: scratch too small for the sort");
     HIP_TRY(sim, hipSetDevice(sim->device));
     uint32_t* scr = nullptr;
     int rc = noalloc_scratch(sim, &scr);

@@ -339,14 +339,14 @@ hipError_t launch_layout(const LayoutArgs& q, bool lb_done, uint32_t chunk_cap, 
                          hipStream_t s);
 
 // ---- radix sort (mpm_sort.hip) ----
-size_t radix_scratch_words(uint32_t n);
 // Where the keys of a sort of n keys of `bits` bits have to be written:
 // `keys` itself or a part of the scratch.
 uint32_t* radix_input(uint32_t* keys, uint32_t n, int bits, uint32_t* scratch);
 // Stable LSD sort on the low `bits` bits: sorted keys in `keys`, the input
-// index of each in `vals`; scratch holds radix_scratch_words(n) u32.  lb (may
-// be null): where the sort finds the first position of every key in [0, n_lb]
-// by the way, it is written there and *lb_done set.
+// index of each in `vals`; scratch holds radix_scratch_words(m) u32 for an
+// m >= n (mpm_radix_plan.hpp).  lb (may be null): where the sort finds the
+// first position of every key in [0, n_lb] by the way, it is written there and
+// *lb_done set.
 hipError_t radix_sort_pairs(uint32_t* keys, uint32_t* vals, uint32_t n, int bits, uint32_t* scratch, uint32_t* lb,
                             uint32_t n_lb, bool* lb_done, hipStream_t s);
 

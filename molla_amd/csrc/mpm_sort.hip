@@ -22,11 +22,10 @@
 
 #include "mpm_internal.hpp"
 #include "mpm_blockscan.hpp"
+#include "mpm_radix_plan.hpp"
 
 namespace mpm {
 
-constexpr int SORT_TILE = 4096;  // keys per block
-constexpr int MAX_DIGIT = 12;
 // Threads of a block, by its digits: eight waves rank 512 keys each in half
 // the rounds of four, but hold twice the counters, whose clear and sums come
 // to outweigh the rounds at 4096 digits.  A key query, four waves / eight: of
@@ -39,30 +38,6 @@ struct SortShape {
     static constexpr int WAVES = THREADS / 64, ITEMS = SORT_TILE / THREADS;
     static constexpr int PER = (1 << (THREADS == 512 ? MANY_DIGIT : MAX_DIGIT)) / THREADS;  // digits per thread
 };
-
-static inline uint32_t sort_blocks(uint32_t n) { return (n + SORT_TILE - 1) / SORT_TILE; }
-
-// Digit width limit: the histogram table (2^width x blocks words, written and
-// read once per pass) stays within 1 MB up to 512 blocks (2 M keys); beyond,
-// 11 bits, because another pass over the keys costs more than the table.
-static inline int max_digit(uint32_t nb) {
-    return nb <= 64 ? MAX_DIGIT : (nb <= 128 ? 11 : (nb <= 256 ? 10 : (nb <= 512 ? 9 : 11)));
-}
-
-struct RadixPlan {
-    int passes, width;
-};
-static inline RadixPlan radix_plan(uint32_t n, int bits) {
-    const int w = max_digit(sort_blocks(n)), b = std::max(bits, 1);
-    const int passes = (b + w - 1) / w;
-    return {passes, (b + passes - 1) / passes};
-}
-
-size_t radix_scratch_words(uint32_t n) {
-    // ping-pong keys + values, histogram table, digit totals
-    const uint32_t nb = sort_blocks(n);
-    return 2 * (size_t)n + ((size_t)nb << max_digit(nb)) + (1u << MAX_DIGIT) + 64;
-}
 
 uint32_t* radix_input(uint32_t* keys, uint32_t n, int bits, uint32_t* scratch) {
     return radix_plan(n, bits).passes % 2 ? scratch : keys;
