@@ -253,6 +253,10 @@ int mpm_step_n(mpm_sim* sim, float dt, uint32_t substeps);
 /* Capture step_n(dt, substeps) into a hipGraph once and replay it
  * (PreparedMpmStep / MpmCommandBatch, mpm_command_batch.rs:10-235). */
 int mpm_step_n_graph(mpm_sim* sim, float dt, uint32_t substeps);
+/* Graphs captured and replays of them since the handle was created, by either
+ * call above, and graphs held now; a setter that drops the graphs also starts
+ * the count of repeated calls over.  Any of the three may be NULL. */
+int mpm_graph_stats(mpm_sim* sim, uint32_t* captures, uint32_t* replays, uint32_t* kept);
 int mpm_synchronize(mpm_sim* sim);
 
 /* ---- grid / status / ordering ---- */

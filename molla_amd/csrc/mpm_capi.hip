@@ -134,6 +134,7 @@ struct mpm_sim {
     // graphs
     std::map<GraphKey, hipGraphExec_t> graphs;
     std::map<GraphKey, uint32_t> seen;  // calls of mpm_step_n by key (recurring_step)
+    uint32_t captures = 0, replays = 0;  // mpm_graph_stats
     bool capturing = false;
     bool dry = false;  // walk the schedule's host bookkeeping without launching
     // differentiable path
@@ -237,6 +238,9 @@ std::string validate(const mpm_scene_config& c) {
     return "";
 }
 
+// The captured steps go, and the counts of the calls that lead to a capture:
+// a program that changes a setting before each frame would otherwise capture
+// every one of them for a single replay.
 void drop_graphs(mpm_sim* s) {
     for (auto& kv : s->graphs) (void)hipGraphExecDestroy(kv.second);
     s->graphs.clear();
@@ -786,6 +790,7 @@ int capture_steps(mpm_sim* s, float dt, uint32_t substeps, hipGraphExec_t* ex) {
     e = hipGraphInstantiate(ex, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
     if (e != hipSuccess) return hip_fail(s, e, "hipGraphInstantiate");
+    s->captures++;
     return MPM_OK;
 }
 
@@ -796,6 +801,7 @@ int replay_steps(mpm_sim* s, hipGraphExec_t ex, float dt, uint32_t substeps) {
     s->dry = false;
     if (rc != MPM_OK) return rc;
     HIP_TRY(s, hipGraphLaunch(ex, s->stream));
+    s->replays++;
     return MPM_OK;
 }
 
@@ -1738,8 +1744,7 @@ int mpm_set_scene_params(mpm_sim* sim, uint32_t scene, const mpm_scene_config* c
     SceneDev d = make_scene(*cfg, sim->sh[scene].tile_base, sim->sh[scene].mat_base);
     sim->cfg[scene] = *cfg;
     sim->sh[scene] = d;
-    for (auto& kv : sim->graphs) (void)hipGraphExecDestroy(kv.second);
-    sim->graphs.clear();
+    drop_graphs(sim);
     sim->sorted = false;
     return upload_scenes(sim);
 }
@@ -1765,8 +1770,7 @@ int mpm_set_time_step(mpm_sim* sim, uint32_t jacobi_iters) {
     HIP_TRY(sim, hipStreamSynchronize(sim->stream));
     if (jacobi_iters > 0 && sim->gmp && !sim->gv2) HIP_TRY(sim, dalloc(&sim->gv2, grid_cells(sim)));
     sim->jacobi_iters = jacobi_iters;
-    for (auto& kv : sim->graphs) (void)hipGraphExecDestroy(kv.second);
-    sim->graphs.clear();
+    drop_graphs(sim);
     return MPM_OK;
 }
 
@@ -1884,6 +1888,14 @@ int mpm_step_n_graph(mpm_sim* sim, float dt, uint32_t substeps) {
     if (rc != MPM_OK) return rc;
     sim->graphs.emplace(key, ex);
     HIP_TRY(sim, hipGraphLaunch(ex, sim->stream));
+    return MPM_OK;
+}
+
+int mpm_graph_stats(mpm_sim* sim, uint32_t* captures, uint32_t* replays, uint32_t* kept) {
+    if (!sim) return MPM_ERR_INVALID;
+    if (captures) *captures = sim->captures;
+    if (replays) *replays = sim->replays;
+    if (kept) *kept = uint32_t(sim->graphs.size());
     return MPM_OK;
 }
 

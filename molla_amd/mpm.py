@@ -117,6 +117,7 @@ _SIGS = {
     "mpm_autotune_config": (C.c_int, [C.c_void_p, C.c_float, C.c_uint32, C.POINTER(LaunchConfig)]),
     "mpm_step_n": (C.c_int, [C.c_void_p, C.c_float, C.c_uint32]),
     "mpm_step_n_graph": (C.c_int, [C.c_void_p, C.c_float, C.c_uint32]),
+    "mpm_graph_stats": (C.c_int, [C.c_void_p, C.c_void_p, C.c_void_p, C.c_void_p]),
     "mpm_synchronize": (C.c_int, [C.c_void_p]),
     "mpm_read_grid_mass_momentum": (C.c_int, [C.c_void_p, C.c_uint32, C.c_void_p, C.c_void_p]),
     "mpm_read_status": (C.c_int, [C.c_void_p, C.POINTER(StatusInfo)]),
@@ -487,6 +488,12 @@ class MpmSimulation:
 
     def step_n_graph(self, dt: float, substeps: int):
         self._check(lib().mpm_step_n_graph(self._h, float(dt), int(substeps)))
+
+    def graph_stats(self) -> dict:
+        """Graphs captured, replays of them, and graphs held now."""
+        w = [C.c_uint32() for _ in range(3)]
+        self._check(lib().mpm_graph_stats(self._h, *(C.byref(v) for v in w)))
+        return dict(zip(("captures", "replays", "kept"), (v.value for v in w)))
 
     def synchronize(self):
         self._check(lib().mpm_synchronize(self._h))
