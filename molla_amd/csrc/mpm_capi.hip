@@ -13,6 +13,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <new>
 #include <string>
 #include <tuple>
 #include <vector>
@@ -20,6 +21,7 @@
 #include "../../include/molla_mpm.h"
 #include "mpm_internal.hpp"
 #include "mpm_radix_plan.hpp"
+#include "mpm_recurring.hpp"
 #include "mpm_rigid.hpp"
 
 using mpm::Chunk;
@@ -132,8 +134,8 @@ struct mpm_sim {
     double prof_ms[MPM_STAGE_COUNT] = {0};
     uint32_t prof_n[MPM_STAGE_COUNT] = {0};
     // graphs
-    std::map<GraphKey, hipGraphExec_t> graphs;
-    std::map<GraphKey, uint32_t> seen;  // calls of mpm_step_n by key (recurring_step)
+    std::map<GraphKey, hipGraphExec_t> graphs;  // of mpm_step_n_graph
+    mpm::RecurringCalls<GraphKey, hipGraphExec_t> recurring;  // of mpm_step_n
     uint32_t captures = 0, replays = 0;  // mpm_graph_stats
     bool capturing = false;
     bool dry = false;  // walk the schedule's host bookkeeping without launching
@@ -244,7 +246,7 @@ std::string validate(const mpm_scene_config& c) {
 void drop_graphs(mpm_sim* s) {
     for (auto& kv : s->graphs) (void)hipGraphExecDestroy(kv.second);
     s->graphs.clear();
-    s->seen.clear();
+    s->recurring.clear([](hipGraphExec_t g) { (void)hipGraphExecDestroy(g); });
 }
 
 template <typename T>
@@ -277,8 +279,7 @@ void release(mpm_sim* s) {
     if (!s) return;
     (void)hipSetDevice(s->device);
     if (s->stream) (void)hipStreamSynchronize(s->stream);
-    for (auto& kv : s->graphs) (void)hipGraphExecDestroy(kv.second);
-    s->graphs.clear();
+    drop_graphs(s);
     for (auto& r : s->prof_pending) {
         (void)hipEventDestroy(r.a);
         (void)hipEventDestroy(r.b);
@@ -811,14 +812,46 @@ int replay_steps(mpm_sim* s, hipGraphExec_t ex, float dt, uint32_t substeps) {
 // time against 32 us for a graph's replay.  A call that comes back in the same
 // state of the launch sequence is therefore captured and replayed: three such
 // handles in turn 191 -> 150 us a frame, eight implicit substeps of 32,768
-// particles 120 -> 108 us, the same bits.  Scenes above the line and calls of
-// fewer substeps wait for the GPU and gain nothing.  The first calls of a key
-// stay eager: a capture costs 50 to 100 us once.
-constexpr uint32_t RECURRING_CALLS = 4;  // eager calls of a key before its capture
-constexpr size_t RECURRING_KEYS = 64;    // keys counted, and graphs kept, per handle
+// particles 120 -> 108 us, the same bits.  The first calls of a key stay
+// eager (RecurringCalls).
+// The lines, three handles in turn, eager / replayed, us a frame: 8 substeps
+// of 1,000 particles 70 / 53, of 8,192 73 / 61, of 32,768 83 / 84; scenes
+// above 131,072 wait for the GPU.  Calls of fewer substeps gain where the host
+// is what they wait for (8,192 particles, 4 substeps 41 / 32) and lose where a
+// handle runs alone (1 substep of 1,000 particles 34.7 / 37.3, 2 substeps 52.3
+// / 53.6), and they cycle through more keys per replayed launch: one substep a
+// call through 32, of 2 MB of graph each.
 bool recurring_step(const mpm_sim* s, uint32_t substeps) {
     return substeps >= 8u && s->n <= ONE_PER_THREAD && s->p2g_mode == MPM_P2G_FUSED && s->gmp && !s->pool_cap &&
            s->rigid_count == 0u && !s->profiling && !s->hold_order && !s->capturing;
+}
+
+// The call as a replay, captured first where that is due.  False: it has to
+// run eagerly (nothing was launched, the host state is as before).
+bool step_recurring(mpm_sim* s, float dt, uint32_t substeps, int* rc) {
+    const GraphKey key = graph_key(s, dt, substeps);
+    auto& e = s->recurring.call(key);
+    if (e.graph) {
+        *rc = replay_steps(s, e.graph, dt, substeps);
+        return true;
+    }
+    if (!s->recurring.due(e, [s](hipGraphExec_t g) {
+            (void)hipStreamSynchronize(s->stream);  // it may still be running
+            (void)hipGraphExecDestroy(g);
+        }))
+        return false;
+    mpm_sim before = *s;  // a capture changes the host state only
+    hipGraphExec_t ex = nullptr;
+    if (capture_steps(s, dt, substeps, &ex) != MPM_OK) {
+        (void)hipGetLastError();
+        *s = std::move(before);
+        s->recurring.reset(key);
+        return false;
+    }
+    s->recurring.keep(e, ex);
+    const hipError_t err = hipGraphLaunch(ex, s->stream);
+    *rc = err == hipSuccess ? MPM_OK : hip_fail(s, err, "hipGraphLaunch");
+    return true;
 }
 
 int field_layout(int field, int* comp0, int* ncomp) {
@@ -1846,22 +1879,10 @@ int mpm_step_n(mpm_sim* sim, float dt, uint32_t substeps) {
     if (sim->n == 0 || substeps == 0) return MPM_OK;
     sim->diff_steps = 0;
     if (recurring_step(sim, substeps)) {
-        const GraphKey key = graph_key(sim, dt, substeps);
-        auto it = sim->graphs.find(key);
-        if (it != sim->graphs.end()) return replay_steps(sim, it->second, dt, substeps);
-        if (sim->seen.size() >= RECURRING_KEYS) sim->seen.clear();
-        if (++sim->seen[key] > RECURRING_CALLS && sim->graphs.size() < RECURRING_KEYS) {
-            // a capture changes the host state only: without a graph the steps run as ever
-            const mpm_sim before = *sim;
-            hipGraphExec_t ex = nullptr;
-            if (capture_steps(sim, dt, substeps, &ex) == MPM_OK) {
-                sim->graphs.emplace(key, ex);
-                HIP_TRY(sim, hipGraphLaunch(ex, sim->stream));
-                return MPM_OK;
-            }
-            (void)hipGetLastError();
-            *sim = before;
-            sim->seen[key] = 0u;
+        try {
+            int rc = MPM_OK;
+            if (step_recurring(sim, dt, substeps, &rc)) return rc;
+        } catch (const std::bad_alloc&) {  // no room to count the call or to keep the state: it runs eagerly
         }
     }
     return run_step_n(sim, dt, substeps);
@@ -1895,7 +1916,7 @@ int mpm_graph_stats(mpm_sim* sim, uint32_t* captures, uint32_t* replays, uint32_
     if (!sim) return MPM_ERR_INVALID;
     if (captures) *captures = sim->captures;
     if (replays) *replays = sim->replays;
-    if (kept) *kept = uint32_t(sim->graphs.size());
+    if (kept) *kept = uint32_t(sim->graphs.size() + sim->recurring.graphs());
     return MPM_OK;
 }
 
