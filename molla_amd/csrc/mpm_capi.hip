@@ -780,13 +780,16 @@ GraphKey graph_key(const mpm_sim* s, float dt, uint32_t substeps) {
 
 // Captures the step's launches; the host state advances as if they had run.
 int capture_steps(mpm_sim* s, float dt, uint32_t substeps, hipGraphExec_t* ex) {
-    hipGraph_t g;
+    hipGraph_t g = nullptr;
     HIP_TRY(s, hipStreamBeginCapture(s->stream, hipStreamCaptureModeThreadLocal));
     s->capturing = true;
     int rc = run_step_n(s, dt, substeps);
     s->capturing = false;
     hipError_t e = hipStreamEndCapture(s->stream, &g);
-    if (rc != MPM_OK) return rc;
+    if (rc != MPM_OK) {
+        if (e == hipSuccess && g) (void)hipGraphDestroy(g);
+        return rc;
+    }
     if (e != hipSuccess) return hip_fail(s, e, "hipStreamEndCapture");
     e = hipGraphInstantiate(ex, g, nullptr, nullptr, 0);
     (void)hipGraphDestroy(g);
