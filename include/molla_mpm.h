@@ -203,9 +203,12 @@ int mpm_set_launch(mpm_sim* sim, uint32_t particle_blocks, uint32_t grid_blocks)
  *   particles_per_thread          1 or 2: particles each thread of the fused
  *                                 pass takes per chunk of the sorted layout
  *                                 (a chunk holds 256 x this many; shader
- *                                 model only, MPM_MODEL_CPUDIFF handles run 1;
- *                                 until a configuration is set or tuned, a
- *                                 handle of up to 131,072 particles runs 1);
+ *                                 model only, MPM_MODEL_CPUDIFF handles run
+ *                                 1).  Until it is set or tuned the handle
+ *                                 chooses, 1 for up to 131,072 particles and
+ *                                 2 beyond, and reads back its choice (2
+ *                                 before it has particles); writing back the
+ *                                 value that was read leaves it the choice;
  *   segment_tiles                 the chunk rule of the sorted layout; all
  *                                 keep a chunk inside one tile row, which
  *                                 bounds the LDS box of its scatter.  4 or
@@ -229,6 +232,9 @@ typedef struct {
 } mpm_launch_config;
 int mpm_set_launch_config(mpm_sim* sim, const mpm_launch_config* cfg);
 int mpm_get_launch_config(mpm_sim* sim, mpm_launch_config* cfg);
+/* particles_per_thread alone: 1 or 2 whatever the handle would choose, now and
+ * for later particle sets; 0 leaves it the choice again. */
+int mpm_set_particles_per_thread(mpm_sim* sim, uint32_t particles_per_thread);
 
 /* Launch autotuner.  No counterpart in the reference, whose dispatch sizes
  * are fixed; it serves the batched mode, where scene mixes differ widely.

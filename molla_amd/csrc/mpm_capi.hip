@@ -52,6 +52,8 @@ struct ProfRec {
 
 }  // namespace
 
+constexpr uint32_t DEFAULT_PPT = 2;
+
 struct mpm_sim {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -123,8 +125,8 @@ struct mpm_sim {
     int write_vc = 1;
     uint32_t pblocks = 0;
     uint32_t gblocks = 0;
-    uint32_t ppt = 2;         // particles per thread asked for (shader model)
-    bool ppt_set = false;     // ... by the caller or the autotuner; else layout_ppt() may take one
+    uint32_t ppt = DEFAULT_PPT;  // particles per thread asked for (shader model)
+    bool ppt_set = false;        // ... by the caller or the autotuner; else layout_ppt() may take one
     uint32_t seg_tiles = 6;   // chunk rule: 4 or 6 greedy rows of at most that many tiles, 8 aligned segments
     uint32_t chunk_ppt = 1;   // particles per thread of the current sorted chunk list
     // profiling
@@ -519,6 +521,26 @@ constexpr uint32_t ONE_PER_THREAD = 256u * 512u;
 uint32_t layout_ppt(const mpm_sim* s) {
     if (s->sh[0].model != MPM_MODEL_SHADER) return 1u;
     return !s->ppt_set && s->n <= ONE_PER_THREAD ? 1u : s->ppt;
+}
+
+// What mpm_get_launch_config reports: the value in effect where the handle
+// chooses.
+uint32_t reported_ppt(const mpm_sim* s) {
+    return s->ppt_set || s->n == 0 || s->sh[0].model != MPM_MODEL_SHADER ? s->ppt : layout_ppt(s);
+}
+
+// Takes a chunking.  A new one makes a new chunk list at the next step (a
+// taped forward is not reversible after it).
+void set_chunking(mpm_sim* s, uint32_t ppt, bool ppt_set, uint32_t seg_tiles) {
+    const uint32_t layout0 = layout_ppt(s), ppt0 = s->ppt, seg0 = s->seg_tiles;
+    s->ppt = ppt;
+    s->ppt_set = ppt_set;
+    s->seg_tiles = seg_tiles;
+    if ((ppt0 != ppt || layout0 != layout_ppt(s) || seg0 != seg_tiles) && s->sorted) {
+        s->sorted = false;
+        s->boxes_valid = false;
+        s->layout_gen++;
+    }
 }
 
 // slot_of_id of the current slots, where a sort since has left it behind.
@@ -1495,7 +1517,7 @@ int autotune(mpm_sim* s, float dt, uint32_t trial, uint32_t* out_pb, uint32_t* o
     // host flags the trials' steps set that belong to the caller's state: a
     // stepped handle reads position/velocity w as 0, and a reset of a latched
     // fault blocks an archive until the caller steps or restores
-    const bool w_stepped0 = s->w_stepped, fault_reset0 = s->fault_reset;
+    const bool w_stepped0 = s->w_stepped, fault_reset0 = s->fault_reset, ppt_set0 = s->ppt_set;
     const int prof = s->profiling;
     s->profiling = 0;
     hipEvent_t ea = nullptr, eb = nullptr;
@@ -1586,6 +1608,7 @@ int autotune(mpm_sim* s, float dt, uint32_t trial, uint32_t* out_pb, uint32_t* o
     s->sort_every = best_se;
     s->ppt = best_ppt;
     s->seg_tiles = best_seg;
+    if (rc != MPM_OK) s->ppt_set = ppt_set0;  // nothing was tuned
     s->sorts = sorts0;
     s->w_stepped = w_stepped0;
     s->fault_reset = fault_reset0;
@@ -1602,7 +1625,7 @@ int autotune(mpm_sim* s, float dt, uint32_t trial, uint32_t* out_pb, uint32_t* o
     if (out_pb) *out_pb = best_pb;
     if (out_gb) *out_gb = best_gb;
     if (out_se) *out_se = best_se;
-    if (out_ppt) *out_ppt = best_ppt;
+    if (out_ppt) *out_ppt = reported_ppt(s);
     if (out_seg) *out_seg = best_seg;
     return MPM_OK;
 }
@@ -1839,19 +1862,18 @@ int mpm_set_launch_config(mpm_sim* sim, const mpm_launch_config* cfg) {
     sim->pblocks = cfg->particle_blocks;
     sim->gblocks = cfg->grid_blocks;
     sim->sort_every = cfg->sort_every;
-    const uint32_t ppt0 = layout_ppt(sim);
-    const bool asked = cfg->particles_per_thread != sim->ppt;
-    sim->ppt = cfg->particles_per_thread;
-    sim->ppt_set = true;
-    if (asked || ppt0 != layout_ppt(sim) || cfg->segment_tiles != sim->seg_tiles) {
-        // a new chunk list at the next step (a taped forward is not reversible after it)
-        sim->seg_tiles = cfg->segment_tiles;
-        if (sim->sorted) {
-            sim->sorted = false;
-            sim->boxes_valid = false;
-            sim->layout_gen++;
-        }
-    }
+    // a value read back from the handle does not end the handle's own choice
+    const bool own = !sim->ppt_set && cfg->particles_per_thread == reported_ppt(sim);
+    set_chunking(sim, own ? sim->ppt : cfg->particles_per_thread, !own, cfg->segment_tiles);
+    return MPM_OK;
+}
+
+int mpm_set_particles_per_thread(mpm_sim* sim, uint32_t particles_per_thread) {
+    if (!sim) return MPM_ERR_INVALID;
+    if (particles_per_thread > uint32_t(mpm::MAX_PPT))
+        return fail(sim, MPM_ERR_INVALID, "particles_per_thread must be 1 or 2, or 0 for the handle's choice");
+    const bool set = particles_per_thread > 0;
+    set_chunking(sim, set ? particles_per_thread : DEFAULT_PPT, set, sim->seg_tiles);
     return MPM_OK;
 }
 
@@ -1861,7 +1883,7 @@ int mpm_get_launch_config(mpm_sim* sim, mpm_launch_config* cfg) {
     cfg->particle_blocks = sim->pblocks;
     cfg->grid_blocks = sim->gblocks;
     cfg->sort_every = sim->sort_every;
-    cfg->particles_per_thread = sim->ppt;
+    cfg->particles_per_thread = reported_ppt(sim);
     cfg->segment_tiles = sim->seg_tiles;
     return MPM_OK;
 }

@@ -114,6 +114,7 @@ _SIGS = {
     "mpm_set_launch": (C.c_int, [C.c_void_p, C.c_uint32, C.c_uint32]),
     "mpm_set_launch_config": (C.c_int, [C.c_void_p, C.POINTER(LaunchConfig)]),
     "mpm_get_launch_config": (C.c_int, [C.c_void_p, C.POINTER(LaunchConfig)]),
+    "mpm_set_particles_per_thread": (C.c_int, [C.c_void_p, C.c_uint32]),
     "mpm_autotune_config": (C.c_int, [C.c_void_p, C.c_float, C.c_uint32, C.POINTER(LaunchConfig)]),
     "mpm_step_n": (C.c_int, [C.c_void_p, C.c_float, C.c_uint32]),
     "mpm_step_n_graph": (C.c_int, [C.c_void_p, C.c_float, C.c_uint32]),
@@ -424,13 +425,16 @@ class MpmSimulation:
         """Change any of particle_blocks, grid_blocks, sort_every,
         particles_per_thread (1, 2) and segment_tiles (the chunk rule: 4 or 6
         greedy rows of at most that many tiles, 8 aligned eight- or four-tile
-        segments)."""
+        segments).  particles_per_thread stays the handle's choice (and
+        launch_config() says what it chose) until it is given here or tuned."""
         cur = self.launch_config()
         unknown = set(kw) - set(cur)
         if unknown:
             raise TypeError(f"unknown launch settings {sorted(unknown)}")
         cur.update(kw)
         self._check(lib().mpm_set_launch_config(self._h, C.byref(LaunchConfig(**{k: int(v) for k, v in cur.items()}))))
+        if "particles_per_thread" in kw:  # also where it is the value that was read back
+            self._check(lib().mpm_set_particles_per_thread(self._h, int(kw["particles_per_thread"])))
 
     # -- stepping --
     def step(self, dt: float):
