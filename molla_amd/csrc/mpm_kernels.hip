@@ -780,15 +780,17 @@ __global__ __launch_bounds__(256) void k_implicit_sweeps(const SceneDev* __restr
                     on[u] = (g.tile_flag[nc >> 6] & (FLAG_STATIC | FLAG_DYN)) != 0u;
                 }
                 if (!g.tile_slot || on[u]) v[u] = src[nc];
-                // cells stamped by a legacy sphere keep their velocity
-                if (v[u].w > 1.0e-9f && rigid_masked_legacy(rg, sc, ix, iy, iz)) v[u].w = -v[u].w;
+                // empty cells and negative masses are no neighbours; cells
+                // stamped by a legacy sphere keep their velocity
+                if (!(v[u].w > 1.0e-9f)) v[u].w = 0.f;
+                else if (rigid_masked_legacy(rg, sc, ix, iy, iz)) v[u].w = -v[u].w;
             }
         }
 #pragma unroll
         for (int u = 0; u < PER; ++u) {
             const int c = tid + 256 * u;
             if (c >= CELLS) continue;
-            if (!on[u] || !(fabsf(v[u].w) > 1.0e-9f)) v[u].w = 0.f;
+            if (!on[u]) v[u].w = 0.f;
             buf[0][c] = v[u];
         }
         __syncthreads();
