@@ -870,7 +870,7 @@ bool step_recurring(mpm_sim* s, float dt, uint32_t substeps, int* rc) {
     if (capture_steps(s, dt, substeps, &ex) != MPM_OK) {
         (void)hipGetLastError();
         *s = std::move(before);
-        s->recurring.reset(key);
+        s->recurring.failed(key);
         return false;
     }
     s->recurring.keep(e, ex);

@@ -38,3 +38,17 @@ def test_long_cycles_and_implicit_steps_replay_the_same_bits(interval, substeps,
     assert got["replays"] >= least and got["captures"] <= 64
     for p, q in zip(a, b):
         assert np.array_equal(p, q)
+
+
+def test_captures_that_are_not_replayed_end():
+    # particles loaded anew every 24 frames drop the graphs after a replay or none
+    cfg, x, meta = workloads.elastic_cube(1000, seed=3)
+    sim = MpmSimulation(cfg)
+    for _ in range(120):
+        sim.set_particles(x)
+        for _ in range(24):
+            sim.step_n(0.02 * meta["dt"], 8)
+    got = sim.graph_stats()
+    log(f"short episodes: {got}")
+    assert 0 < got["captures"] <= 64 + got["replays"] // 16
+    sim.close()

@@ -1,6 +1,7 @@
 """Which repeated calls get a captured graph (host code only): every key of a
 cycle that fits the table comes back to its count, however long the cycle; a
-failed capture waits; graphs are bounded and give way only to keys that last."""
+failed capture waits; graphs are bounded and give way only to keys that last;
+captures that are not replayed end."""
 import os
 import subprocess
 
@@ -63,12 +64,26 @@ int main() {
         for (int k = 0; k < 30000; ++k) u.step(k % 3000);
         CHECK(u.captures == 0);
     }
+    // everything is dropped every `len` calls of a cycle of 4 keys, as where
+    // particles are loaded anew: captures that do not pay end, others go on
+    for (int len : {24, 30, 60, 100, 400}) {
+        Run u;
+        for (int ep = 0; ep < 2000; ++ep) {
+            for (int k = 0; k < len; ++k) u.step(k % 4);
+            u.r.clear([&](int* g) { CHECK(u.live.erase(g) == 1); });
+        }
+        CHECK(u.captures <= int(R::GRAPHS) + u.replays / int(R::CAPTURE_COST));
+        if (len >= 100) CHECK(u.captures == 4 * 2000 && u.replays == 2000 * (len - 20));
+    }
     {  // a failed capture waits for its calls again
         R r;
         int asked = 0;
         for (int k = 0; k < 25; ++k)
-            if (r.due(r.call(7), [](int*) {})) { asked++; r.reset(7); }
+            if (r.due(r.call(7), [](int*) {})) { asked++; r.failed(7); }
         CHECK(asked == 5 && r.graphs() == 0);
+        for (int k = 0; k < 5000; ++k)
+            if (r.due(r.call(7), [](int*) {})) { asked++; r.failed(7); }
+        CHECK(asked == int(R::GRAPHS));  // and not for ever
     }
     return bad != 0;
 }
