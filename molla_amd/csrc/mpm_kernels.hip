@@ -1507,7 +1507,7 @@ hipError_t launch_gather_prepare(const StepArgs& a, float* affine, int blocks, h
     return hipGetLastError();
 }
 
-// One block per active tile.  For each cell, the particles of the 27 neighbour
+// One block per active tile, or a wave.  For each cell, the particles of the 27 neighbour
 // tiles are listed in tile order dx + 3 dy + 9 dz, then in ascending sorted
 // slot (mpm_deterministic_p2g.wgsl:100-144), and summed in a fixed order, so
 // the result is bitwise repeatable: 16 sums of every 16th particle, then a
@@ -1532,6 +1532,16 @@ hipError_t launch_gather_prepare(const StepArgs& a, float* affine, int blocks, h
 // one serial sum); a lane per record and channel reads each record once for
 // four cells, 6 LDS instructions per 16 records: 38 us, and 35 with a batch's
 // loads issued before the sums of the one before.
+// A block fills its CU, so a grid of many thin tiles (20,000 particles over
+// 128^3 cells: 32,768 active tiles of 5 candidates) waits for one tile after
+// the other, 641 us against 191 with a tile per wave.  Above GATHER_BLOCKS
+// tiles a block therefore takes 16 at once, a wave sums a tile of up to
+// GATHER_WAVE_RECS records by itself, row by row and in the same order, and
+// what is left goes to the block.  Two substeps with / without it: 1,000
+// particles over 64^3 289 / 374 us, 20,000 over 128^3 879 / 1,780, 200,000 921
+// / 1,860, 1 M 2,382 / 2,364; 200,000 within 12^3 cells 1,177 / 1,231.  Up to
+// GATHER_BLOCKS tiles the block's whole attention is faster: 50 particles in
+// 16^3 126 us against 149, 16,384 sand particles (4 substeps) 170 / 176.
 constexpr int GATHER_THREADS = 1024;
 constexpr int GATHER_WAVES = GATHER_THREADS / 64;
 constexpr int GATHER_PER = 4;
@@ -1539,6 +1549,9 @@ constexpr int GATHER_FLY = 2;  // records per lane in flight
 constexpr int GATHER_STEP = 16 * GATHER_FLY;
 constexpr int GATHER_RECS = 512;
 constexpr int GATHER_LIST = 8192;
+constexpr int GATHER_WAVE_RECS = GATHER_RECS / GATHER_WAVES;
+constexpr int GATHER_BLOCKS = 512;
+static_assert(GATHER_WAVE_RECS <= GATHER_STEP && GATHER_RECS + GATHER_STEP >= 8 * GATHER_STEP, "four lists of a step each");
 
 // A particle relative to a tile: the four channels as c + r0 d0 + r1 d1 + r2 d2
 // (mass: r = 0), the weight product of the tile's 4 x 4 cell columns in x and y
@@ -1553,6 +1566,87 @@ struct alignas(16) GatherRec {
     float pad[6];  // 52 words: 16 records' rows lie in different LDS banks
 };
 
+// Stencil base of a position relative to the tile tc (the tile's first cell's
+// offset in it) and its fraction.
+__device__ __forceinline__ void gather_stencil(const SceneDev& sc, const int* tc, const float* x, int* r, float* fx) {
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        const float xp = (x[k] - sc.origin[k]) * sc.inv_dx;
+        const float bf = floorf(xp - 0.5f);
+        fx[k] = xp - bf;
+        r[k] = 4 * tc[k] - (int(bf) - sc.window[k]);
+    }
+}
+
+// A particle's record; returns its x-rows of the tile (bit y + 4 z).
+__device__ __forceinline__ uint32_t gather_record(const SceneDev& sc, const int* tc, const float* px, const float* A,
+                                                  float mass, GatherRec& q) {
+    int r[3];
+    float fx[3];
+    gather_stencil(sc, tc, px, r, fx);
+    float w[3][4], d[3][4];  // weight (-1: none) and node offset of the tile's cells
+    uint32_t in[3] = {0u, 0u, 0u}, rm = 0u;
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {
+        float wk[3];
+        quad_weights(fx[k], wk);
+#pragma unroll
+        for (int c2 = 0; c2 < 4; ++c2) {
+            const int off = r[k] + c2;
+            w[k][c2] = off == 0 ? wk[0] : (off == 1 ? wk[1] : (off == 2 ? wk[2] : -1.0f));
+            d[k][c2] = (float(off) - fx[k]) * sc.dx;
+            if (off >= 0 && off <= 2) in[k] |= 1u << c2;
+        }
+    }
+#pragma unroll
+    for (int z = 0; z < 4; ++z)
+        if (in[2] & (1u << z)) rm |= in[1] << (4 * z);
+#pragma unroll
+    for (int y = 0; y < 4; ++y) {
+        float v[4];
+#pragma unroll
+        for (int c2 = 0; c2 < 4; ++c2) v[c2] = w[0][c2] < 0.f || w[1][y] < 0.f ? -1.0f : w[0][c2] * w[1][y];
+        q.wxy[y] = make_float4(v[0], v[1], v[2], v[3]);
+        q.z[y] = make_float2(w[2][y], d[2][y]);
+    }
+    q.dy = make_float4(d[1][0], d[1][1], d[1][2], d[1][3]);
+    q.x = make_float2(float(r[0]), fx[0]);
+    q.row[0] = make_float4(mass, 0.f, 0.f, 0.f);
+#pragma unroll
+    for (int k = 0; k < 3; ++k) q.row[1 + k] = make_float4(A[9 + k], A[3 * k], A[3 * k + 1], A[3 * k + 2]);
+    return rm;
+}
+
+// Adds a record to the lane's four cells of the x-row (cy, cz), channel
+// lane & 3.
+__device__ __forceinline__ void gather_add(const GatherRec& q, int cy, int cz, float dx, float* acc) {
+    const float4 r = q.row[threadIdx.x & 3], wv = q.wxy[cy];
+    const float2 z = q.z[cz], qx = q.x;
+    const float base = r.x + r.z * reinterpret_cast<const float*>(&q.dy)[cy] + r.w * z.y;
+    const float w[4] = {wv.x, wv.y, wv.z, wv.w};
+#pragma unroll
+    for (int c2 = 0; c2 < 4; ++c2) {
+        const float t = w[c2] * z.x * (base + r.y * ((qx.x + float(c2) - qx.y) * dx));
+        acc[c2] += w[c2] < 0.f ? 0.f : t;
+    }
+}
+
+// The tree over the 16 sums, and the row's cells.
+__device__ __forceinline__ void gather_store(const SceneDev& sc, const int* tc, uint32_t t, int cy, int cz, float* acc,
+                                             float4* gmp) {
+    const int lane = threadIdx.x & 63, ch = lane & 3, grp = lane >> 2;
+#pragma unroll
+    for (int c2 = 0; c2 < 4; ++c2)
+#pragma unroll
+        for (int o = 4; o < 64; o *= 2) acc[c2] += __shfl_xor(acc[c2], o, 64);
+    if (grp >= 4) return;  // lane's cell of the row
+    const int G = int(sc.G);
+    const bool valid = 4 * tc[0] + grp < G && 4 * tc[1] + cy < G && 4 * tc[2] + cz < G;
+    const uint32_t c = (t << 6) | uint32_t(grp | (cy << 2) | (cz << 4));
+    const float v = grp == 0 ? acc[0] : (grp == 1 ? acc[1] : (grp == 2 ? acc[2] : acc[3]));
+    reinterpret_cast<float*>(gmp)[4 * (size_t)c + ch] = valid ? v : 0.f;
+}
+
 __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const uint32_t* __restrict__ tile_scene,
                                                                const uint32_t* __restrict__ lb,
                                                                const float* __restrict__ aff,
@@ -1562,50 +1656,137 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
     __shared__ uint16_t rows[GATHER_RECS];      // bit y + 4 z: the record reaches that x-row of the tile
     __shared__ uint16_t wlist[GATHER_WAVES][GATHER_RECS + GATHER_STEP];
     __shared__ uint32_t slots[GATHER_LIST];
-    __shared__ uint32_t rbeg[9], roff[10];
+    __shared__ alignas(16) uint32_t rbeg[GATHER_WAVES][12], roff[GATHER_WAVES][12];  // each wave's tile's ranges
     __shared__ uint32_t wcnt[64];  // [GATHER_PER][GATHER_WAVES]
+    __shared__ uint4 whole[GATHER_WAVES];  // a wave's tile that needs the block: id (~0: none), scene, coordinates
     static_assert(GATHER_PER * GATHER_WAVES <= 64, "one lane per count");
     const uint32_t n = *count;
     const int tid = threadIdx.x, lane = tid & 63, wave = wave_id();
     const uint32_t cap = a.cap;
-    // lane: channel, record of a step's 16; wave: the tile's row
-    const int ch = lane & 3, grp = lane >> 2, cy = wave & 3, cz = wave >> 2;
+    const uint64_t lt = (1ull << lane) - 1ull;
     if (tid < int(sizeof(GatherRec) / 4))
         reinterpret_cast<float*>(&rec[GATHER_RECS])[tid] = tid >= 16 && tid < 32 ? -1.f : 0.f;
-    for (uint32_t i = blockIdx.x; i < n; i += gridDim.x) {
-        const uint32_t t = list[i];
-        const SceneDev sc = const_load(a.scenes + tile_scene[t]);
+    __syncthreads();
+    auto tile = [&](uint32_t t, uint32_t scene, SceneDev& sc, int* tc) __attribute__((always_inline)) {
+        sc = const_load(a.scenes + scene);
         const uint32_t tl = t - sc.tile_base;
+        tc[0] = int(tl % sc.W);
+        tc[1] = int((tl / sc.W) % sc.W);
+        tc[2] = int(tl / (sc.W * sc.W));
+    };
+    // slot of candidate j of a wave's tile, and whether its stencil reaches the tile
+    auto candidate = [&](int w, uint32_t j) __attribute__((always_inline)) {
+        int r = 0;
+#pragma unroll
+        for (int q = 1; q < 9; ++q) r += j >= roff[w][q] ? 1 : 0;
+        return rbeg[w][r] + (j - roff[w][r]);
+    };
+    auto reaches = [&](const SceneDev& sc, const int* tc, uint32_t j) __attribute__((always_inline)) {
+        const float x[3] = {a.ps[(size_t)CX * cap + j], a.ps[(size_t)(CX + 1) * cap + j],
+                            a.ps[(size_t)(CX + 2) * cap + j]};
+        int r[3];
+        float fx[3];
+        gather_stencil(sc, tc, x, r, fx);
+        bool hit = true;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) hit = hit && r[k] >= -3 && r[k] <= 2;
+        return hit;
+    };
+    float px[3], A[12], mass = 0.f;
+    auto load = [&](uint32_t j) __attribute__((always_inline)) {
+#pragma unroll
+        for (int k = 0; k < 3; ++k) px[k] = a.ps[(size_t)(CX + k) * cap + j];
+#pragma unroll
+        for (int k = 0; k < 12; ++k) A[k] = aff[(size_t)k * cap + j];
+        mass = a.ps[(size_t)CMASS * cap + j];
+    };
+    // The ranges of the wave's tile; their particles.
+    auto ranges = [&](const SceneDev& sc, const int* tc) __attribute__((always_inline)) {
         const int W = int(sc.W);
-        const int tc[3] = {int(tl % sc.W), int((tl / sc.W) % sc.W), int(tl / (sc.W * sc.W))};
-        if (tid < 9) {
-            const int ny = tc[1] + tid % 3 - 1, nz = tc[2] + tid / 3 - 1;
-            uint32_t b = 0u, e = 0u;
+        uint32_t b = 0u, e = 0u;
+        if (lane < 9) {
+            const int ny = tc[1] + lane % 3 - 1, nz = tc[2] + lane / 3 - 1;
             if (ny >= 0 && nz >= 0 && ny < W && nz < W) {
                 const uint32_t row = sc.tile_base + uint32_t(W * (ny + W * nz));
                 b = lb[row + uint32_t(max(tc[0] - 1, 0))];
                 e = lb[row + uint32_t(min(tc[0] + 1, W - 1)) + 1u];
             }
-            rbeg[tid] = b;
-            roff[tid + 1] = e - b;
         }
-        __syncthreads();
-        if (tid == 0) {
-            roff[0] = 0u;
-            for (int r = 1; r < 10; ++r) roff[r] += roff[r - 1];
+        const uint32_t incl = wave_incl_scan(e - b);
+        if (lane < 9) {
+            rbeg[wave][lane] = b;
+            roff[wave][lane + 1] = incl;
         }
-        __syncthreads();
-        const uint32_t total = roff[9];
-        // base cell relative to the tile and fractional offset of a position
-        auto stencil = [&](const float* x, int* r, float* fx) {
+        if (lane == 0) roff[wave][0] = 0u;
+        __builtin_amdgcn_wave_barrier();
+        return (uint32_t)__shfl(int(incl), 63, 64);
+    };
+    // The wave's tile; false: it needs the block.
+    auto by_wave = [&](const SceneDev& sc, const int* tc, uint32_t t, uint32_t total) __attribute__((always_inline)) {
+        if (total > uint32_t(GATHER_LIST / GATHER_WAVES)) return false;
+        uint32_t* own = slots + wave * (GATHER_LIST / GATHER_WAVES);
+        uint32_t held = 0u;
+        for (uint32_t c0 = 0; c0 < total && held <= uint32_t(GATHER_WAVE_RECS); c0 += 64u * GATHER_PER) {
+            uint32_t slot[GATHER_PER];
+            bool hit[GATHER_PER];
 #pragma unroll
-            for (int k = 0; k < 3; ++k) {
-                const float xp = (x[k] - sc.origin[k]) * sc.inv_dx;
-                const float bf = floorf(xp - 0.5f);
-                fx[k] = xp - bf;
-                r[k] = 4 * tc[k] - (int(bf) - sc.window[k]);  // offset of the tile's first cell
+            for (int u = 0; u < GATHER_PER; ++u) {
+                const uint32_t j = c0 + uint32_t(64 * u + lane);
+                hit[u] = j < total;
+                slot[u] = hit[u] ? candidate(wave, j) : 0u;
             }
-        };
+#pragma unroll
+            for (int u = 0; u < GATHER_PER; ++u) {
+                if (hit[u]) hit[u] = reaches(sc, tc, slot[u]);
+                const uint64_t m = __ballot(hit[u]);
+                if (hit[u]) own[held + uint32_t(__popcll(m & lt))] = slot[u];
+                held += uint32_t(__popcll(m));
+            }
+        }
+        if (held > uint32_t(GATHER_WAVE_RECS)) return false;
+        if (held == 0u) {
+            a.gmp[(size_t)(t << 6) | uint32_t(lane)] = make_float4(0.f, 0.f, 0.f, 0.f);
+        } else {
+            __builtin_amdgcn_wave_barrier();
+            uint32_t rm = 0u;
+            if (uint32_t(lane) < held) {
+                load(own[lane]);
+                rm = gather_record(sc, tc, px, A, mass, rec[wave * GATHER_WAVE_RECS + lane]);
+            }
+            // four rows in flight; a row's list is one step
+#pragma unroll 1
+            for (int cz = 0; cz < 4; ++cz) {
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int cy = 0; cy < 4; ++cy) {
+                    uint16_t* wl = wlist[wave] + 2 * GATHER_STEP * cy;
+                    const bool on = (rm >> (4 * cz + cy)) & 1u;
+                    const uint64_t m = __ballot(on);
+                    if (on) wl[__popcll(m & lt)] = uint16_t(wave * GATHER_WAVE_RECS + lane);
+                    if (lane < GATHER_STEP) wl[__popcll(m) + lane] = uint16_t(GATHER_RECS);
+                }
+                __builtin_amdgcn_wave_barrier();
+                float acc[4][4];
+#pragma unroll
+                for (int cy = 0; cy < 4; ++cy)
+#pragma unroll
+                    for (int c2 = 0; c2 < 4; ++c2) acc[cy][c2] = 0.f;
+#pragma unroll 1
+                for (uint32_t g = 0; g < held; g += 16u)
+#pragma unroll
+                    for (int cy = 0; cy < 4; ++cy)
+                        gather_add(rec[wlist[wave][2 * GATHER_STEP * cy + g + (lane >> 2)]], cy, cz, sc.dx, acc[cy]);
+#pragma unroll
+                for (int cy = 0; cy < 4; ++cy) gather_store(sc, tc, t, cy, cz, acc[cy], a.gmp);
+            }
+        }
+        if (lane == 0) a.tile_flag[t] |= FLAG_GMP;
+        return true;
+    };
+    // A tile by the whole block, with the ranges that wave w has found.
+    auto by_block = [&](const SceneDev& sc, const int* tc, uint32_t t, int w) __attribute__((always_inline)) {
+        const int cy = wave & 3, cz = wave >> 2;  // the wave's row
+        const uint32_t total = roff[w][9];
         float acc[4] = {0.f, 0.f, 0.f, 0.f};
         uint32_t held = 0u;  // slots in the list (block-uniform)
         for (uint32_t c0 = 0; c0 < total; c0 += GATHER_THREADS * GATHER_PER) {
@@ -1614,27 +1795,13 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
 #pragma unroll
             for (int u = 0; u < GATHER_PER; ++u) {
                 const uint32_t j = c0 + uint32_t(u * GATHER_THREADS + tid);
-                slot[u] = 0u;
                 hit[u] = j < total;
-                if (hit[u]) {
-                    int r = 0;
-#pragma unroll
-                    for (int q = 1; q < 9; ++q) r += j >= roff[q] ? 1 : 0;
-                    slot[u] = rbeg[r] + (j - roff[r]);
-                }
+                slot[u] = hit[u] ? candidate(w, j) : 0u;
             }
             uint64_t m[GATHER_PER];
 #pragma unroll
             for (int u = 0; u < GATHER_PER; ++u) {
-                int r[3];
-                float fx[3];
-                if (hit[u]) {
-                    const float x[3] = {a.ps[(size_t)CX * cap + slot[u]], a.ps[(size_t)(CX + 1) * cap + slot[u]],
-                                        a.ps[(size_t)(CX + 2) * cap + slot[u]]};
-                    stencil(x, r, fx);
-#pragma unroll
-                    for (int k = 0; k < 3; ++k) hit[u] = hit[u] && r[k] >= -3 && r[k] <= 2;
-                }
+                if (hit[u]) hit[u] = reaches(sc, tc, slot[u]);
                 m[u] = __ballot(hit[u]);
                 if (lane == 0) wcnt[u * GATHER_WAVES + wave] = uint32_t(__popcll(m[u]));
             }
@@ -1644,7 +1811,7 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
 #pragma unroll
             for (int u = 0; u < GATHER_PER; ++u) {
                 const uint32_t at = held + (uint32_t)__shfl(int(incl - c), u * GATHER_WAVES + wave, 64);
-                if (hit[u]) slots[at + uint32_t(__popcll(m[u] & ((1ull << lane) - 1ull)))] = slot[u];
+                if (hit[u]) slots[at + uint32_t(__popcll(m[u] & lt))] = slot[u];
             }
             held += (uint32_t)__shfl(int(incl), 63, 64);
             __syncthreads();
@@ -1652,59 +1819,11 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
             const bool last = c0 + GATHER_THREADS * GATHER_PER >= total;
             if (!last && held + GATHER_THREADS * GATHER_PER <= GATHER_LIST) continue;
             // a batch's loads are issued before the sums of the batch before it
-            float px[3], A[12], mass = 0.f;
-            auto load = [&](uint32_t j) __attribute__((always_inline)) {
-#pragma unroll
-                for (int k = 0; k < 3; ++k) px[k] = a.ps[(size_t)(CX + k) * cap + j];
-#pragma unroll
-                for (int k = 0; k < 12; ++k) A[k] = aff[(size_t)k * cap + j];
-                mass = a.ps[(size_t)CMASS * cap + j];
-            };
             if (tid < GATHER_RECS && uint32_t(tid) < held) load(slots[tid]);
             for (uint32_t b0 = 0; b0 < held; b0 += GATHER_RECS) {
                 const uint32_t cnt = min(held - b0, uint32_t(GATHER_RECS));
-                if (tid < GATHER_RECS) {
-                    uint32_t rm = 0u;
-                    if (uint32_t(tid) < cnt) {
-                        int r[3];
-                        float fx[3];
-                        stencil(px, r, fx);
-                        GatherRec& q = rec[tid];
-                        float w[3][4], d[3][4];  // weight (-1: none) and node offset of the tile's cells
-                        uint32_t in[3] = {0u, 0u, 0u};
-#pragma unroll
-                        for (int k = 0; k < 3; ++k) {
-                            float wk[3];
-                            quad_weights(fx[k], wk);
-#pragma unroll
-                            for (int c2 = 0; c2 < 4; ++c2) {
-                                const int off = r[k] + c2;
-                                w[k][c2] = off == 0 ? wk[0] : (off == 1 ? wk[1] : (off == 2 ? wk[2] : -1.0f));
-                                d[k][c2] = (float(off) - fx[k]) * sc.dx;
-                                if (off >= 0 && off <= 2) in[k] |= 1u << c2;
-                            }
-                        }
-#pragma unroll
-                        for (int z = 0; z < 4; ++z)
-                            if (in[2] & (1u << z)) rm |= in[1] << (4 * z);
-#pragma unroll
-                        for (int y = 0; y < 4; ++y) {
-                            float v[4];
-#pragma unroll
-                            for (int c2 = 0; c2 < 4; ++c2)
-                                v[c2] = w[0][c2] < 0.f || w[1][y] < 0.f ? -1.0f : w[0][c2] * w[1][y];
-                            q.wxy[y] = make_float4(v[0], v[1], v[2], v[3]);
-                            q.z[y] = make_float2(w[2][y], d[2][y]);
-                        }
-                        q.dy = make_float4(d[1][0], d[1][1], d[1][2], d[1][3]);
-                        q.x = make_float2(float(r[0]), fx[0]);
-                        q.row[0] = make_float4(mass, 0.f, 0.f, 0.f);
-#pragma unroll
-                        for (int k = 0; k < 3; ++k)
-                            q.row[1 + k] = make_float4(A[9 + k], A[3 * k], A[3 * k + 1], A[3 * k + 2]);
-                    }
-                    rows[tid] = uint16_t(rm);
-                }
+                if (tid < GATHER_RECS)
+                    rows[tid] = uint16_t(uint32_t(tid) < cnt ? gather_record(sc, tc, px, A, mass, rec[tid]) : 0u);
                 __syncthreads();
                 if (tid < GATHER_RECS && b0 + GATHER_RECS + uint32_t(tid) < held)
                     load(slots[b0 + GATHER_RECS + uint32_t(tid)]);
@@ -1714,43 +1833,63 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                 for (uint32_t g = 0; g < cnt; g += 64) {
                     const bool on = (rows[g + uint32_t(lane)] >> wave) & 1u;
                     const uint64_t mm = __ballot(on);
-                    if (on) wlist[wave][len + uint32_t(__popcll(mm & ((1ull << lane) - 1ull)))] = uint16_t(g + lane);
+                    if (on) wlist[wave][len + uint32_t(__popcll(mm & lt))] = uint16_t(g + lane);
                     len += uint32_t(__popcll(mm));
                 }
                 if (lane < GATHER_STEP) wlist[wave][len + uint32_t(lane)] = uint16_t(GATHER_RECS);
                 __builtin_amdgcn_wave_barrier();
-                for (uint32_t g = 0; g < len; g += GATHER_STEP) {
+                for (uint32_t g = 0; g < len; g += GATHER_STEP)
 #pragma unroll
-                    for (int f = 0; f < GATHER_FLY; ++f) {
-                        const GatherRec& q = rec[wlist[wave][g + uint32_t(16 * f + grp)]];
-                        const float4 r = q.row[ch], wv = q.wxy[cy];
-                        const float2 z = q.z[cz], qx = q.x;
-                        const float base = r.x + r.z * reinterpret_cast<const float*>(&q.dy)[cy] + r.w * z.y;
-                        const float w[4] = {wv.x, wv.y, wv.z, wv.w};
-#pragma unroll
-                        for (int c2 = 0; c2 < 4; ++c2) {
-                            const float t = w[c2] * z.x * (base + r.y * ((qx.x + float(c2) - qx.y) * sc.dx));
-                            acc[c2] += w[c2] < 0.f ? 0.f : t;
-                        }
-                    }
-                }
+                    for (int f = 0; f < GATHER_FLY; ++f)
+                        gather_add(rec[wlist[wave][g + uint32_t(16 * f + (lane >> 2))]], cy, cz, sc.dx, acc);
                 __syncthreads();
             }
             held = 0u;
         }
-#pragma unroll
-        for (int c2 = 0; c2 < 4; ++c2)
-#pragma unroll
-            for (int o = 4; o < 64; o *= 2) acc[c2] += __shfl_xor(acc[c2], o, 64);
-        if (grp < 4) {  // lane's cell of the row
-            const int G = int(sc.G);
-            const bool valid = 4 * tc[0] + grp < G && 4 * tc[1] + cy < G && 4 * tc[2] + cz < G;
-            const uint32_t c = (t << 6) | uint32_t(grp | (cy << 2) | (cz << 4));
-            const float v = grp == 0 ? acc[0] : (grp == 1 ? acc[1] : (grp == 2 ? acc[2] : acc[3]));
-            reinterpret_cast<float*>(a.gmp)[4 * (size_t)c + ch] = valid ? v : 0.f;
-        }
+        gather_store(sc, tc, t, cy, cz, acc, a.gmp);
         if (tid == 0) a.tile_flag[t] |= FLAG_GMP;
-        __syncthreads();  // rbeg, roff and the records are reused by the next tile
+    };
+    // few tiles: one per block, whose waves all find its ranges; else a tile
+    // per wave, on as many blocks
+    const uint32_t nb = min(gridDim.x, max(n / 8u, uint32_t(GATHER_BLOCKS)));
+    SceneDev sc;
+    int tc[3];
+    uint32_t scene = ~0u;  // whose record sc is
+    if (n <= nb) {
+        if (blockIdx.x >= n) return;
+        const uint32_t t = list[blockIdx.x];
+        tile(t, tile_scene[t], sc, tc);
+        ranges(sc, tc);
+        by_block(sc, tc, t, wave);
+        return;
+    }
+    if (blockIdx.x >= nb) return;
+    for (uint32_t i0 = blockIdx.x; i0 < n; i0 += nb * GATHER_WAVES) {
+        const uint32_t i = i0 + nb * uint32_t(wave);
+        uint4 left = make_uint4(~0u, 0u, 0u, 0u);
+        if (i < n) {
+            const uint32_t t = list[i];
+            scene = tile_scene[t];
+            tile(t, scene, sc, tc);
+            if (!by_wave(sc, tc, t, ranges(sc, tc)))
+                left = make_uint4(t, scene, uint32_t(tc[0]) | uint32_t(tc[1]) << 16, uint32_t(tc[2]));
+        }
+        if (lane == 0) whole[wave] = left;
+        __syncthreads();
+        for (int w = 0; w < GATHER_WAVES; ++w) {
+            const uint4 q = whole[w];
+            const uint32_t t = uint32_t(__builtin_amdgcn_readfirstlane(int(q.x)));
+            if (t == ~0u) continue;
+            const uint32_t its = uint32_t(__builtin_amdgcn_readfirstlane(int(q.y)));
+            const uint32_t xy = uint32_t(__builtin_amdgcn_readfirstlane(int(q.z)));
+            if (its != scene) sc = const_load(a.scenes + its);
+            scene = its;
+            tc[0] = int(xy & 0xffffu);
+            tc[1] = int(xy >> 16);
+            tc[2] = __builtin_amdgcn_readfirstlane(int(q.w));
+            by_block(sc, tc, t, w);
+        }
+        __syncthreads();  // the ranges and the marks are the next tiles'
     }
 }
 
