@@ -1071,10 +1071,9 @@ hipError_t launch_reorder(const float* src, float* dst, uint32_t cap, const uint
                           uint32_t* slot_of_id, const RecordArgs& rec, hipStream_t s) {
     if (n == 0) return hipSuccess;
     const unsigned blocks = std::min<unsigned>((n + 255) / 256, 16384u);
-    // nine threads per static tile, whose count is on the device: at most one
-    // per tile row of the grid, and few enough not to be the launch's work
-    const unsigned rec_blocks =
-        rec.srec ? std::min<unsigned>({rec.max_static / 28u + 1u, std::max(8u, n / 1024u), 2048u}) : 0u;
+    // nine threads per static tile, whose count is on the device: at most 27
+    // tiles a particle; blocks without a tile end at once
+    const unsigned rec_blocks = rec.srec ? std::min<unsigned>({rec.max_static / 28u + 1u, n, 1024u}) : 0u;
     hipLaunchKernelGGL(k_reorder, dim3(blocks + rec_blocks), dim3(256), 0, s, src, dst, cap, src_slot, n, slot_of_id,
                        rec, rec_blocks);
     return hipGetLastError();
