@@ -89,6 +89,7 @@ struct mpm_sim {
     uint32_t max_W = 0;         // tiles of the longest tile row
     uint32_t* list[2] = {nullptr, nullptr};
     uint32_t* status = nullptr;  // ST_WORDS u32
+    uint32_t* tickets = nullptr;  // TICKET_WORDS u32
     uint32_t* slot_of_id = nullptr;
     bool index_valid = false;  // slot_of_id describes the current slots (the fused layout sorts leave it behind)
     uint32_t* keys = nullptr;
@@ -288,7 +289,7 @@ void release(mpm_sim* s) {
     }
     for (hipEvent_t e : s->ev_pool) (void)hipEventDestroy(e);
     void* bufs[] = {s->d_scenes, s->d_mats, s->ps[0], s->ps[1], s->gmp, s->gv, s->tile_flag, s->tile_scene,
-                    s->list[0], s->list[1], s->status, s->slot_of_id, s->keys, s->vals, s->sort_scratch,
+                    s->list[0], s->list[1], s->status, s->tickets, s->slot_of_id, s->keys, s->vals, s->sort_scratch,
                     s->d_chunks, s->affine, s->staging, s->tile_lb, s->slist,
                     s->src_slot, s->chunk_box, s->part, s->schunks, s->chunk_of_slot, s->lscan, s->tile_slot,
                     s->tile_mark, s->slot_tile, s->defer_list, s->srec};
@@ -505,7 +506,7 @@ int clear_grid(mpm_sim* s) {
         return MPM_OK;
     }
     HIP_TRY(s, mpm::launch_clear_tiles(griddev(s), s->list[s->list_cur], s->status + mpm::ST_COUNT0 + s->list_cur,
-                                       s->status + mpm::ST_TICKET, grid_blocks(s), s->stream));
+                                       s->tickets, grid_blocks(s), s->stream));
     s->grid_dirty = false;
     return MPM_OK;
 }
@@ -695,7 +696,7 @@ int grid_update(mpm_sim* s, float dt, bool zero_after, bool react = false) {
                                            rigid ? &rg : nullptr, grid_split(s)));
         HIP_TRY(s, mpm::launch_implicit_sweeps(s->d_scenes, g, s->gv2, s->jacobi_iters, s->list[s->list_cur],
                                                cur_count, dt, grid_blocks(s),
-                                               zero_after ? s->status + mpm::ST_TICKET : nullptr, s->stream,
+                                               zero_after ? s->tickets : nullptr, s->stream,
                                                rigid ? &rg : nullptr));
         if (rg.wrench && !s->prescribed)
             HIP_TRY(s, mpm::launch_rigid_shell(s->d_scenes, g, s->list[s->list_cur], cur_count, dt, rg,
@@ -969,6 +970,7 @@ int create(const mpm_scene_config* cfgs, uint32_t n_scenes, mpm_sim** out) {
     HIP_TRY(s, dalloc(&s->ps[0], (size_t)mpm::NCOMP * s->cap));
     HIP_TRY(s, dalloc(&s->ps[1], (size_t)mpm::NCOMP * s->cap));
     HIP_TRY(s, dalloc(&s->status, mpm::ST_WORDS));
+    HIP_TRY(s, dalloc(&s->tickets, mpm::TICKET_WORDS));
     HIP_TRY(s, dalloc(&s->slot_of_id, s->cap));
     HIP_TRY(s, dalloc(&s->keys, s->cap));
     HIP_TRY(s, dalloc(&s->vals, s->cap));
@@ -978,6 +980,7 @@ int create(const mpm_scene_config* cfgs, uint32_t n_scenes, mpm_sim** out) {
     HIP_TRY(s, dalloc(&s->d_chunks, (size_t)s->max_chunks));
     HIP_TRY(s, dalloc(&s->staging, (size_t)9 * s->cap));
     HIP_TRY(s, hipMemsetAsync(s->status, 0, mpm::ST_WORDS * 4, s->stream));
+    HIP_TRY(s, hipMemsetAsync(s->tickets, 0, mpm::TICKET_WORDS * 4, s->stream));
     HIP_TRY(s, hipMemsetAsync(s->ps[0], 0, (size_t)mpm::NCOMP * s->cap * 4, s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     (void)cells;
@@ -1342,7 +1345,7 @@ int diff_backward_pass(mpm_sim* s, bool has_gv, bool checked, Stage& span) {
             }
             mpm::GridDev gc = g;
             gc.gmp = s->gadj;
-            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), s->status + mpm::ST_TICKET, gb, s->stream));
+            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), s->tickets, gb, s->stream));
             L = R;
             continue;
         }
@@ -1361,7 +1364,7 @@ int diff_backward_pass(mpm_sim* s, bool has_gv, bool checked, Stage& span) {
             HIP_TRY(s, mpm::launch_adj_p2g(q, blocks, s->stream));
             mpm::GridDev gc = g;
             gc.gmp = s->gadj;
-            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), s->status + mpm::ST_TICKET, gb, s->stream));
+            HIP_TRY(s, mpm::launch_clear_tiles(gc, s->list[R], count(R), s->tickets, gb, s->stream));
         }
         L = R;
     }

@@ -42,12 +42,19 @@ constexpr uint32_t FAULT_NUMERICAL = 2u;
 // ST_COUNT0/1: the two dynamic active-tile lists; ST_SCOUNT: the static list.
 // Sparse tile pool: ST_POOL the tiles marked by the last substep (slots in
 // use, or the demand that overflowed the pool), ST_DEFER the particles whose
-// global-atomic scatter waits for the slots.  ST_TICKET: blocks of a clear or
-// of the last sweep launch that are done (zero between launches).
+// global-atomic scatter waits for the slots.
 enum StatusWord : int {
     ST_FAULT = 0, ST_GATHERS = 1, ST_COUNT0 = 2, ST_COUNT1 = 3, ST_SCOUNT = 4, ST_ESCAPES = 5, ST_NCHUNKS = 6,
-    ST_FALLBACK = 7, ST_POOL = 8, ST_DEFER = 9, ST_TICKET = 10, ST_WORDS = 11
+    ST_FALLBACK = 7, ST_POOL = 8, ST_DEFER = 9, ST_WORDS = 10
 };
+
+// Counters of the blocks of a launch that are done (last_block; zero between
+// launches).  Atomics on one word cost about 35 ns each, 71 us for 2,048
+// blocks, so the blocks count in groups and the last of each group counts the
+// groups: words of their own cache lines, the groups' after the first.
+constexpr uint32_t TICKET_GROUPS = 32;
+constexpr uint32_t TICKET_STRIDE = 32;  // words
+constexpr uint32_t TICKET_WORDS = (1 + TICKET_GROUPS) * TICKET_STRIDE;
 
 struct SceneDev {
     float origin[3];
@@ -212,16 +219,16 @@ hipError_t launch_grid_update(const SceneDev* scenes, const GridDev& g, const ui
 hipError_t launch_rigid_shell(const SceneDev* scenes, const GridDev& g, const uint32_t* dlist,
                               const uint32_t* dcount, float dt, const RigidDev& rg, int blocks, hipStream_t s);
 hipError_t launch_zero_f64(double* p, uint32_t n, hipStream_t s);
-hipError_t launch_clear_tiles(const GridDev& g, const uint32_t* dlist, uint32_t* dcount, uint32_t* ticket, int blocks,
+hipError_t launch_clear_tiles(const GridDev& g, const uint32_t* dlist, uint32_t* dcount, uint32_t* tickets, int blocks,
                               hipStream_t s, float4* also = nullptr);
 // `iters` > 0 semi-implicit Jacobi sweeps over the active tiles: they start
 // from the buffer implicit_first() names (g.gv or the second cell buffer
 // `scratch`), where the grid update has to leave its velocities, and end in
 // g.gv.  Tile flags must still mark this substep's dynamic tiles (FLAG_DYN);
-// `ticket` (a zero word, or null) takes those marks off at the end.
+// `tickets` (TICKET_WORDS zeros, or null) takes those marks off at the end.
 float4* implicit_first(float4* gv, float4* scratch, uint32_t iters);
 hipError_t launch_implicit_sweeps(const SceneDev* scenes, const GridDev& g, float4* scratch, uint32_t iters,
-                                  const uint32_t* dlist, const uint32_t* dcount, float dt, int blocks, uint32_t* ticket,
+                                  const uint32_t* dlist, const uint32_t* dcount, float dt, int blocks, uint32_t* tickets,
                                   hipStream_t s, const RigidDev* rigid = nullptr);
 hipError_t launch_set_u32(uint32_t* p, uint32_t v, hipStream_t s);
 hipError_t launch_snap_counters(const uint32_t* status, uint32_t* dst, hipStream_t s);

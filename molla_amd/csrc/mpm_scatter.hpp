@@ -36,6 +36,19 @@ __device__ __forceinline__ ChunkWalk chunk_walk(uint32_t nch) {
     return {lo + blockIdx.x / NUM_XCD, hi, g / NUM_XCD};
 }
 
+// Whether the calling block is the last of blocks 0 .. busy - 1 to get here
+// (one thread of each calls it, once); the counters are zero again then.
+__device__ __forceinline__ bool last_block(uint32_t* tickets, uint32_t busy) {
+    const uint32_t g = blockIdx.x % TICKET_GROUPS;
+    const uint32_t members = (busy - g + TICKET_GROUPS - 1u) / TICKET_GROUPS;
+    uint32_t* t = tickets + (1u + g) * TICKET_STRIDE;
+    if (atomicAdd(t, 1u) + 1u != members) return false;
+    *t = 0u;
+    if (atomicAdd(tickets, 1u) + 1u != min(busy, TICKET_GROUPS)) return false;
+    *tickets = 0u;
+    return true;
+}
+
 // A record at a wave-uniform address that nothing writes during the launch,
 // through scalar loads: behind a barrier or a store the compiler takes such a
 // record with vector loads, whose fields then sit in vector registers.  The
