@@ -122,6 +122,7 @@ struct mpm_sim {
     int p2g_mode = MPM_P2G_FUSED;
     uint32_t jacobi_iters = 0;  // semi-implicit sweeps per substep (MpmTimeStep::Implicit)
     float4* gv2 = nullptr;      // their ping-pong buffer
+    uint32_t* hcount = nullptr; // pinned: the static tiles of the last sort that has ended (0: none yet; many_tiles)
     uint32_t sort_every = 16;
     int write_vc = 1;
     uint32_t pblocks = 0;
@@ -301,6 +302,7 @@ void release(mpm_sim* s) {
         if (b) (void)hipFree(b);
     if (s->hpin) (void)hipHostFree(s->hpin);
     if (s->mail) (void)hipHostFree(s->mail);
+    if (s->hcount) (void)hipHostFree(s->hcount);
     if (s->stream) (void)hipStreamDestroy(s->stream);
 }
 
@@ -451,6 +453,21 @@ uint32_t chunk_bound(const mpm_sim* s) {
 // Cells of grid storage: every tile of a dense grid, the pool of a sparse one.
 size_t grid_cells(const mpm_sim* s) { return (size_t)(s->pool_cap ? s->pool_cap : s->total_tiles) * 64; }
 
+// The second cell buffer of the semi-implicit sweeps, and the word their rule
+// reads (many_tiles).
+int ensure_implicit(mpm_sim* s) {
+    if (!s->gv2) HIP_TRY(s, dalloc(&s->gv2, grid_cells(s)));
+    if (!s->hcount) {
+        if (hipHostMalloc((void**)&s->hcount, 64, hipHostMallocDefault) == hipSuccess) {
+            *s->hcount = 0u;
+        } else {
+            (void)hipGetLastError();
+            s->hcount = nullptr;
+        }
+    }
+    return MPM_OK;
+}
+
 // The dense tile grid is allocated on first use, so contexts that only order
 // particles (or read keys) never pay for it.
 int ensure_grid(mpm_sim* s) {
@@ -466,7 +483,7 @@ int ensure_grid(mpm_sim* s) {
     }
     HIP_TRY(s, dalloc(&s->gmp, cells));
     HIP_TRY(s, dalloc(&s->gv, cells));
-    if (s->jacobi_iters > 0 && !s->gv2) HIP_TRY(s, dalloc(&s->gv2, cells));
+    if (int rc = s->jacobi_iters > 0 ? ensure_implicit(s) : MPM_OK) return rc;
     HIP_TRY(s, dalloc(&s->tile_flag, s->total_tiles));
     HIP_TRY(s, dalloc(&s->tile_scene, s->total_tiles));
     HIP_TRY(s, dalloc(&s->list[0], s->total_tiles));
@@ -595,6 +612,7 @@ int sort_particles(mpm_sim* s, bool reorder) {
     q.tile_flag = s->tile_flag;
     q.slist = s->slist;
     q.scount = s->status + mpm::ST_SCOUNT;
+    q.host_scount = s->hcount;
     q.tile_lb = s->tile_lb;
     q.keys = s->keys;
     q.src = by_slot ? s->vals : s->src_slot;
@@ -671,6 +689,24 @@ int particle_pass(mpm_sim* s, int mode, float dt, int list_out, float* ps = null
     return MPM_OK;
 }
 
+// Whether the semi-implicit sweeps go one per launch (launch_implicit_sweeps).
+// Three to a launch save launches and cost four times the cell updates, so the
+// line lies where the active tiles fill the chip: a substep of three sweeps,
+// three to a launch / one, 1,300 tiles (300,000 particles) 73 / 79 us, 2,744
+// 107 / 112, 3,400 (1 M) 148 / 142, 4,096 149 / 139, 32,768 (200,000 particles
+// over 128^3) 765 / 601.  The number of tiles is on the device; the sorts also
+// leave it in pinned memory, and what the last sort that has ended wrote there
+// is near enough: both ways leave the same bits.  Before one has, or without
+// sorts, grids beyond the line count as full.
+constexpr uint32_t MANY_TILES = 3072;
+bool many_tiles(const mpm_sim* s) {
+    if (s->jacobi_iters == 0) return false;
+    const uint32_t most = s->pool_cap ? s->pool_cap : s->total_tiles;
+    if (std::min<uint64_t>(most, 27ull * s->n) <= MANY_TILES) return false;
+    const uint32_t tiles = s->hcount ? *static_cast<volatile uint32_t*>(s->hcount) : 0u;
+    return tiles == 0u || s->p2g_mode == MPM_P2G_GLOBAL_ATOMIC || tiles > MANY_TILES;
+}
+
 // `react`: this substep reports the rigid bodies' reaction (the last
 // substep of a step: the reference resets the wrench every substep, so only
 // the last one is observable).
@@ -688,15 +724,16 @@ int grid_update(mpm_sim* s, float dt, bool zero_after, bool react = false) {
         // Semi-implicit step (mpm.rs:2515-2530): the sweeps need this substep's
         // dynamic-tile marks, so the grid update keeps them and the last sweep
         // launch takes them off.
+        const bool many = many_tiles(s);
         mpm::GridDev g0 = g;
-        g0.gv = mpm::implicit_first(s->gv, s->gv2, s->jacobi_iters);
+        g0.gv = mpm::implicit_first(s->gv, s->gv2, s->jacobi_iters, many);
         HIP_TRY(s, mpm::launch_grid_update(s->d_scenes, g0, s->list[s->list_cur], cur_count,
                                            zero_after ? s->status + mpm::ST_COUNT0 + nxt : nullptr, dt,
                                            zero_after ? 2 : 0, parts, grid_blocks(s), s->stream, nullptr,
                                            rigid ? &rg : nullptr, grid_split(s)));
-        HIP_TRY(s, mpm::launch_implicit_sweeps(s->d_scenes, g, s->gv2, s->jacobi_iters, s->list[s->list_cur],
-                                               cur_count, dt, grid_blocks(s),
-                                               zero_after ? s->tickets : nullptr, s->stream,
+        HIP_TRY(s, mpm::launch_implicit_sweeps(s->d_scenes, g, s->gv2, s->jacobi_iters, many,
+                                               s->list[s->list_cur], cur_count, dt, grid_blocks(s), s->tickets,
+                                               zero_after, s->p2g_mode == MPM_P2G_GLOBAL_ATOMIC, s->stream,
                                                rigid ? &rg : nullptr));
         if (rg.wrench && !s->prescribed)
             HIP_TRY(s, mpm::launch_rigid_shell(s->d_scenes, g, s->list[s->list_cur], cur_count, dt, rg,
@@ -798,7 +835,7 @@ GraphKey graph_key(const mpm_sim* s, float dt, uint32_t substeps) {
                     uint32_t(s->grid_dirty), uint32_t(sort_start) | (s->since_sort << 1), uint32_t(s->write_vc),
                     s->pblocks, s->gblocks, s->sort_every, uint32_t(s->has_E),
                     s->ppt | (uint32_t(s->ppt_set) << 2) | (s->seg_tiles << 4) | (s->chunk_ppt << 8) |
-                        (uint32_t(s->index_valid) << 12)};
+                        (uint32_t(s->index_valid) << 12) | (uint32_t(many_tiles(s)) << 13)};
 }
 
 // Captures the step's launches; the host state advances as if they had run.
@@ -999,6 +1036,7 @@ int set_particles(mpm_sim* s, const uint32_t* counts, const float* pos, const fl
     }
     if (total > 0 && !pos) return fail(s, MPM_ERR_INVALID, "positions must not be NULL");
     HIP_TRY(s, hipStreamSynchronize(s->stream));
+    if (s->hcount) *s->hcount = 0u;  // of other particles
     s->n = uint32_t(total);
     s->counts.assign(counts, counts + s->n_scenes);
     s->pbase.clear();
@@ -1830,7 +1868,7 @@ int mpm_set_time_step(mpm_sim* sim, uint32_t jacobi_iters) {
                 return fail(sim, MPM_ERR_INVALID, "the semi-implicit step is defined for MPM_MODEL_SHADER scenes");
     if (jacobi_iters > 1024) return fail(sim, MPM_ERR_INVALID, "jacobi_iters must be <= 1024");
     HIP_TRY(sim, hipStreamSynchronize(sim->stream));
-    if (jacobi_iters > 0 && sim->gmp && !sim->gv2) HIP_TRY(sim, dalloc(&sim->gv2, grid_cells(sim)));
+    if (int rc = jacobi_iters > 0 && sim->gmp ? ensure_implicit(sim) : MPM_OK) return rc;
     sim->jacobi_iters = jacobi_iters;
     drop_graphs(sim);
     return MPM_OK;
@@ -2477,6 +2515,7 @@ int mpm_checkpoint_restore(mpm_sim* sim, const mpm_soil_meta* meta, const uint32
     nc.n_materials = n_rows;
     sim->cfg[0] = nc;
     sim->sh[0] = make_scene(nc, sim->sh[0].tile_base, sim->sh[0].mat_base);
+    if (sim->hcount) *sim->hcount = 0u;  // of other particles
     sim->n = n;
     sim->counts.assign(1, n);
     sim->pbase.assign(1, 0);

@@ -225,11 +225,13 @@ hipError_t launch_clear_tiles(const GridDev& g, const uint32_t* dlist, uint32_t*
 // from the buffer implicit_first() names (g.gv or the second cell buffer
 // `scratch`), where the grid update has to leave its velocities, and end in
 // g.gv.  Tile flags must still mark this substep's dynamic tiles (FLAG_DYN);
-// `tickets` (TICKET_WORDS zeros, or null) takes those marks off at the end.
-float4* implicit_first(float4* gv, float4* scratch, uint32_t iters);
-hipError_t launch_implicit_sweeps(const SceneDev* scenes, const GridDev& g, float4* scratch, uint32_t iters,
+// `end` takes those marks off at the end (tickets: TICKET_WORDS zeros; listed:
+// the list holds every tile).  many: one sweep per launch, a wave per tile, for
+// thousands of active tiles; the same bits.
+float4* implicit_first(float4* gv, float4* scratch, uint32_t iters, bool many);
+hipError_t launch_implicit_sweeps(const SceneDev* scenes, const GridDev& g, float4* scratch, uint32_t iters, bool many,
                                   const uint32_t* dlist, const uint32_t* dcount, float dt, int blocks, uint32_t* tickets,
-                                  hipStream_t s, const RigidDev* rigid = nullptr);
+                                  bool end, bool listed, hipStream_t s, const RigidDev* rigid = nullptr);
 hipError_t launch_set_u32(uint32_t* p, uint32_t v, hipStream_t s);
 hipError_t launch_snap_counters(const uint32_t* status, uint32_t* dst, hipStream_t s);
 hipError_t launch_copy_u32(const uint32_t* src, uint32_t* dst, hipStream_t s);
@@ -328,6 +330,7 @@ struct LayoutArgs {
     uint32_t* tile_flag;  // the static bit is rewritten
     uint32_t* slist;      // static active list, ascending tiles
     uint32_t* scount;
+    uint32_t* host_scount;  // null, or pinned host memory that receives the static count too
     uint32_t* tile_lb;    // first sorted slot of every tile key, and n (total_tiles + 1)
     uint32_t* keys;       // sorted tile keys
     uint32_t* src;        // launch_layout_one: previous slot of every sorted slot

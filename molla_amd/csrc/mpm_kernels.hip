@@ -735,14 +735,34 @@ hipError_t launch_zero_f64(double* p, uint32_t n, hipStream_t s) {
 // cells around it into LDS and sweeps a region that shrinks by one cell per
 // sweep, so the K sweeps of a tile need nothing of its neighbours' blocks.
 // The halo is computed again by every block that needs it (K = 3: 792 cell
-// updates for 192), which costs less than the launches it saves: 32,768 sand
-// particles, three sweeps 9.7 us in a trace against 19.5 us as one launch each
-// and 3.9 us for the copy that made an odd count end in gv.  A frame of 8
-// substeps with three against one sweep per launch: 8,000 particles 273 / 361
-// us, 100,000 376 / 409, 1 M 1,253 / 1,380, 3 M 3,343 / 3,630 us.
+// updates for 192), which costs less than the launches it saves up to some
+// 3,000 tiles: 32,768 sand particles, three sweeps 9.7 us in a trace against
+// 19.5 us as one launch each and 3.9 us for the copy that made an odd count
+// end in gv.  A frame of 8 substeps with three against one sweep per launch:
+// 8,000 particles 273 / 361 us, 100,000 376 / 409.
 // `tickets` (not null in the launch that ends the substep's sweeps): where the
 // dynamic list holds tiles, the last block to finish takes FLAG_DYN off them,
 // which every block has read by then.
+// A cell of mass m > 1e-9 and the sum of its cnt neighbours' velocities.
+__device__ __forceinline__ float4 implicit_cell(const SceneDev& sc, const float4& me, float ax, float ay, float az,
+                                                float cnt, float dt) {
+    const float m = me.w;
+    if (cnt > 0.f) {
+        ax = ax / cnt;
+        ay = ay / cnt;
+        az = az / cnt;
+    } else {
+        ax = me.x;
+        ay = me.y;
+        az = me.z;
+    }
+    const float alpha = dt * dt * m * (sc.youngs / 1500.0f) * sc.inv_dx * sc.inv_dx;
+    const float den = m + alpha;
+    const float vx = (m * me.x + alpha * ax) / den, vy = (m * me.y + alpha * ay) / den,
+                vz = (m * me.z + alpha * az) / den;
+    return vx == vx && vy == vy && vz == vz ? make_float4(vx, vy, vz, m) : me;
+}
+
 template <int K>
 __global__ __launch_bounds__(256) void k_implicit_sweeps(const SceneDev* __restrict__ scenes, GridDev g,
                                                          const float4* __restrict__ src, float4* __restrict__ dst,
@@ -762,6 +782,8 @@ __global__ __launch_bounds__(256) void k_implicit_sweeps(const SceneDev* __restr
         const SceneDev sc = scenes[g.tile_scene[t]];
         int tx, ty, tz, ix0, iy0, iz0;
         tile_cell(sc, t, 0, tx, ty, tz, ix0, iy0, iz0);
+        const int lo[3] = {ix0 - K, iy0 - K, iz0 - K}, hi[3] = {ix0 + 3 + K, iy0 + 3 + K, iz0 + 3 + K};
+        const uint64_t near = rigid_near_legacy(rg, sc, lo, hi);
         float4 v[PER];
         bool on[PER];
 #pragma unroll
@@ -783,7 +805,7 @@ __global__ __launch_bounds__(256) void k_implicit_sweeps(const SceneDev* __restr
                 // empty cells and negative masses are no neighbours; cells
                 // stamped by a legacy sphere keep their velocity
                 if (!(v[u].w > 1.0e-9f)) v[u].w = 0.f;
-                else if (rigid_masked_legacy(rg, sc, ix, iy, iz)) v[u].w = -v[u].w;
+                else if (rigid_masked_near(rg, near, sc, ix, iy, iz)) v[u].w = -v[u].w;
             }
         }
 #pragma unroll
@@ -798,9 +820,9 @@ __global__ __launch_bounds__(256) void k_implicit_sweeps(const SceneDev* __restr
         for (int s = 1; s <= K; ++s) {
             const float4* a = buf[(s - 1) & 1];
             float4* b = buf[s & 1];
-            const int lo = s, side = R - 2 * s;  // cells [lo, lo + side) on each axis
+            const int first = s, side = R - 2 * s;  // cells [first, first + side) on each axis
             for (int c = tid; c < side * side * side; c += 256) {
-                const int lx = lo + c % side, ly = lo + (c / side) % side, lz = lo + c / (side * side);
+                const int lx = first + c % side, ly = first + (c / side) % side, lz = first + c / (side * side);
                 const int at = lx + R * (ly + R * lz);
                 const float4 me = a[at];
                 const float m = me.w;
@@ -817,20 +839,7 @@ __global__ __launch_bounds__(256) void k_implicit_sweeps(const SceneDev* __restr
                         az += nb.z;
                         cnt += 1.0f;
                     }
-                    if (cnt > 0.f) {
-                        ax = ax / cnt;
-                        ay = ay / cnt;
-                        az = az / cnt;
-                    } else {
-                        ax = me.x;
-                        ay = me.y;
-                        az = me.z;
-                    }
-                    const float alpha = dt * dt * m * (sc.youngs / 1500.0f) * sc.inv_dx * sc.inv_dx;
-                    const float den = m + alpha;
-                    const float vx = (m * me.x + alpha * ax) / den, vy = (m * me.y + alpha * ay) / den,
-                                vz = (m * me.z + alpha * az) / den;
-                    if (vx == vx && vy == vy && vz == vz) out = make_float4(vx, vy, vz, m);
+                    out = implicit_cell(sc, me, ax, ay, az, cnt, dt);
                 }
                 b[at] = out;
             }
@@ -854,30 +863,92 @@ __global__ __launch_bounds__(256) void k_implicit_sweeps(const SceneDev* __restr
     for (uint32_t i = tid; i < nd; i += 256u) g.tile_flag[dlist[i]] &= ~FLAG_DYN;
 }
 
-constexpr uint32_t SWEEPS_PER_LAUNCH = 3;
-
-float4* implicit_first(float4* gv, float4* scratch, uint32_t iters) {
-    return ((iters + SWEEPS_PER_LAUNCH - 1) / SWEEPS_PER_LAUNCH) % 2 ? scratch : gv;
+// One sweep per launch, a wave per tile and a lane per cell: half the cell
+// updates of K = 2, a quarter of K = 3.  A chain of dependent loads per wave,
+// so it needs its 8,192 waves in flight at once: with the tickets in it, 96
+// scalar registers, seven blocks fitted on a CU and 32,768 tiles took 50
+// instead of 32 us.
+__global__ __launch_bounds__(256) void k_implicit_sweep(const SceneDev* __restrict__ scenes, GridDev g,
+                                                        const float4* __restrict__ src, float4* __restrict__ dst,
+                                                        const uint32_t* __restrict__ dlist,
+                                                        const uint32_t* __restrict__ dcount, float dt, RigidDev rg) {
+    const TileWalk walk(g, dcount);
+    const int lane = threadIdx.x & 63;
+    for (uint32_t i = blockIdx.x * 4 + uint32_t(wave_id()); i < walk.n; i += gridDim.x * 4) {
+        uint32_t t, st;
+        walk.at(g, dlist, i, t, st);
+        const SceneDev sc = scenes[g.tile_scene[t]];
+        int tx, ty, tz, ix, iy, iz;
+        tile_cell(sc, t, lane, tx, ty, tz, ix, iy, iz);
+        const uint32_t c = (st << 6) | uint32_t(lane);
+        const float4 me = src[c];
+        // empty cells and cells stamped by a legacy sphere keep their velocity
+        if (!(me.w > 1.0e-9f) || rigid_masked_legacy(rg, sc, ix, iy, iz)) {
+            dst[c] = me;
+            continue;
+        }
+        const int off[6][3] = {{1, 0, 0}, {-1, 0, 0}, {0, 1, 0}, {0, -1, 0}, {0, 0, 1}, {0, 0, -1}};
+        float ax = 0.f, ay = 0.f, az = 0.f, cnt = 0.f;
+#pragma unroll
+        for (int k = 0; k < 6; ++k) {
+            const int jx = ix + off[k][0], jy = iy + off[k][1], jz = iz + off[k][2];
+            if (!in_grid(sc, jx, jy, jz)) continue;
+            uint32_t nc;
+            if (g.tile_slot) {
+                if (!cell_storage(sc, g.tile_slot, jx, jy, jz, nc)) continue;  // no slot: no P2G mass
+            } else {
+                nc = cell_index(sc, jx, jy, jz);
+                if ((g.tile_flag[nc >> 6] & (FLAG_STATIC | FLAG_DYN)) == 0u) continue;
+            }
+            const float4 nb = src[nc];
+            if (!(nb.w > 1.0e-9f)) continue;
+            ax += nb.x;
+            ay += nb.y;
+            az += nb.z;
+            cnt += 1.0f;
+        }
+        dst[c] = implicit_cell(sc, me, ax, ay, az, cnt, dt);
+    }
 }
 
-hipError_t launch_implicit_sweeps(const SceneDev* scenes, const GridDev& g, float4* scratch, uint32_t iters,
+// Takes FLAG_DYN off the listed tiles.
+__global__ __launch_bounds__(256) void k_end_dynamic(GridDev g, const uint32_t* __restrict__ dlist,
+                                                     const uint32_t* __restrict__ dcount) {
+    const uint32_t nd = *dcount;
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < nd; i += gridDim.x * blockDim.x)
+        g.tile_flag[dlist[i]] &= ~FLAG_DYN;
+}
+
+constexpr uint32_t SWEEPS_PER_LAUNCH = 3;
+
+float4* implicit_first(float4* gv, float4* scratch, uint32_t iters, bool many) {
+    const uint32_t launches = many ? iters : (iters + SWEEPS_PER_LAUNCH - 1) / SWEEPS_PER_LAUNCH;
+    return launches % 2 ? scratch : gv;
+}
+
+hipError_t launch_implicit_sweeps(const SceneDev* scenes, const GridDev& g, float4* scratch, uint32_t iters, bool many,
                                   const uint32_t* dlist, const uint32_t* dcount, float dt, int blocks, uint32_t* tickets,
-                                  hipStream_t s, const RigidDev* rigid) {
+                                  bool end, bool listed, hipStream_t s, const RigidDev* rigid) {
     const RigidDev rg = rigid ? *rigid : RigidDev{nullptr, nullptr, 0u, 0u};
-    float4* a = implicit_first(g.gv, scratch, iters);
+    // one block takes the few marks of escaped particles off by the way
+    const bool ticket = end && !many && !listed;
+    float4* a = implicit_first(g.gv, scratch, iters, many);
     while (iters > 0) {
         float4* b = a == scratch ? g.gv : scratch;
-        const uint32_t k = std::min(iters, SWEEPS_PER_LAUNCH);
+        const uint32_t k = many ? 1u : std::min(iters, SWEEPS_PER_LAUNCH);
         iters -= k;
-        uint32_t* tk = iters == 0 ? tickets : nullptr;
+        uint32_t* tk = iters == 0 && ticket ? tickets : nullptr;
 #define MPM_SWEEPS(K) \
     hipLaunchKernelGGL(k_implicit_sweeps<K>, dim3(blocks), dim3(256), 0, s, scenes, g, a, b, dlist, dcount, dt, rg, tk)
-        if (k == 3) MPM_SWEEPS(3);
+        if (many)
+            hipLaunchKernelGGL(k_implicit_sweep, dim3(blocks), dim3(256), 0, s, scenes, g, a, b, dlist, dcount, dt, rg);
+        else if (k == 3) MPM_SWEEPS(3);
         else if (k == 2) MPM_SWEEPS(2);
         else MPM_SWEEPS(1);
 #undef MPM_SWEEPS
         a = b;
     }
+    if (end && !ticket) hipLaunchKernelGGL(k_end_dynamic, dim3(256), dim3(256), 0, s, g, dlist, dcount);
     return hipGetLastError();
 }
 

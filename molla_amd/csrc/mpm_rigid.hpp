@@ -14,6 +14,7 @@
 // (set_prescribed_solids: the sand mass keeps its mass and sticks).
 #pragma once
 
+#include "../../include/molla_mpm.h"
 #include "mpm_internal.hpp"
 
 namespace mpm {
@@ -105,6 +106,38 @@ __device__ __forceinline__ bool rigid_masked_legacy(const RigidDev& rg, const Sc
         if (rigid_contains(b, arm)) return true;
     }
     return false;
+}
+
+// The same for the bodies in `near` only.
+__device__ __forceinline__ bool rigid_masked_near(const RigidDev& rg, uint64_t near, const SceneDev& sc, int ix,
+                                                  int iy, int iz) {
+    if (near == 0ull) return false;
+    const float3 node = node_position(sc, ix, iy, iz);
+    for (uint64_t m = near; m; m &= m - 1ull) {
+        const float4* b = rg.body + RIGID_ROWS * (__ffsll((unsigned long long)m) - 1);
+        const float3 arm = make_float3(node.x - b[0].x, node.y - b[0].y, node.z - b[0].z);
+        if (rigid_contains(b, arm)) return true;
+    }
+    return false;
+}
+
+// The legacy spheres (bit r: body r, lane r decides) that may hold a node of
+// the cells from lo to hi; a cell's margin covers the rounding.  All 64 lanes
+// call it.
+__device__ __forceinline__ uint64_t rigid_near_legacy(const RigidDev& rg, const SceneDev& sc, const int* lo,
+                                                      const int* hi) {
+    static_assert(MPM_MAX_RIGID <= 64, "a lane per body");
+    if (rg.count == 0 || rg.prescribed) return 0ull;
+    const uint32_t lane = threadIdx.x & 63u;
+    bool on = false;
+    if (lane < rg.count) {
+        const float4 b = rg.body[RIGID_ROWS * lane];
+        const float3 l = node_position(sc, lo[0], lo[1], lo[2]), h = node_position(sc, hi[0], hi[1], hi[2]);
+        const float dx = fmaxf(fmaxf(l.x - b.x, b.x - h.x), 0.f), dy = fmaxf(fmaxf(l.y - b.y, b.y - h.y), 0.f),
+                    dz = fmaxf(fmaxf(l.z - b.z, b.z - h.z), 0.f);
+        on = !(sqrtf(dx * dx + dy * dy + dz * dz) > b.w + sc.dx);
+    }
+    return __ballot(on);
 }
 
 __device__ __forceinline__ double wave_sum_f64(double v) {

@@ -170,6 +170,7 @@ __device__ __forceinline__ void layout_lists(LB lb, const LayoutArgs& q, const C
     }
     if (threadIdx.x == 0) {
         *q.scount = uint32_t(total);
+        if (q.host_scount) *q.host_scount = uint32_t(total);
         *q.n_chunks = uint32_t(total >> 32);
     }
 }
@@ -370,7 +371,11 @@ __global__ __launch_bounds__(TILE_THREADS) void k_tile_emit(LayoutArgs q, ChunkR
     const bool on = (q.tile_flag[t] & FLAG_STATIC) != 0u;
     if (on) q.slist[uint32_t(at)] = t;
     // the last tile knows the static count, the last row's first tile the chunk count
-    if (t + 1 == q.total_tiles) *q.scount = uint32_t(at) + (on ? 1u : 0u);
+    if (t + 1 == q.total_tiles) {
+        const uint32_t tiles = uint32_t(at) + (on ? 1u : 0u);
+        *q.scount = tiles;
+        if (q.host_scount) *q.host_scount = tiles;
+    }
     if (p.x == 0u) {
         const uint32_t end = emit_row(lb, t, p, rule, uint32_t(at >> 32), q.chunks);
         if (t + p.sc->W == q.total_tiles) *q.n_chunks = end;
