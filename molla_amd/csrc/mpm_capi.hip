@@ -453,11 +453,28 @@ uint32_t chunk_bound(const mpm_sim* s) {
 // Cells of grid storage: every tile of a dense grid, the pool of a sparse one.
 size_t grid_cells(const mpm_sim* s) { return (size_t)(s->pool_cap ? s->pool_cap : s->total_tiles) * 64; }
 
+// Whether the semi-implicit sweeps go one per launch (launch_implicit_sweeps).
+// Three to a launch save launches and cost four times the cell updates, so the
+// line lies where the active tiles fill the chip: a substep of three sweeps,
+// three to a launch / one, 1,300 tiles (300,000 particles) 73 / 79 us, 2,744
+// 107 / 112, 3,400 (1 M) 148 / 142, 4,096 149 / 139, 32,768 (200,000 particles
+// over 128^3) 765 / 601.  The number of tiles is on the device; the sorts also
+// leave it in pinned memory, and what the last sort that has ended wrote there
+// is near enough: both ways leave the same bits.  Before one has, or without
+// sorts, grids beyond the line count as full.
+constexpr uint32_t MANY_TILES = 3072;
+uint32_t most_tiles(const mpm_sim* s) { return s->pool_cap ? s->pool_cap : s->total_tiles; }
+bool many_tiles(const mpm_sim* s) {
+    if (s->jacobi_iters == 0 || std::min<uint64_t>(most_tiles(s), 27ull * s->n) <= MANY_TILES) return false;
+    const uint32_t tiles = s->hcount ? *static_cast<volatile uint32_t*>(s->hcount) : 0u;
+    return tiles == 0u || s->p2g_mode == MPM_P2G_GLOBAL_ATOMIC || tiles > MANY_TILES;
+}
+
 // The second cell buffer of the semi-implicit sweeps, and the word their rule
 // reads (many_tiles).
 int ensure_implicit(mpm_sim* s) {
     if (!s->gv2) HIP_TRY(s, dalloc(&s->gv2, grid_cells(s)));
-    if (!s->hcount) {
+    if (!s->hcount && most_tiles(s) > MANY_TILES) {
         if (hipHostMalloc((void**)&s->hcount, 64, hipHostMallocDefault) == hipSuccess) {
             *s->hcount = 0u;
         } else {
@@ -687,24 +704,6 @@ int particle_pass(mpm_sim* s, int mode, float dt, int list_out, float* ps = null
     HIP_TRY(s, mpm::launch_particle_pass(mode, int(s->sh[0].model), a, sorted_chunks ? int(s->chunk_ppt) : 1, blocks,
                                          s->stream));
     return MPM_OK;
-}
-
-// Whether the semi-implicit sweeps go one per launch (launch_implicit_sweeps).
-// Three to a launch save launches and cost four times the cell updates, so the
-// line lies where the active tiles fill the chip: a substep of three sweeps,
-// three to a launch / one, 1,300 tiles (300,000 particles) 73 / 79 us, 2,744
-// 107 / 112, 3,400 (1 M) 148 / 142, 4,096 149 / 139, 32,768 (200,000 particles
-// over 128^3) 765 / 601.  The number of tiles is on the device; the sorts also
-// leave it in pinned memory, and what the last sort that has ended wrote there
-// is near enough: both ways leave the same bits.  Before one has, or without
-// sorts, grids beyond the line count as full.
-constexpr uint32_t MANY_TILES = 3072;
-bool many_tiles(const mpm_sim* s) {
-    if (s->jacobi_iters == 0) return false;
-    const uint32_t most = s->pool_cap ? s->pool_cap : s->total_tiles;
-    if (std::min<uint64_t>(most, 27ull * s->n) <= MANY_TILES) return false;
-    const uint32_t tiles = s->hcount ? *static_cast<volatile uint32_t*>(s->hcount) : 0u;
-    return tiles == 0u || s->p2g_mode == MPM_P2G_GLOBAL_ATOMIC || tiles > MANY_TILES;
 }
 
 // `react`: this substep reports the rigid bodies' reaction (the last
@@ -2100,7 +2099,7 @@ int mpm_reserve_sparse_tiles(mpm_sim* sim, uint32_t tile_capacity) {
     }
     sim->pool_cap = tile_capacity;
     drop_graphs(sim);
-    return MPM_OK;
+    return sim->gv2 ? ensure_implicit(sim) : MPM_OK;
 }
 
 int mpm_grid_storage_bytes(mpm_sim* sim, uint64_t* bytes) {
