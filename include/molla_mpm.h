@@ -93,7 +93,9 @@ typedef struct mpm_sim mpm_sim;
 typedef enum {
     MPM_P2G_FUSED = 0,         /* fused G2P->P2G kernel, LDS-staged (default)      */
     MPM_P2G_GLOBAL_ATOMIC = 1, /* unfused, one global atomic per node (legacy p2g) */
-    MPM_P2G_DETERMINISTIC = 2  /* sorted gather-order P2G, bitwise repeatable      */
+    MPM_P2G_DETERMINISTIC = 2  /* sorted gather-order P2G, bitwise repeatable: the
+                                * reference's order, added as 16 interleaved sums
+                                * in a fixed tree (less rounding, other last bits) */
 } mpm_p2g_mode;
 
 typedef struct {
@@ -254,7 +256,8 @@ int mpm_autotune_config(mpm_sim* sim, float dt, uint32_t trial_substeps, mpm_lau
 
 /* ---- stepping (step / step_n, mpm.rs:2232-2272) ---- */
 /* Small scenes' repeated calls replay a captured graph, with the same bits
- * (the fused mode, 8 substeps or more, up to 131,072 particles). */
+ * (the fused mode, 8 substeps or more, up to 131,072 particles; at most 64
+ * graphs a handle, of about 2 MB of device memory each). */
 int mpm_step_n(mpm_sim* sim, float dt, uint32_t substeps);
 /* Capture step_n(dt, substeps) into a hipGraph once and replay it
  * (PreparedMpmStep / MpmCommandBatch, mpm_command_batch.rs:10-235). */

@@ -262,11 +262,13 @@ hipError_t dalloc(T** p, size_t count) {
 
 // Pinned host memory that kernels of the handle write small results to, so
 // that a read is one launch, one wait and a host copy.  The writes of a field
-// are scattered by id and cost about 1 ns a particle over the bus, the copy
-// from device memory into the caller's pages a fixed 15 to 45 us.  Positions
-// of 1,000 particles 29.8 -> 15.3 us, of 6,001 53.6 -> 20.9, of 10,000 70.0 ->
-// 25.9; of 16,384 33.8 -> 33.3 and one-word fields there 27.1 -> 29.8, hence
-// the line.
+// are scattered by id and cost about 0.8 ns a particle over the bus, the copy
+// from device memory into the caller's pages a fixed 15 us and 0.1 ns a byte.
+// Copy / mailbox, one, three and nine words a particle: 1,000 particles 26.3 /
+// 14.3, 29.3 / 14.5, 38.3 / 15.9 us; 10,000 25.5 / 22.4, 29.1 / 24.5, 39.5 /
+// 33.3; 14,000 26.3 / 26.5, 30.9 / 29.2, 45.3 / 41.3; 20,000 27.4 / 29.9, 33.8
+// / 33.9, 54.7 / 51.1.  One word meets at about 13,000 particles, so no read is
+// slower up to the line, which keeps the block at 360 KB.
 constexpr uint32_t MAIL_PARTICLES = 10000;
 constexpr size_t MAIL_BYTES = (size_t)MAIL_PARTICLES * 9 * sizeof(float);
 static_assert(MAIL_BYTES >= MPM_MAX_RIGID * std::max(8 * sizeof(double), mpm::RIGID_ROWS * sizeof(float4)),

@@ -31,8 +31,9 @@
 // us), of 2 M in 256^3 15 (290 us); lists built from per-particle flags took
 // 27 to 32 launches and about 130, 190 and 480 us.  The lines: k_layout_one
 // still beats the separate launches at its 16,384 particles (36 us against
-// ~60), where its LDS ends; one block walks 8,192 tiles in 15 us, as long as
-// the four launches it saves.
+// ~60), where the 14 bits of a slot and its 16 keys per thread end (98 of the
+// CU's 160 KB of LDS are in use); one block walks 8,192 tiles in 15 us, as long
+// as the four launches it saves.
 #include <algorithm>
 
 #include "mpm_internal.hpp"
