@@ -760,7 +760,7 @@ int deterministic_p2g(mpm_sim* s, float dt) {
     mpm::StepArgs a = args(s, dt, s->list_cur);
     HIP_TRY(s, mpm::launch_gather_prepare(a, s->affine, particle_blocks(s), s->stream));
     HIP_TRY(s, mpm::launch_gather_p2g(a, s->tile_scene, s->tile_lb, s->affine, s->slist,
-                                      s->status + mpm::ST_SCOUNT, int(std::min(s->total_tiles, 2048u)), s->stream));
+                                      s->status + mpm::ST_SCOUNT, s->total_tiles, s->n, s->stream));
     return MPM_OK;
 }
 

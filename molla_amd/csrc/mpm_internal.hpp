@@ -288,7 +288,7 @@ hipError_t launch_grid_to_dense(const float4* gmp, const SceneDev* scenes, uint3
 hipError_t launch_gather_prepare(const StepArgs& a, float* affine, int blocks, hipStream_t s);
 hipError_t launch_gather_p2g(const StepArgs& a, const uint32_t* tile_scene, const uint32_t* tile_lb,
                              const float* affine, const uint32_t* slist, const uint32_t* scount,
-                             int blocks, hipStream_t s);
+                             uint32_t total_tiles, uint32_t n, hipStream_t s);
 hipError_t launch_reorder_index(const uint32_t* sorted_ids, const uint32_t* slot_of_id,
                                 uint32_t* src_slot, uint32_t n, hipStream_t s);
 

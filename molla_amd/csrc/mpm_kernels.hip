@@ -1601,14 +1601,17 @@ hipError_t launch_gather_prepare(const StepArgs& a, float* affine, int blocks, h
 // loads issued before the sums of the one before.
 // A block fills its CU, so a grid of many thin tiles (20,000 particles over
 // 128^3 cells: 32,768 active tiles of 5 candidates) waits for one tile after
-// the other, 641 us against 191 with a tile per wave.  Above GATHER_BLOCKS
-// tiles a block therefore takes 16 at once, a wave sums a tile of up to
-// GATHER_WAVE_RECS records by itself, row by row and in the same order, and
-// what is left goes to the block.  Two substeps with / without it: 1,000
-// particles over 64^3 289 / 374 us, 20,000 over 128^3 879 / 1,780, 200,000 921
-// / 1,860, 1 M 2,382 / 2,364; 200,000 within 12^3 cells 1,177 / 1,231.  Up to
-// GATHER_BLOCKS tiles the block's whole attention is faster: 50 particles in
-// 16^3 126 us against 149, 16,384 sand particles (4 substeps) 170 / 176.
+// the other, 641 us against 190 with a tile per wave.  Scenes of more than 512
+// active tiles and fewer than GATHER_THIN particles a tile therefore give a
+// block 16 tiles at once; a wave sums a tile of up to GATHER_WAVE_RECS records
+// by itself, row by row and in the same order, and what is left goes to the
+// block.  A substep with / without it: 1,000 particles over 64^3 113 / 188 us,
+// 3,000 over 40^3 102 / 112, 20,000 over 128^3 361 / 897, 40,000 over 96^3 242 /
+// 455, 200,000 over 128^3 461 / 930.  Denser or fewer tiles are faster with the
+// block's whole attention: 20,000 particles over 27^3 cells 106 / 128 us,
+// 300,000 over 46^3 289 / 322, 16,384 sand particles (a frame of 4) 170 / 176.
+// The line lies where a tile's records outgrow its wave: eight particles a tile
+// are 27 records.
 constexpr int GATHER_THREADS = 1024;
 constexpr int GATHER_WAVES = GATHER_THREADS / 64;
 constexpr int GATHER_PER = 4;
@@ -1617,7 +1620,9 @@ constexpr int GATHER_STEP = 16 * GATHER_FLY;
 constexpr int GATHER_RECS = 512;
 constexpr int GATHER_LIST = 8192;
 constexpr int GATHER_WAVE_RECS = GATHER_RECS / GATHER_WAVES;
-constexpr int GATHER_BLOCKS = 512;
+constexpr int GATHER_GRID = 2048;
+constexpr int GATHER_BLOCKS = 256;  // one per CU
+constexpr uint32_t GATHER_THIN = 8;  // particles per active tile
 static_assert(GATHER_WAVE_RECS <= GATHER_STEP && GATHER_RECS + GATHER_STEP >= 8 * GATHER_STEP, "four lists of a step each");
 
 // A particle relative to a tile: the four channels as c + r0 d0 + r1 d1 + r2 d2
@@ -1718,7 +1723,7 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
                                                                const uint32_t* __restrict__ lb,
                                                                const float* __restrict__ aff,
                                                                const uint32_t* __restrict__ list,
-                                                               const uint32_t* __restrict__ count) {
+                                                               const uint32_t* __restrict__ count, uint32_t thin) {
     __shared__ GatherRec rec[GATHER_RECS + 1];  // the last one reaches no cell
     __shared__ uint16_t rows[GATHER_RECS];      // bit y + 4 z: the record reaches that x-row of the tile
     __shared__ uint16_t wlist[GATHER_WAVES][GATHER_RECS + GATHER_STEP];
@@ -1916,13 +1921,9 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
         gather_store(sc, tc, t, cy, cz, acc, a.gmp);
         if (tid == 0) a.tile_flag[t] |= FLAG_GMP;
     };
-    // few tiles: one per block, whose waves all find its ranges; else a tile
-    // per wave, on as many blocks
-    const uint32_t nb = min(gridDim.x, max(n / 8u, uint32_t(GATHER_BLOCKS)));
     SceneDev sc;
     int tc[3];
-    uint32_t scene = ~0u;  // whose record sc is
-    if (n <= nb) {
+    if (n <= thin && n <= gridDim.x) {  // the whole block takes a tile; each wave finds its ranges
         if (blockIdx.x >= n) return;
         const uint32_t t = list[blockIdx.x];
         tile(t, tile_scene[t], sc, tc);
@@ -1930,7 +1931,10 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
         by_block(sc, tc, t, wave);
         return;
     }
+    // a tile per wave first, on so many blocks that their waves have work
+    const uint32_t nb = n > thin ? min(gridDim.x, max(n / uint32_t(GATHER_WAVES), uint32_t(GATHER_BLOCKS))) : gridDim.x;
     if (blockIdx.x >= nb) return;
+    uint32_t scene = ~0u;  // whose record sc is
     for (uint32_t i0 = blockIdx.x; i0 < n; i0 += nb * GATHER_WAVES) {
         const uint32_t i = i0 + nb * uint32_t(wave);
         uint4 left = make_uint4(~0u, 0u, 0u, 0u);
@@ -1938,12 +1942,14 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
             const uint32_t t = list[i];
             scene = tile_scene[t];
             tile(t, scene, sc, tc);
-            if (!by_wave(sc, tc, t, ranges(sc, tc)))
+            const uint32_t total = ranges(sc, tc);
+            if (n <= thin || !by_wave(sc, tc, t, total))
                 left = make_uint4(t, scene, uint32_t(tc[0]) | uint32_t(tc[1]) << 16, uint32_t(tc[2]));
         }
         if (lane == 0) whole[wave] = left;
         __syncthreads();
-        for (int w = 0; w < GATHER_WAVES; ++w) {
+        const int held = int(min((n - i0 + nb - 1u) / nb, uint32_t(GATHER_WAVES)));  // waves with a tile
+        for (int w = 0; w < held; ++w) {
             const uint4 q = whole[w];
             const uint32_t t = uint32_t(__builtin_amdgcn_readfirstlane(int(q.x)));
             if (t == ~0u) continue;
@@ -1962,9 +1968,10 @@ __global__ __launch_bounds__(GATHER_THREADS) void k_gather_p2g(StepArgs a, const
 
 hipError_t launch_gather_p2g(const StepArgs& a, const uint32_t* tile_scene, const uint32_t* tile_lb,
                              const float* affine, const uint32_t* slist, const uint32_t* scount,
-                             int blocks, hipStream_t s) {
+                             uint32_t total_tiles, uint32_t n, hipStream_t s) {
+    const unsigned blocks = std::min(total_tiles, uint32_t(GATHER_GRID));
     hipLaunchKernelGGL(k_gather_p2g, dim3(blocks), dim3(GATHER_THREADS), 0, s, a, tile_scene, tile_lb, affine, slist,
-                       scount);
+                       scount, std::max(n / GATHER_THIN, 2u * GATHER_BLOCKS));
     return hipGetLastError();
 }
 

@@ -1,7 +1,8 @@
-"""The ordered gather's two ways to sum a tile, by its own wave (up to 32
-records, up to 512 candidates) and by the whole block, leave the same bits: a
-particle of no mass and no volume adds nothing but moves its tiles across the
-line; grids of more tiles than a launch has blocks match the oracle."""
+"""The ordered gather's two ways to sum a tile of a thin scene, by its own wave
+(up to 32 records, up to 512 candidates) and by the whole block, leave the same
+bits: a particle of no mass and no volume adds nothing but moves its tiles
+across the line.  So do a thin scene and a dense one, and grids of more tiles
+than a launch has blocks match the oracle."""
 import numpy as np
 import pytest
 
@@ -24,28 +25,51 @@ def _grid(cfg, x, v, mass, vol):
     return m, p
 
 
-@pytest.mark.parametrize("near,far", [(1, 0), (31, 0), (32, 0), (33, 0), (32, 470), (32, 480), (20, 492), (5, 600)])
-def test_both_ways_leave_the_same_bits(near, far):
-    # `near` particles whose stencils reach the tile, `far` candidates in the
-    # tiles beside it that do not; then one more of each without mass
-    G, dx = 32, 1.0 / 32
+def _tile(near, far):
+    """`near` particles whose stencils reach tile (4, 4, 4) of a 64^3 grid, and
+    `far` candidates in the tiles beside it that do not."""
     rng = np.random.default_rng(near + far)
-    cfg = MpmConfig.sand().copy(gravity_y=0.0, grid_origin=(0.0, 0.0, 0.0), grid_size=G, cell_size=dx)
-    a = 16.6 + 2.8 * rng.random((near, 3))  # in tile (4, 4, 4)
-    b = 16.6 + 2.8 * rng.random((far, 3))
-    b[:, 0] = 21.6 + 1.8 * rng.random(far)  # nodes from 21 on: two cells beyond it
-    x = (dx * np.concatenate([a, b])).astype(np.float32)
-    v = rng.standard_normal(x.shape).astype(np.float32)
-    mass = (1e-3 * (1.0 + rng.random(len(x)))).astype(np.float32)
-    vol = np.full(len(x), cfg.particle_volume, np.float32)
-    want = _grid(cfg, x, v, mass, vol)
+    x = np.concatenate([16.6 + 2.8 * rng.random((near, 3)), 16.6 + 2.8 * rng.random((far, 3))])
+    x[near:, 0] = 21.6 + 1.8 * rng.random(far)  # nodes from 21 on: two cells beyond it
+    return x, rng.standard_normal(x.shape), 1e-3 * (1.0 + rng.random(len(x)))
+
+
+def _scattered(n):
+    rng = np.random.default_rng(n)
+    x = 32.0 + 28.0 * rng.random((n, 3))  # three tiles away and more
+    return x, rng.standard_normal(x.shape), 1e-3 * (1.0 + rng.random(n))
+
+
+def _cfg(n):
+    return MpmConfig.sand().copy(gravity_y=0.0, grid_origin=(0.0, 0.0, 0.0), grid_size=64, cell_size=1.0 / 64,
+                                 max_particles=n)
+
+
+def _run(parts, massless):
+    x, v, m = (np.concatenate(q) for q in zip(*parts))
+    cfg = _cfg(len(x) + massless)
+    y = np.concatenate([x, np.full((massless, 3), 18.2)]) / 64.0
+    vol = np.concatenate([np.full(len(x), cfg.particle_volume), np.zeros(massless)])
+    f = np.float32
+    return _grid(cfg, y.astype(f), np.concatenate([v, np.zeros((massless, 3))]).astype(f),
+                 np.concatenate([m, np.zeros(massless)]).astype(f), vol.astype(f))
+
+
+@pytest.mark.parametrize("near,far", [(1, 0), (16, 0), (17, 0), (31, 0), (32, 0), (33, 0), (32, 470), (32, 480),
+                                      (20, 492), (5, 600)])
+def test_both_ways_leave_the_same_bits(near, far):
+    parts = [_tile(near, far), _scattered(600)]  # more than 600 active tiles, and few particles for them
+    want = _run(parts, 0)
     assert want[0].max() > 0
-    for extra in (1, 2, 40, 600):  # near the tile's middle
-        y = np.concatenate([x, np.tile(np.float32(dx * 18.2), (extra, 3))])
-        got = _grid(cfg, y, np.concatenate([v, np.zeros((extra, 3), np.float32)]),
-                    np.concatenate([mass, np.zeros(extra, np.float32)]),
-                    np.concatenate([vol, np.zeros(extra, np.float32)]))
+    for extra in (1, 2, 40, 600):
+        got = _run(parts, extra)
         assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1]), extra
+    # without the scattered ones the scene has few tiles and each takes a block
+    alone = _run(parts[:1], 0)
+    box = np.zeros((64, 64, 64), bool)
+    box[:28, :28, :28] = True  # z, y, x: the cells of the tile and its neighbours
+    box = box.ravel()
+    assert np.array_equal(alone[0][box], want[0][box]) and np.array_equal(alone[1][box], want[1][box])
 
 
 def test_many_thin_tiles_match_the_oracle():
