@@ -89,7 +89,7 @@ struct mpm_sim {
     uint32_t max_W = 0;         // tiles of the longest tile row
     uint32_t* list[2] = {nullptr, nullptr};
     uint32_t* status = nullptr;  // ST_WORDS u32
-    uint32_t* tickets = nullptr;  // TICKET_WORDS u32
+    uint32_t* tickets = nullptr;  // TICKET_WORDS u32, in the status words' allocation
     uint32_t* slot_of_id = nullptr;
     bool index_valid = false;  // slot_of_id describes the current slots (the fused layout sorts leave it behind)
     uint32_t* keys = nullptr;
@@ -292,7 +292,7 @@ void release(mpm_sim* s) {
     }
     for (hipEvent_t e : s->ev_pool) (void)hipEventDestroy(e);
     void* bufs[] = {s->d_scenes, s->d_mats, s->ps[0], s->ps[1], s->gmp, s->gv, s->tile_flag, s->tile_scene,
-                    s->list[0], s->list[1], s->status, s->tickets, s->slot_of_id, s->keys, s->vals, s->sort_scratch,
+                    s->list[0], s->list[1], s->status, s->slot_of_id, s->keys, s->vals, s->sort_scratch,
                     s->d_chunks, s->affine, s->staging, s->tile_lb, s->slist,
                     s->src_slot, s->chunk_box, s->part, s->schunks, s->chunk_of_slot, s->lscan, s->tile_slot,
                     s->tile_mark, s->slot_tile, s->defer_list, s->srec};
@@ -1007,8 +1007,9 @@ int create(const mpm_scene_config* cfgs, uint32_t n_scenes, mpm_sim** out) {
     HIP_TRY(s, dalloc(&s->d_mats, (size_t)n_scenes * MPM_MAX_MATERIALS * mpm::MAT_STRIDE));
     HIP_TRY(s, dalloc(&s->ps[0], (size_t)mpm::NCOMP * s->cap));
     HIP_TRY(s, dalloc(&s->ps[1], (size_t)mpm::NCOMP * s->cap));
-    HIP_TRY(s, dalloc(&s->status, mpm::ST_WORDS));
-    HIP_TRY(s, dalloc(&s->tickets, mpm::TICKET_WORDS));
+    static_assert(mpm::ST_WORDS <= mpm::TICKET_STRIDE, "the tickets' cache lines are their own");
+    HIP_TRY(s, dalloc(&s->status, mpm::TICKET_STRIDE + mpm::TICKET_WORDS));
+    s->tickets = s->status + mpm::TICKET_STRIDE;
     HIP_TRY(s, dalloc(&s->slot_of_id, s->cap));
     HIP_TRY(s, dalloc(&s->keys, s->cap));
     HIP_TRY(s, dalloc(&s->vals, s->cap));
@@ -1017,8 +1018,7 @@ int create(const mpm_scene_config* cfgs, uint32_t n_scenes, mpm_sim** out) {
     s->max_chunks = s->cap / CHUNK + n_scenes + 1;
     HIP_TRY(s, dalloc(&s->d_chunks, (size_t)s->max_chunks));
     HIP_TRY(s, dalloc(&s->staging, (size_t)9 * s->cap));
-    HIP_TRY(s, hipMemsetAsync(s->status, 0, mpm::ST_WORDS * 4, s->stream));
-    HIP_TRY(s, hipMemsetAsync(s->tickets, 0, mpm::TICKET_WORDS * 4, s->stream));
+    HIP_TRY(s, hipMemsetAsync(s->status, 0, (mpm::TICKET_STRIDE + mpm::TICKET_WORDS) * 4, s->stream));
     HIP_TRY(s, hipMemsetAsync(s->ps[0], 0, (size_t)mpm::NCOMP * s->cap * 4, s->stream));
     HIP_TRY(s, hipStreamSynchronize(s->stream));
     (void)cells;
